@@ -102,14 +102,12 @@ __device__ __forceinline__ unsigned short f2bf(float x)
  *   A: X[row0 + l % 32][8 s + 4 (l / 32) + j]
  *   B: W[l % 32][8 s + 4 (l / 32) + j]
  *   D: register r holds Y[row0 + 8 (r / 4) + 4 (l / 32) + r % 4][l % 32]
- * EPI 0: z   1: relu(z)   2: R + relu(z)   3: R + z   4: z / max(deg, 1)
- * Z (optional) receives z. */
+ * EPI 0: z   3: R + z   4: z / max(deg, 1) */
 template <int K1, int K2, int EPI, bool MASK>
 __global__ __launch_bounds__(64) void k_dense32(uint32_t N, const float *__restrict__ X1, const float *__restrict__ X2,
                                                 const float *__restrict__ M1, const unsigned short *__restrict__ W,
                                                 const float *__restrict__ bias, const float *__restrict__ R,
-                                                const uint32_t *__restrict__ deg, float *__restrict__ Z,
-                                                float *__restrict__ Y)
+                                                const uint32_t *__restrict__ deg, float *__restrict__ Y)
 {
   constexpr int K = K1 + K2;
   static_assert(K1 % 8 == 0 && K2 % 8 == 0, "k-steps of 8");
@@ -145,15 +143,142 @@ __global__ __launch_bounds__(64) void k_dense32(uint32_t N, const float *__restr
     if (row >= N) continue;
     const size_t o = (size_t)row * MP_H + li;
     const float z = acc[r] + b;
-    if (Z) Z[o] = z;
     float y;
     if (EPI == 0) y = z;
-    else if (EPI == 1) y = fmaxf(z, 0.0f);
-    else if (EPI == 2) y = R[o] + fmaxf(z, 0.0f);
     else if (EPI == 3) y = R[o] + z;
     else y = z * (1.0f / (float)max(deg[row], 1u));
     Y[o] = y;
   }
+}
+
+/* ---- the context network's dense layers, 32 vertices per wavefront ------------
+ *
+ * Layers that follow one another on the same vertices run in one kernel on
+ * registers.  The product is formed transposed, D = W X^T, so that lane l
+ * holds vertex row0 + l % 32 and D's register 4 q + j holds output channel
+ * 8 q + 4 (l / 32) + j -- exactly the B operand of the next layer's k-step q,
+ * with no exchange between lanes; memory sees 16-byte loads and stores.  The
+ * k-steps run in k_dense32's order, so every value has its bits.  Bound by
+ * the activations' bytes (backward reads them all): the first kernel moves
+ * 640 bytes a vertex, a round 768.  331,776 vertices: 46 us and 68 us (3.8
+ * TB/s) against 115 us (features and three layers) and 185 us (three layers)
+ * with a kernel per layer; 112,035: 17 and 22 us against 56 and 73 us. */
+__device__ __forceinline__ bf16x4 mp_bf4(const float *x)
+{
+  bf16x4 v;
+#pragma unroll
+  for (int j = 0; j < 4; j++) v[j] = (short)f2bf(x[j]);
+  return v;
+}
+
+/* acc += W[.][k0 ...] x for S k-steps; x: the lane's 4 S channels, W row-major
+ * with row stride K */
+template <int S, int K>
+__device__ __forceinline__ f32x16 mp_mm(const unsigned short *__restrict__ W, int k0, const float *x, f32x16 acc)
+{
+  const uint32_t li = threadIdx.x & 31u, h4 = (threadIdx.x & 32u) >> 3;
+#pragma unroll
+  for (int s = 0; s < S; s++) {
+    const bf16x4 a = *reinterpret_cast<const bf16x4 *>(W + li * K + k0 + 8 * s + h4);
+    acc = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(a, mp_bf4(x + 4 * s), acc, 0, 0, 0);
+  }
+  return acc;
+}
+
+__device__ __forceinline__ f32x16 mp_zero()
+{
+  f32x16 z;
+#pragma unroll
+  for (int r = 0; r < 16; r++) z[r] = 0.0f;
+  return z;
+}
+
+/* the lane's 16 channels of row n of a [N][32] array, and back */
+__device__ __forceinline__ void mp_row_ld(const float *__restrict__ X, uint32_t n, float x[16])
+{
+  const float4 *p = reinterpret_cast<const float4 *>(X + (size_t)n * MP_H + ((threadIdx.x & 32u) >> 3));
+#pragma unroll
+  for (int q = 0; q < 4; q++) {
+    const float4 t = p[2 * q];
+    x[4 * q] = t.x; x[4 * q + 1] = t.y; x[4 * q + 2] = t.z; x[4 * q + 3] = t.w;
+  }
+}
+
+__device__ __forceinline__ void mp_row_st(float *__restrict__ X, uint32_t n, const float x[16])
+{
+  float4 *p = reinterpret_cast<float4 *>(X + (size_t)n * MP_H + ((threadIdx.x & 32u) >> 3));
+#pragma unroll
+  for (int q = 0; q < 4; q++) p[2 * q] = make_float4(x[4 * q], x[4 * q + 1], x[4 * q + 2], x[4 * q + 3]);
+}
+
+/* acc + b per channel (b NULL: + 0, as k_dense32 adds) */
+__device__ __forceinline__ void mp_bias(const f32x16 &acc, const float *__restrict__ b, float z[16])
+{
+  const float4 *p = reinterpret_cast<const float4 *>(b + ((threadIdx.x & 32u) >> 3));
+#pragma unroll
+  for (int q = 0; q < 4; q++) {
+    const float4 t = b ? p[2 * q] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    z[4 * q] = acc[4 * q] + t.x; z[4 * q + 1] = acc[4 * q + 1] + t.y;
+    z[4 * q + 2] = acc[4 * q + 2] + t.z; z[4 * q + 3] = acc[4 * q + 3] + t.w;
+  }
+}
+
+#define MP_TW (MP_RB / 64)   /* tiles of 32 vertices per workgroup, one per wavefront */
+
+/* x = D / sd, z0 = W0 x + b0, h = relu(z0), P = A h, Q = B h */
+__global__ __launch_bounds__(MP_RB) void k_mp_in(uint32_t N, const float *__restrict__ D,
+                                                 const float *__restrict__ isd_p, const unsigned short *__restrict__ wb,
+                                                 const float *__restrict__ theta, float *__restrict__ X,
+                                                 float *__restrict__ Z0, float *__restrict__ H, float *__restrict__ P,
+                                                 float *__restrict__ Q)
+{
+  const uint32_t v = (kf_xcd_block() * MP_TW + (threadIdx.x >> 6)) * 32u + (threadIdx.x & 31u);
+  const uint32_t n = min(v, N - 1), h4 = (threadIdx.x & 32u) >> 3;
+  const bool on = v < N;
+  const float isd = *isd_p;
+  float x[8], z[16], y[16];
+#pragma unroll
+  for (int s = 0; s < 2; s++) {
+    const float4 t = *reinterpret_cast<const float4 *>(D + (size_t)n * MP_NIN + 8 * s + h4);
+    x[4 * s] = t.x * isd; x[4 * s + 1] = t.y * isd; x[4 * s + 2] = t.z * isd; x[4 * s + 3] = t.w * isd;
+    if (on)
+      *reinterpret_cast<float4 *>(X + (size_t)n * MP_NIN + 8 * s + h4) =
+          make_float4(x[4 * s], x[4 * s + 1], x[4 * s + 2], x[4 * s + 3]);
+  }
+  mp_bias(mp_mm<2, MP_NIN>(wb + MPB_W0, 0, x, mp_zero()), theta + MP_B0, z);
+#pragma unroll
+  for (int r = 0; r < 16; r++) y[r] = fmaxf(z[r], 0.0f);
+  if (on) { mp_row_st(Z0, n, z); mp_row_st(H, n, y); }
+  mp_bias(mp_mm<4, MP_H>(wb + MPB_A(0), 0, y, mp_zero()), NULL, z);
+  if (on) mp_row_st(P, n, z);
+  mp_bias(mp_mm<4, MP_H>(wb + MPB_B(0), 0, y, mp_zero()), NULL, z);
+  if (on) mp_row_st(Q, n, z);
+}
+
+/* zu = U h + V m + u, h' = h + relu(zu), then P = W1 h' + b1 and Q = W2 h':
+ * the next round's A and B, or after the last round the heads WSA and Wb */
+__global__ __launch_bounds__(MP_RB) void k_mp_update(uint32_t N, const float *__restrict__ H,
+                                                     const float *__restrict__ M, const unsigned short *__restrict__ UV,
+                                                     const float *__restrict__ ub, const unsigned short *__restrict__ W1,
+                                                     const float *__restrict__ b1, const unsigned short *__restrict__ W2,
+                                                     float *__restrict__ ZU, float *__restrict__ Hn,
+                                                     float *__restrict__ P, float *__restrict__ Q)
+{
+  const uint32_t v = (kf_xcd_block() * MP_TW + (threadIdx.x >> 6)) * 32u + (threadIdx.x & 31u);
+  const uint32_t n = min(v, N - 1);
+  const bool on = v < N;
+  float h[16], m[16], z[16];
+  mp_row_ld(H, n, h);
+  mp_row_ld(M, n, m);
+  f32x16 acc = mp_mm<4, 2 * MP_H>(UV, 0, h, mp_zero());
+  mp_bias(mp_mm<4, 2 * MP_H>(UV, MP_H, m, acc), ub, z);
+#pragma unroll
+  for (int r = 0; r < 16; r++) h[r] = h[r] + fmaxf(z[r], 0.0f);
+  if (on) { mp_row_st(ZU, n, z); mp_row_st(Hn, n, h); }
+  mp_bias(mp_mm<4, MP_H>(W1, 0, h, mp_zero()), b1, z);
+  if (on) mp_row_st(P, n, z);
+  mp_bias(mp_mm<4, MP_H>(W2, 0, h, mp_zero()), NULL, z);
+  if (on) mp_row_st(Q, n, z);
 }
 
 /* ---- weight gradients on the matrix cores --------------------------------------
@@ -268,14 +393,6 @@ __global__ __launch_bounds__(MP_RB) void k_mp_take_diag(uint32_t N, const uint32
   const size_t k = (size_t)blockIdx.x * MP_RB + threadIdx.x;
   if (k >= 16 * (size_t)N) return;
   D[k] = (float)a[16 * (size_t)diag[k >> 4] + (k & 15)];
-}
-
-/* x_n = D_n / sd */
-__global__ __launch_bounds__(MP_RB) void k_mp_features(size_t n, const float *__restrict__ D,
-                                                       const float *__restrict__ isd_p, float *__restrict__ X)
-{
-  const size_t k = (size_t)blockIdx.x * MP_RB + threadIdx.x;
-  if (k < n) X[k] = D[k] * *isd_p;
 }
 
 /* signed edge vector of every sliced-ELL slot: (nx, ny, nz) area, negated
@@ -818,29 +935,20 @@ static void mp_context(kf_mpnn *net, int slot)
 {
   kf_ctx *c = net->c;
   hipStream_t st = c->stream;
-  const uint32_t N = net->N, nw = kf_blocks_for(N, 32);
-  const float *nf = NULL;
-  const uint32_t *nu = NULL;
-  float *nz = NULL;
-  hipLaunchKernelGGL(k_mp_features, dim3(kf_blocks_for(16 * (size_t)N, MP_RB)), dim3(MP_RB), 0, st,
-                     16 * (size_t)N, net->dstore + (size_t)slot * 16 * N, net->isd + slot, net->X);
-  hipLaunchKernelGGL((k_dense32<MP_NIN, 0, 1, false>), dim3(nw), dim3(64), 0, st, N, net->X, nf, nf,
-                     net->wb + MPB_W0, net->theta + MP_B0, nf, nu, net->Z0, net->H[0]);
+  const uint32_t N = net->N, nt = kf_blocks_for(N, 32 * MP_TW);
+  const float *th = net->theta, *nf = NULL;
+  const unsigned short *wb = net->wb;
+  hipLaunchKernelGGL(k_mp_in, dim3(nt), dim3(MP_RB), 0, st, N, net->dstore + (size_t)slot * 16 * N, net->isd + slot, wb,
+                     th, net->X, net->Z0, net->H[0], net->P[0], net->Q[0]);
   for (int l = 0; l < MP_NR; l++) {
-    hipLaunchKernelGGL((k_dense32<MP_H, 0, 0, false>), dim3(nw), dim3(64), 0, st, N, net->H[l], nf, nf,
-                       net->wb + MPB_A(l), nf, nf, nu, nz, net->P[l]);
-    hipLaunchKernelGGL((k_dense32<MP_H, 0, 0, false>), dim3(nw), dim3(64), 0, st, N, net->H[l], nf, nf,
-                       net->wb + MPB_B(l), nf, nf, nu, nz, net->Q[l]);
+    const bool last = l == MP_NR - 1;
     hipLaunchKernelGGL(k_mp_message, dim3(kf_blocks_for(N, MP_VW)), dim3(MP_RB), 0, st, c->d, net->ev, net->P[l],
-                       net->Q[l], net->theta, (uint32_t)MP_C(l), (uint32_t)MP_CB(l), net->M[l], net->pos[l],
-                       net->words);
-    hipLaunchKernelGGL((k_dense32<MP_H, MP_H, 2, false>), dim3(nw), dim3(64), 0, st, N, net->H[l], net->M[l], nf,
-                       net->wb + MPB_UV(l), net->theta + MP_UB(l), net->H[l], nu, net->ZU[l], net->H[l + 1]);
+                       net->Q[l], th, (uint32_t)MP_C(l), (uint32_t)MP_CB(l), net->M[l], net->pos[l], net->words);
+    hipLaunchKernelGGL(k_mp_update, dim3(nt), dim3(MP_RB), 0, st, N, net->H[l], net->M[l], wb + MPB_UV(l),
+                       th + MP_UB(l), wb + (last ? MPB_WSA : MPB_A(l + 1)), last ? th + MP_BSA : nf,
+                       wb + (last ? MPB_WB : MPB_B(l + 1)), net->ZU[l], net->H[l + 1], last ? net->OP1 : net->P[l + 1],
+                       last ? net->OPQ : net->Q[l + 1]);
   }
-  hipLaunchKernelGGL((k_dense32<MP_H, 0, 0, false>), dim3(nw), dim3(64), 0, st, N, net->H[MP_NR], nf, nf,
-                     net->wb + MPB_WSA, net->theta + MP_BSA, nf, nu, nz, net->OP1);
-  hipLaunchKernelGGL((k_dense32<MP_H, 0, 0, false>), dim3(nw), dim3(64), 0, st, N, net->H[MP_NR], nf, nf,
-                     net->wb + MPB_WB, nf, nf, nu, nz, net->OPQ);
   KF_LAUNCH_CHECK();
   net->prepared = slot;
 }
@@ -857,7 +965,6 @@ static void mp_loss_grad(kf_mpnn *net, int slot, const double *v, const double *
   const uint32_t nb4 = kf_blocks_for(n4, MP_RB);
   const float *nf = NULL;
   const uint32_t *nu = NULL;
-  float *nz = NULL;
   const int metric = net->metric;
   const float *A = net->mslot[slot];
   if (metric >= 1 && !A) {
@@ -889,7 +996,7 @@ static void mp_loss_grad(kf_mpnn *net, int slot, const double *v, const double *
   hipLaunchKernelGGL((k_wgrad<4, 12, 4, 12, false>), dim3(P), dim3(64), 0, st, N, ch, net->gd, nf, net->Ez,
                      net->part, (uint32_t)MP_WE, -1);
   hipLaunchKernelGGL((k_dense32<MP_H, MP_H, 0, false>), dim3(nw), dim3(64), 0, st, N, net->dOP1, net->dOPQ, nf,
-                     net->wb + MPB_HT, nf, nf, nu, nz, net->dh);
+                     net->wb + MPB_HT, nf, nf, nu, net->dh);
   for (int l = MP_NR - 1; l >= 0; l--) {
     /* dzu = dh [zu > 0]: gradients of U, u and V */
     hipLaunchKernelGGL((k_wgrad<MP_H, MP_H, MP_H, MP_H, true>), dim3(P), dim3(64), 0, st, N, ch, net->dh, net->ZU[l],
@@ -898,9 +1005,9 @@ static void mp_loss_grad(kf_mpnn *net, int slot, const double *v, const double *
                        net->M[l], net->part, (uint32_t)MP_V(l), -1);
     /* dhn = dh + dzu U;  dm = (dzu V) / deg */
     hipLaunchKernelGGL((k_dense32<MP_H, 0, 3, true>), dim3(nw), dim3(64), 0, st, N, net->dh, nf, net->ZU[l],
-                       net->wb + MPB_UT(l), nf, net->dh, nu, nz, net->dhn);
+                       net->wb + MPB_UT(l), nf, net->dh, nu, net->dhn);
     hipLaunchKernelGGL((k_dense32<MP_H, 0, 4, true>), dim3(nw), dim3(64), 0, st, N, net->dh, nf, net->ZU[l],
-                       net->wb + MPB_VT(l), nf, nf, c->d.deg, nz, net->dm);
+                       net->wb + MPB_VT(l), nf, nf, c->d.deg, net->dm);
     hipLaunchKernelGGL(k_mp_message_bwd, dim3(P), dim3(MP_RB), 0, st, c->d, ch, net->ev, net->pos[l], net->words,
                        net->dm, (uint32_t)MP_C(l), (uint32_t)MP_CB(l), net->dP, net->dQ, net->part);
     hipLaunchKernelGGL((k_wgrad<MP_H, MP_H, MP_H, MP_H, false>), dim3(P), dim3(64), 0, st, N, ch, net->dP, nf,
@@ -909,7 +1016,7 @@ static void mp_loss_grad(kf_mpnn *net, int slot, const double *v, const double *
                        net->H[l], net->part, (uint32_t)MP_B(l), -1);
     /* dh = dhn + dP A + dQ B */
     hipLaunchKernelGGL((k_dense32<MP_H, MP_H, 3, false>), dim3(nw), dim3(64), 0, st, N, net->dP, net->dQ, nf,
-                       net->wb + MPB_ABT(l), nf, net->dhn, nu, nz, net->dh);
+                       net->wb + MPB_ABT(l), nf, net->dhn, nu, net->dh);
   }
   hipLaunchKernelGGL((k_wgrad<MP_H, MP_NIN, MP_H, MP_NIN, true>), dim3(P), dim3(64), 0, st, N, ch, net->dh, net->Z0,
                      net->X, net->part, (uint32_t)MP_W0, (int)MP_B0);
