@@ -36,7 +36,7 @@
 #include <math.h>
 #include <string.h>
 
-#include "kf_dev.h"
+#include "sync.h"
 
 #define MP_H 32
 #define MP_NIN 16 /* inputs: one diagonal block (a multiple of the MFMA k-step) */
@@ -85,6 +85,8 @@ static_assert(MP_NPARAM == 14928, "parameter layout of the network");
 
 typedef short bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 hwbf4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ unsigned short f2bf(float x)
 {
@@ -93,82 +95,27 @@ __device__ __forceinline__ unsigned short f2bf(float x)
   return (unsigned short)(u >> 16);
 }
 
-/* ---- dense layer on the matrix cores ----------------------------------------
- * Y[n][o] = epi(sum_k X[n][k] W[o][k] + bias[o]) for o < 32 and k < K1 + K2:
- * the first K1 columns come from X1 (row stride K1), the rest from X2 (row
- * stride K2).  MASK: X1[n][k] counts only where M1[n][k] > 0 (the ReLU
- * derivative in backward).  One wavefront computes 32 rows.
- * Operand layout of v_mfma_f32_32x32x8_bf16 (lane l, element j < 4):
- *   A: X[row0 + l % 32][8 s + 4 (l / 32) + j]
- *   B: W[l % 32][8 s + 4 (l / 32) + j]
- *   D: register r holds Y[row0 + 8 (r / 4) + 4 (l / 32) + r % 4][l % 32]
- * EPI 0: z   3: R + z   4: z / max(deg, 1) */
-template <int K1, int K2, int EPI, bool MASK>
-__global__ __launch_bounds__(64) void k_dense32(uint32_t N, const float *__restrict__ X1, const float *__restrict__ X2,
-                                                const float *__restrict__ M1, const unsigned short *__restrict__ W,
-                                                const float *__restrict__ bias, const float *__restrict__ R,
-                                                const uint32_t *__restrict__ deg, float *__restrict__ Y)
-{
-  constexpr int K = K1 + K2;
-  static_assert(K1 % 8 == 0 && K2 % 8 == 0, "k-steps of 8");
-  const uint32_t lane = threadIdx.x, li = lane & 31u, lk = (lane >> 5) * 4u;
-  const uint32_t row0 = blockIdx.x * 32u, n = row0 + li;
-  f32x16 acc;
-#pragma unroll
-  for (int r = 0; r < 16; r++) acc[r] = 0.0f;
-#pragma unroll
-  for (int s = 0; s < K / 8; s++) {
-    const int k = 8 * s + (int)lk;
-    bf16x4 av, bv;
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-      float x = 0.0f;
-      if (n < N) {
-        if (k < K1) {
-          x = X1[(size_t)n * K1 + k + j];
-          if (MASK && !(M1[(size_t)n * K1 + k + j] > 0.0f)) x = 0.0f;
-        } else {
-          x = X2[(size_t)n * K2 + (k - K1) + j];
-        }
-      }
-      av[j] = (short)f2bf(x);
-      bv[j] = (short)W[li * K + k + j];
-    }
-    acc = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(av, bv, acc, 0, 0, 0);
-  }
-  const float b = bias ? bias[li] : 0.0f;
-#pragma unroll
-  for (int r = 0; r < 16; r++) {
-    const uint32_t row = row0 + 8u * (r / 4) + lk + (r % 4);
-    if (row >= N) continue;
-    const size_t o = (size_t)row * MP_H + li;
-    const float z = acc[r] + b;
-    float y;
-    if (EPI == 0) y = z;
-    else if (EPI == 3) y = R[o] + z;
-    else y = z * (1.0f / (float)max(deg[row], 1u));
-    Y[o] = y;
-  }
-}
-
 /* ---- the context network's dense layers, 32 vertices per wavefront ------------
  *
  * Layers that follow one another on the same vertices run in one kernel on
  * registers.  The product is formed transposed, D = W X^T, so that lane l
  * holds vertex row0 + l % 32 and D's register 4 q + j holds output channel
  * 8 q + 4 (l / 32) + j -- exactly the B operand of the next layer's k-step q,
- * with no exchange between lanes; memory sees 16-byte loads and stores.  The
- * k-steps run in k_dense32's order, so every value has its bits.  Bound by
+ * with no exchange between lanes; memory sees 16-byte loads and stores.
+ * Operand layout of v_mfma_f32_32x32x8_bf16 (lane l, element j < 4):
+ *   A: W[l % 32][8 s + 4 (l / 32) + j]
+ *   B: X[row0 + l % 32][8 s + 4 (l / 32) + j]
+ * The k-steps run in ascending s from a zero accumulator.  Bound by
  * the activations' bytes (backward reads them all): the first kernel moves
  * 640 bytes a vertex, a round 768.  331,776 vertices: 46 us and 68 us (3.8
  * TB/s) against 115 us (features and three layers) and 185 us (three layers)
  * with a kernel per layer; 112,035: 17 and 22 us against 56 and 73 us. */
 __device__ __forceinline__ bf16x4 mp_bf4(const float *x)
 {
-  bf16x4 v;
-#pragma unroll
-  for (int j = 0; j < 4; j++) v[j] = (short)f2bf(x[j]);
-  return v;
+  const f32x4 f = {x[0], x[1], x[2], x[3]};
+  union { hwbf4 h; bf16x4 s; } u;
+  u.h = __builtin_convertvector(f, hwbf4);   /* v_cvt_pk_bf16_f32: to nearest, ties to even */
+  return u.s;
 }
 
 /* acc += W[.][k0 ...] x for S k-steps; x: the lane's 4 S channels, W row-major
@@ -211,7 +158,7 @@ __device__ __forceinline__ void mp_row_st(float *__restrict__ X, uint32_t n, con
   for (int q = 0; q < 4; q++) p[2 * q] = make_float4(x[4 * q], x[4 * q + 1], x[4 * q + 2], x[4 * q + 3]);
 }
 
-/* acc + b per channel (b NULL: + 0, as k_dense32 adds) */
+/* acc + b per channel (b NULL: + 0) */
 __device__ __forceinline__ void mp_bias(const f32x16 &acc, const float *__restrict__ b, float z[16])
 {
   const float4 *p = reinterpret_cast<const float4 *>(b + ((threadIdx.x & 32u) >> 3));
@@ -282,65 +229,102 @@ __global__ __launch_bounds__(MP_RB) void k_mp_update(uint32_t N, const float *__
 }
 
 /* ---- weight gradients on the matrix cores --------------------------------------
- * For vertex partition p = blockIdx.x (vertices [p chunk, (p+1) chunk)):
- *   part[p][offw + o KX + k] = sum_n dY[n][o] X[n][k]      o < OY, k < KX
- *   part[p][offb + o]        = sum_n dY[n][o]              (offb >= 0)
- * dY has row stride DYW, X row stride XW; MASK: dY[n][o] counts only where
- * Mz[n][o] > 0 (Mz with dY's layout).  The k dimension of the MFMA runs
- * over 8 vertices at a time:
- *   A: dY[n0 + 4 (l / 32) + j][l % 32]      (rows: o)
- *   B: X[n0 + 4 (l / 32) + j][l % 32]       (columns: k)
- * The bias sums are taken of the unrounded FP32 values. */
-template <int DYW, int XW, int OY, int KX, bool MASK>
-__global__ __launch_bounds__(64) void k_wgrad(uint32_t N, uint32_t chunk, const float *__restrict__ dY,
-                                              const float *__restrict__ Mz, const float *__restrict__ X,
-                                              float *__restrict__ part, uint32_t offw, int offb)
+ *
+ * A weight gradient sum_n dY[n][o] X[n][k] is a product over vertices, whose
+ * operands want a lane per channel; the dense layers hold a lane per vertex.
+ * Each wavefront turns its 32 x 32 tiles in LDS: rows are channels, MP_TS
+ * bfloat16 values apart (72 bytes: the rows of 32 lanes start in different
+ * banks), and the sums stay in registers over all of the wavefront's tiles.
+ * With one wavefront per 328 vertices reading both operands again from memory
+ * for every gradient, a pair of them took 160 us a round on 331,776 vertices. */
+#define MP_TS 36
+
+template <int Q>
+__device__ __forceinline__ void mp_tile_put(short *T, const float *x)
 {
-  static_assert(OY <= 32 && OY <= DYW && KX <= 32 && KX <= XW, "one 32 x 32 tile");
-  const uint32_t lane = threadIdx.x, li = lane & 31u, lk = (lane >> 5) * 4u;
-  const uint32_t p = blockIdx.x, n0 = p * chunk, n1 = min(N, n0 + chunk);
-  f32x16 acc;
+  const uint32_t li = threadIdx.x & 31u, h4 = (threadIdx.x & 32u) >> 3;
 #pragma unroll
-  for (int r = 0; r < 16; r++) acc[r] = 0.0f;
-  float bsum = 0.0f;
-  for (uint32_t nb = n0; nb < n1; nb += 8) {
-    bf16x4 av, bv;
+  for (int q = 0; q < Q; q++) {
+    const bf16x4 b = mp_bf4(x + 4 * q);
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
-      const uint32_t n = nb + lk + j;
-      float y = 0.0f, x = 0.0f;
-      if (n < n1) {
-        if (li < (uint32_t)OY) {
-          y = dY[(size_t)n * DYW + li];
-          if (MASK && !(Mz[(size_t)n * DYW + li] > 0.0f)) y = 0.0f;
-        }
-        if (li < (uint32_t)KX) x = X[(size_t)n * XW + li];
-      }
-      bsum += y;
-      av[j] = (short)f2bf(y);
-      bv[j] = (short)f2bf(x);
-    }
-    acc = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(av, bv, acc, 0, 0, 0);
+    for (int j = 0; j < 4; j++) T[(8 * q + h4 + j) * MP_TS + li] = b[j];
   }
-  bsum += __shfl_xor(bsum, 32);
-  float *pp = part + (size_t)p * MP_NPARAM;
-#pragma unroll
-  for (int r = 0; r < 16; r++) {
-    const uint32_t o = 8u * (r / 4) + lk + (r % 4);
-    if (o < (uint32_t)OY && li < (uint32_t)KX) pp[offw + o * KX + li] = acc[r];
-  }
-  if (offb >= 0 && lane < (uint32_t)OY) pp[offb + lane] = bsum;
 }
 
-/* grad[i] = sum over partitions of part[p][i], in partition order (FP64) */
-__global__ __launch_bounds__(MP_RB) void k_mp_grad_reduce(const float *__restrict__ part, uint32_t nparts,
-                                                          float *__restrict__ grad)
+/* the operand of lane l for vertices 8 t + 4 (l / 32) + j: row `row`, or 0 */
+__device__ __forceinline__ bf16x4 mp_tile_get(const short *T, uint32_t row, bool on, int t)
 {
-  const uint32_t i = blockIdx.x * MP_RB + threadIdx.x;
-  if (i >= MP_NPARAM) return;
+  const bf16x4 z = {0, 0, 0, 0};
+  return on ? *reinterpret_cast<const bf16x4 *>(T + row * MP_TS + 8 * t + ((threadIdx.x & 32u) >> 3)) : z;
+}
+
+/* acc[o][k] += sum over the tile's vertices of A[o] B[k], o < OY, k < KX */
+template <int OY, int KX>
+__device__ __forceinline__ f32x16 mp_tile_mm(const short *A, const short *B, f32x16 acc)
+{
+  const uint32_t li = threadIdx.x & 31u;
+#pragma unroll
+  for (int t = 0; t < 4; t++)
+    acc = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(mp_tile_get(A, OY < 32 ? min(li, OY - 1u) : li, OY == 32 || li < OY, t),
+                                                   mp_tile_get(B, KX < 32 ? min(li, KX - 1u) : li, KX == 32 || li < KX, t),
+                                                   acc, 0, 0, 0);
+  return acc;
+}
+
+/* the workgroup's sums of a weight gradient (o < OY, k < KX) into
+ * out[o KX + k], wavefronts in order; sh holds MP_TW x 1024 floats */
+template <int OY, int KX>
+__device__ __forceinline__ void mp_wsum(const f32x16 &acc, float *sh, float *__restrict__ out)
+{
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < 16; r++) sh[(threadIdx.x >> 6) * 1024 + 64 * r + (threadIdx.x & 63u)] = acc[r];
+  __syncthreads();
+  for (uint32_t e = threadIdx.x; e < 1024; e += MP_RB) {
+    float t = 0.0f;
+    for (int w = 0; w < MP_TW; w++) t += sh[1024 * w + e];
+    const uint32_t r = e >> 6, o = 8 * (r >> 2) + ((e & 32u) >> 3) + (r & 3u), k = e & 31u;
+    if (o < (uint32_t)OY && k < (uint32_t)KX) out[o * KX + k] = t;
+  }
+}
+
+/* the workgroup's sums of the lanes' 16 channels over all vertices */
+__device__ __forceinline__ void mp_bsum(const float b[16], float *sh, float *__restrict__ out)
+{
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < 16; r++) {
+    float x = b[r];
+#pragma unroll
+    for (int m = 1; m < 32; m <<= 1) x += __shfl_xor(x, m, 64);
+    if ((threadIdx.x & 31u) == 0) sh[(threadIdx.x >> 6) * 32 + 8 * (r >> 2) + ((threadIdx.x & 32u) >> 3) + (r & 3)] = x;
+  }
+  __syncthreads();
+  if (threadIdx.x < 32) {
+    float t = 0.0f;
+    for (int w = 0; w < MP_TW; w++) t += sh[32 * w + threadIdx.x];
+    out[threadIdx.x] = t;
+  }
+}
+
+/* grad[i] = sum over partitions of part[p][i] (FP64): a workgroup takes 64
+ * parameters, its 16 wavefronts every 16th partition each, then the
+ * wavefronts in order (943 partitions: 30 us, against 396 us for one thread
+ * per parameter) */
+__global__ __launch_bounds__(1024) void k_mp_grad_reduce(const float *__restrict__ part, uint32_t nparts,
+                                                         float *__restrict__ grad)
+{
+  __shared__ double sh[16][64];
+  const uint32_t lane = threadIdx.x & 63u, w = threadIdx.x >> 6, i = blockIdx.x * 64u + lane;
   double acc = 0.0;
-  for (uint32_t p = 0; p < nparts; p++) acc += (double)part[(size_t)p * MP_NPARAM + i];
-  grad[i] = (float)acc;
+  if (i < MP_NPARAM)
+    for (uint32_t p = w; p < nparts; p += 16) acc += (double)part[(size_t)p * MP_NPARAM + i];
+  sh[w][lane] = acc;
+  __syncthreads();
+  if (w == 0 && i < MP_NPARAM) {
+    for (int k = 1; k < 16; k++) acc += sh[k][lane];
+    grad[i] = (float)acc;
+  }
 }
 
 /* ---- reductions and features ---------------------------------------------------- */
@@ -399,7 +383,7 @@ __global__ __launch_bounds__(MP_RB) void k_mp_take_diag(uint32_t N, const uint32
  * where the vertex is the edge's second end; the fourth word holds the edge's
  * place in the neighbour's own list (an integer), where the backward pass
  * finds the message that went the other way */
-__global__ __launch_bounds__(MP_RB) void k_mp_edge_vectors(kf_dv d, float4 *__restrict__ ev)
+__global__ __launch_bounds__(MP_RB) void k_mp_edge_vectors(kf_dv d, float4 *__restrict__ ev, float *__restrict__ ideg)
 {
   const uint32_t v = blockIdx.x * MP_RB + threadIdx.x;
   if (v >= d.N) return;
@@ -413,6 +397,7 @@ __global__ __launch_bounds__(MP_RB) void k_mp_edge_vectors(kf_dv d, float4 *__re
     while (kr + 1 < d.deg[u] && d.sell_ent[ui + 64 * (size_t)kr] != (ent ^ 1u)) kr++;   /* u holds the other side */
     ev[idx] = make_float4((float)(eg.xn * ar), (float)(eg.yn * ar), (float)(eg.zn * ar), __uint_as_float(kr));
   }
+  ideg[v] = 1.0f / (float)max(d.deg[v], 1u);
 }
 
 /* ---- messages ------------------------------------------------------------------ */
@@ -647,58 +632,258 @@ __global__ __launch_bounds__(MP_RB) void k_mp_apply(kf_dv d, const float4 *__res
   }
 }
 
-/* Backward of the correction given gv = dL/d delta (N x 4, FP32) and z:
- *   dOP1_v = [g_v z_v^T | (g_v / deg v) zs_v^T]       (N x 32)
- *   dOPQ_v = [gbar_v z_v^T | 0],  gbar_v = sum_u g_u / deg u   (N x 32)
- *   gd_v   = g_v / deg v (N x 4),  Ez_v (N x 12, [j][k] as 3 j + k)
- * (the gradient of We is then sum_v gd_v Ez_v^T, a weight gradient). */
-__global__ __launch_bounds__(MP_RB) void k_mp_apply_bwd(kf_dv d, const float4 *__restrict__ ev,
-                                                        const double *__restrict__ z, const float *__restrict__ gv,
-                                                        float *__restrict__ dOP1, float *__restrict__ dOPQ,
-                                                        float *__restrict__ gd, float *__restrict__ Ez)
+/* ---- backward of the dense layers, per vertex partition -------------------------
+ *
+ * blockIdx.x is a partition of `chunk` vertices (a multiple of 32), its
+ * wavefronts take tiles of 32 vertices in turn, and the layers of the context
+ * network run backward on registers as in k_mp_update; the weight gradients
+ * of the partition go to part[p].  Everything that follows on a vertex's own
+ * values is one kernel; the messages' backward, which gathers, lies between.
+ * Bound by the bytes: 1.1 KB a vertex and round, 91 us on 331,776 vertices
+ * (4.1 TB/s), where a kernel per layer and gradient took 530 us.  The sums of
+ * four gradients leave two wavefronts per SIMD (256 registers). */
+
+/* dzu = dh where zu > 0; dhn = dh + dzu U, dm = (dzu V) / deg; tiles of dzu,
+ * h and m for the gradients of U and V; bu += dzu */
+__device__ __forceinline__ void mp_update_bwd(const float dh[16], uint32_t n, bool on, const float *__restrict__ ZU,
+                                              const float *__restrict__ H, const float *__restrict__ M,
+                                              const unsigned short *__restrict__ wut,
+                                              const unsigned short *__restrict__ wvt, float idg,
+                                              float *__restrict__ dhn, float *__restrict__ dm, short *T, float bu[16],
+                                              f32x16 &gu, f32x16 &gv)
 {
-  const uint32_t v = blockIdx.x * MP_RB + threadIdx.x;
-  if (v >= d.N) return;
-  const uint32_t deg = d.deg[v];
-  size_t idx = (size_t)d.sell_ptr[v >> 6] * 64u + (v & 63u);
-  float zs[4] = {0.0f, 0.0f, 0.0f, 0.0f}, gb[4] = {0.0f, 0.0f, 0.0f, 0.0f}, ez[12];
+  float x[16], z[16];
+  mp_row_ld(ZU, n, x);
 #pragma unroll
-  for (int i = 0; i < 12; i++) ez[i] = 0.0f;
-  for (uint32_t k = 0; k < deg; k++, idx += 64) {
-    const uint32_t u = d.sell_nbr[idx];
-    const float4 e = ev[idx], zu4 = ld4(z, u), gu = *(const float4 *)(gv + 4 * (size_t)u);
-    const float iu = 1.0f / (float)max(d.deg[u], 1u);
-    const float zu[4] = {zu4.x, zu4.y, zu4.z, zu4.w};
-    gb[0] += gu.x * iu;
-    gb[1] += gu.y * iu;
-    gb[2] += gu.z * iu;
-    gb[3] += gu.w * iu;
+  for (int r = 0; r < 16; r++) {
+    x[r] = on && x[r] > 0.0f ? dh[r] : 0.0f;
+    bu[r] += x[r];
+  }
+  mp_bias(mp_mm<4, MP_H>(wut, 0, x, mp_zero()), NULL, z);
+#pragma unroll
+  for (int r = 0; r < 16; r++) z[r] = dh[r] + z[r];
+  if (on) mp_row_st(dhn, n, z);
+  mp_bias(mp_mm<4, MP_H>(wvt, 0, x, mp_zero()), NULL, z);
+#pragma unroll
+  for (int r = 0; r < 16; r++) z[r] = z[r] * idg;
+  if (on) mp_row_st(dm, n, z);
+  wave_lds_sync();   /* the tiles' last readers are done */
+  mp_tile_put<4>(T, x);
+  mp_row_ld(H, n, z);
+  mp_tile_put<4>(T + 32 * MP_TS, z);
+  mp_row_ld(M, n, z);
+  mp_tile_put<4>(T + 64 * MP_TS, z);
+  wave_lds_sync();
+  gu = mp_tile_mm<32, 32>(T, T + 32 * MP_TS, gu);
+  gv = mp_tile_mm<32, 32>(T, T + 64 * MP_TS, gv);
+}
+
+#define MP_BWD_LDS (MP_TW * 4096)   /* bytes: the wavefronts' sums, or their 3 tiles of 2304 */
+#define MP_BWD_TILES (96 * MP_TS)   /* values: a wavefront's tiles */
+static_assert(MP_TW * MP_BWD_TILES * 2 <= 2 * MP_BWD_LDS, "the tiles fit");
+
+/* Backward of the correction given gv = dL/d delta (N x 4, FP32) and z:
+ *   dOP1_v = [g_v z_v^T | (g_v / deg v) zs_v^T]       zs_v = sum_u z_u
+ *   dOPQ_v = gbar_v z_v^T,  gbar_v = sum_u g_u / deg u
+ *   gd_v   = g_v / deg v,  Ez_v[3 j + k] = sum_u z_u[j] e_vu[k]
+ * (the gradient of We is sum_v gd_v Ez_v^T), the heads' weight gradients, dh
+ * = dOP1 WSA + dOPQ Wb, and the last round's update backward (148 us on
+ * 331,776 vertices; two gathers in flight took 197 us, separate kernels 470). */
+__global__ __launch_bounds__(MP_RB, 2) void k_mp_head_bwd(kf_dv d, uint32_t chunk, const float4 *__restrict__ ev,
+                                                       const float *__restrict__ ideg, const double *__restrict__ z,
+                                                       const float *__restrict__ gv, const unsigned short *__restrict__ wb,
+                                                       const float *__restrict__ Hl, const float *__restrict__ ZU,
+                                                       const float *__restrict__ H, const float *__restrict__ M,
+                                                       float *__restrict__ dhn, float *__restrict__ dm,
+                                                       float *__restrict__ part)
+{
+  __shared__ __align__(16) unsigned char lds[2 * MP_BWD_LDS];
+  short *T = reinterpret_cast<short *>(lds) + (threadIdx.x >> 6) * MP_BWD_TILES;
+  float *sh = reinterpret_cast<float *>(lds);
+  const uint32_t li = threadIdx.x & 31u, hf = (threadIdx.x >> 5) & 1u;
+  const uint32_t p = kf_xcd_block(), n0 = p * chunk, n1 = min(d.N, n0 + chunk);
+  f32x16 gs = mp_zero(), gq = mp_zero(), ge = mp_zero(), gu = mp_zero(), gw = mp_zero();
+  float bs[16], bu[16];
+#pragma unroll
+  for (int r = 0; r < 16; r++) bs[r] = bu[r] = 0.0f;
+  for (uint32_t row = n0 + 32 * (threadIdx.x >> 6); row < n1; row += 32 * MP_TW) {
+    const uint32_t v = min(row + li, n1 - 1);
+    const bool on = row + li < n1;
+    const uint32_t deg = d.deg[v];
+    const size_t base = (size_t)d.sell_ptr[v >> 6] * 64u + (v & 63u);
+    float zs[4] = {0.0f, 0.0f, 0.0f, 0.0f}, gb[4] = {0.0f, 0.0f, 0.0f, 0.0f}, ez[12];
+#pragma unroll
+    for (int i = 0; i < 12; i++) ez[i] = 0.0f;
+    /* four incidences' gathers in flight: at two wavefronts per SIMD their
+     * latency is what this kernel waits for */
+    for (uint32_t k0 = 0; k0 < deg; k0 += 4) {
+      uint32_t u[4];
+      float4 e[4], zu[4], gu4[4];
+      float iu[4];
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const size_t idx = base + 64 * (size_t)min(k0 + i, deg - 1);
+        u[i] = d.sell_nbr[idx];
+        e[i] = ev[idx];
+      }
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        zu[i] = ld4(z, u[i]);
+        gu4[i] = *(const float4 *)(gv + 4 * (size_t)u[i]);
+        iu[i] = ideg[u[i]];
+      }
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const bool in = k0 + i < deg;
+        const float zz[4] = {in ? zu[i].x : 0.0f, in ? zu[i].y : 0.0f, in ? zu[i].z : 0.0f, in ? zu[i].w : 0.0f};
+        gb[0] += (in ? gu4[i].x : 0.0f) * iu[i];
+        gb[1] += (in ? gu4[i].y : 0.0f) * iu[i];
+        gb[2] += (in ? gu4[i].z : 0.0f) * iu[i];
+        gb[3] += (in ? gu4[i].w : 0.0f) * iu[i];
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+          zs[j] += zz[j];
+          ez[3 * j] += zz[j] * e[i].x;
+          ez[3 * j + 1] += zz[j] * e[i].y;
+          ez[3 * j + 2] += zz[j] * e[i].z;
+        }
+      }
+    }
+    const float4 zv4 = ld4(z, v), g4 = *(const float4 *)(gv + 4 * (size_t)v);
+    const float idg = ideg[v];
+    const float zv[4] = {zv4.x, zv4.y, zv4.z, zv4.w}, g[4] = {g4.x, g4.y, g4.z, g4.w};
+    float gi[4], x1[16], x2[8], x3[12];
+#pragma unroll
+    for (int i = 0; i < 4; i++) gi[i] = on ? g[i] * idg : 0.0f;
+    /* the lane's channels 8 q + 4 (lane / 32) + j: row 2 q + lane / 32 of the
+     * 4 x 4 blocks, column j */
+#pragma unroll
+    for (int q = 0; q < 2; q++) {
+      const float a = on ? (hf ? g[2 * q + 1] : g[2 * q]) : 0.0f, b = hf ? gi[2 * q + 1] : gi[2 * q];
+      const float c = on ? (hf ? gb[2 * q + 1] : gb[2 * q]) : 0.0f;
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        x1[4 * q + j] = a * zv[j];
+        x1[8 + 4 * q + j] = b * zs[j];
+        x2[4 * q + j] = c * zv[j];
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < 16; r++) bs[r] += x1[r];
+    float hl[16], dh[16];
+    mp_row_ld(Hl, v, hl);
+    f32x16 acc = mp_mm<4, 2 * MP_H>(wb + MPB_HT, 0, x1, mp_zero());
+    acc = mp_mm<2, 2 * MP_H>(wb + MPB_HT, MP_H, x2, acc);   /* the padded half of Wb^T is 0 */
+    mp_bias(acc, NULL, dh);
+    wave_lds_sync();
+    mp_tile_put<4>(T, x1);
+    mp_tile_put<2>(T + 32 * MP_TS, x2);
+    mp_tile_put<4>(T + 64 * MP_TS, hl);
+    /* rows 48 .. 63: Ez (12) and gd (4), 8 per half */
+#pragma unroll
+    for (int i = 0; i < 12; i++) x3[i] = ez[i];
 #pragma unroll
     for (int j = 0; j < 4; j++) {
-      zs[j] += zu[j];
-      ez[3 * j] += zu[j] * e.x;
-      ez[3 * j + 1] += zu[j] * e.y;
-      ez[3 * j + 2] += zu[j] * e.z;
+      const float y[4] = {hf ? x3[4 + j] : x3[j], hf ? x3[8 + j] : gi[j], 0.0f, 0.0f};
+      const bf16x4 b = mp_bf4(y);
+      T[(48 + (hf ? 4 : 0) + j) * MP_TS + li] = b[0];
+      T[(48 + (hf ? 8 : 12) + j) * MP_TS + li] = b[1];
+    }
+    wave_lds_sync();
+    gs = mp_tile_mm<32, 32>(T, T + 64 * MP_TS, gs);
+    gq = mp_tile_mm<16, 32>(T + 32 * MP_TS, T + 64 * MP_TS, gq);
+    ge = mp_tile_mm<4, 12>(T + 60 * MP_TS, T + 48 * MP_TS, ge);
+    mp_update_bwd(dh, v, on, ZU, H, M, wb + MPB_UT(MP_NR - 1), wb + MPB_VT(MP_NR - 1), idg, dhn, dm, T, bu, gu, gw);
+  }
+  float *pp = part + (size_t)p * MP_NPARAM;
+  mp_wsum<32, MP_H>(gs, sh, pp + MP_WSA);
+  mp_bsum(bs, sh, pp + MP_BSA);
+  mp_wsum<16, MP_H>(gq, sh, pp + MP_WB);
+  mp_wsum<4, 12>(ge, sh, pp + MP_WE);
+  mp_wsum<MP_H, MP_H>(gu, sh, pp + MP_U(MP_NR - 1));
+  mp_wsum<MP_H, MP_H>(gw, sh, pp + MP_V(MP_NR - 1));
+  mp_bsum(bu, sh, pp + MP_UB(MP_NR - 1));
+}
+
+/* After round l's messages: the gradients of A_l and B_l, dh = dhn + dP A +
+ * dQ B, and then the update backward of round l - 1 or, after round 0, the
+ * gradients of W0 and b0 (dz0 = dh where z0 > 0) */
+template <bool FIRST>
+__global__ __launch_bounds__(MP_RB, 2) void k_mp_round_bwd(uint32_t N, uint32_t chunk, int l, const float *__restrict__ ideg,
+                                                        const unsigned short *__restrict__ wb,
+                                                        const float *__restrict__ dP, const float *__restrict__ dQ,
+                                                        const float *__restrict__ Hl, const float *__restrict__ ZU,
+                                                        const float *__restrict__ H, const float *__restrict__ M,
+                                                        float *__restrict__ dhn, float *__restrict__ dm,
+                                                        float *__restrict__ part)
+{
+  __shared__ __align__(16) unsigned char lds[2 * MP_BWD_LDS];
+  short *T = reinterpret_cast<short *>(lds) + (threadIdx.x >> 6) * MP_BWD_TILES;
+  float *sh = reinterpret_cast<float *>(lds);
+  const uint32_t li = threadIdx.x & 31u, h4 = (threadIdx.x & 32u) >> 3;
+  const uint32_t p = kf_xcd_block(), n0 = p * chunk, n1 = min(N, n0 + chunk);
+  f32x16 ga = mp_zero(), gb = mp_zero(), gu = mp_zero(), gw = mp_zero();
+  float bu[16];
+#pragma unroll
+  for (int r = 0; r < 16; r++) bu[r] = 0.0f;
+  for (uint32_t row = n0 + 32 * (threadIdx.x >> 6); row < n1; row += 32 * MP_TW) {
+    const uint32_t v = min(row + li, n1 - 1);
+    const bool on = row + li < n1;
+    float x[16], y[16], h[16], dh[16];
+    mp_row_ld(dP, v, x);
+    mp_row_ld(dQ, v, y);
+    mp_row_ld(Hl, v, h);
+    mp_row_ld(dhn, v, dh);
+    wave_lds_sync();
+    f32x16 acc = mp_mm<4, 2 * MP_H>(wb + MPB_ABT(l), 0, x, mp_zero());
+    acc = mp_mm<4, 2 * MP_H>(wb + MPB_ABT(l), MP_H, y, acc);
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+      x[r] = on ? x[r] : 0.0f;
+      y[r] = on ? y[r] : 0.0f;
+    }
+    mp_tile_put<4>(T, x);
+    mp_tile_put<4>(T + 32 * MP_TS, y);
+    mp_tile_put<4>(T + 64 * MP_TS, h);
+    mp_bias(acc, NULL, x);
+#pragma unroll
+    for (int r = 0; r < 16; r++) dh[r] = dh[r] + x[r];
+    wave_lds_sync();
+    ga = mp_tile_mm<32, 32>(T, T + 64 * MP_TS, ga);
+    gb = mp_tile_mm<32, 32>(T + 32 * MP_TS, T + 64 * MP_TS, gb);
+    if (!FIRST) {
+      mp_update_bwd(dh, v, on, ZU, H, M, wb + MPB_UT(l - 1), wb + MPB_VT(l - 1), ideg[v], dhn, dm, T, bu, gu, gw);
+    } else {
+      /* ZU is z0, H the features (16 per vertex) */
+      mp_row_ld(ZU, v, x);
+#pragma unroll
+      for (int r = 0; r < 16; r++) {
+        x[r] = on && x[r] > 0.0f ? dh[r] : 0.0f;
+        bu[r] += x[r];
+      }
+#pragma unroll
+      for (int q = 0; q < 2; q++) {
+        const float4 t = *reinterpret_cast<const float4 *>(H + (size_t)v * MP_NIN + 8 * q + h4);
+        y[4 * q] = t.x; y[4 * q + 1] = t.y; y[4 * q + 2] = t.z; y[4 * q + 3] = t.w;
+      }
+      wave_lds_sync();
+      mp_tile_put<4>(T, x);
+      mp_tile_put<2>(T + 32 * MP_TS, y);
+      wave_lds_sync();
+      gu = mp_tile_mm<32, MP_NIN>(T, T + 32 * MP_TS, gu);
     }
   }
-  const float4 zv4 = ld4(z, v), g4 = *(const float4 *)(gv + 4 * (size_t)v);
-  const float zv[4] = {zv4.x, zv4.y, zv4.z, zv4.w}, g[4] = {g4.x, g4.y, g4.z, g4.w};
-  const float idg = 1.0f / (float)max(deg, 1u);
-  float *o1 = dOP1 + (size_t)v * MP_H, *oq = dOPQ + (size_t)v * MP_H;
-#pragma unroll
-  for (int i = 0; i < 4; i++) {
-    const float gi = g[i] * idg;
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-      o1[4 * i + j] = g[i] * zv[j];
-      o1[16 + 4 * i + j] = gi * zs[j];
-      oq[4 * i + j] = gb[i] * zv[j];
-      oq[16 + 4 * i + j] = 0.0f;
-    }
-    gd[4 * (size_t)v + i] = gi;
+  float *pp = part + (size_t)p * MP_NPARAM;
+  mp_wsum<MP_H, MP_H>(ga, sh, pp + MP_A(l));
+  mp_wsum<MP_H, MP_H>(gb, sh, pp + MP_B(l));
+  if (!FIRST) {
+    mp_wsum<MP_H, MP_H>(gu, sh, pp + MP_U(l - 1));
+    mp_wsum<MP_H, MP_H>(gw, sh, pp + MP_V(l - 1));
+    mp_bsum(bu, sh, pp + MP_UB(l - 1));
+  } else {
+    mp_wsum<MP_H, MP_NIN>(gu, sh, pp + MP_W0);
+    mp_bsum(bu, sh, pp + MP_B0);
   }
-#pragma unroll
-  for (int i = 0; i < 12; i++) Ez[12 * (size_t)v + i] = ez[i];
 }
 
 /* ---- loss ---------------------------------------------------------------------------- */
@@ -892,8 +1077,8 @@ struct kf_mpnn {
   uint32_t *pos[MP_NR];      /* per round: which messages were positive (k_mp_message) */
   uint32_t words;            /* ... words per vertex and lane */
   float *OP1, *OPQ;          /* operator coefficients of the prepared slot */
-  float *dh, *dhn, *dm, *dP, *dQ;
-  float *dOP1, *dOPQ, *gd, *Ez;
+  float *dhn, *dm, *dP, *dQ; /* backward: d h before the messages' part, d m / deg, d P, d Q */
+  float *ideg;               /* 1 / max(degree, 1) */
   float *dstore, *isd;       /* per slot: FP32 [N][16] diagonal blocks, 1 / their RMS */
   double *red, *tred, *lpart;
   float *dl, *ebuf, *ybuf, *gbuf; /* loss: correction, error, A error, gradient (N x 4) */
@@ -960,11 +1145,10 @@ static void mp_loss_grad(kf_mpnn *net, int slot, const double *v, const double *
 {
   kf_ctx *c = net->c;
   hipStream_t st = c->stream;
-  const uint32_t N = net->N, nw = kf_blocks_for(N, 32), P = net->nparts, ch = net->chunk, nb = net->nlblk;
+  const uint32_t N = net->N, P = net->nparts, ch = net->chunk, nb = net->nlblk;
   const size_t n4 = 4 * (size_t)N;
   const uint32_t nb4 = kf_blocks_for(n4, MP_RB);
   const float *nf = NULL;
-  const uint32_t *nu = NULL;
   const int metric = net->metric;
   const float *A = net->mslot[slot];
   if (metric >= 1 && !A) {
@@ -986,42 +1170,20 @@ static void mp_loss_grad(kf_mpnn *net, int slot, const double *v, const double *
     hipLaunchKernelGGL(k_mp_bsr_mvt, dim3(nb), dim3(MP_RB), 0, st, N, c->d.rowptr, c->d.col, net->tpos, A, net->ybuf,
                        net->ebuf);
   hipLaunchKernelGGL(k_mp_scale, dim3(nb4), dim3(MP_RB), 0, st, n4, net->ebuf, net->sc, net->gbuf);
-  /* the operator heads */
-  hipLaunchKernelGGL(k_mp_apply_bwd, dim3(nb), dim3(MP_RB), 0, st, c->d, net->ev, base, net->gbuf, net->dOP1,
-                     net->dOPQ, net->gd, net->Ez);
-  hipLaunchKernelGGL((k_wgrad<MP_H, MP_H, 32, MP_H, false>), dim3(P), dim3(64), 0, st, N, ch, net->dOP1, nf,
-                     net->H[MP_NR], net->part, (uint32_t)MP_WSA, (int)MP_BSA);
-  hipLaunchKernelGGL((k_wgrad<MP_H, MP_H, 16, MP_H, false>), dim3(P), dim3(64), 0, st, N, ch, net->dOPQ, nf,
-                     net->H[MP_NR], net->part, (uint32_t)MP_WB, -1);
-  hipLaunchKernelGGL((k_wgrad<4, 12, 4, 12, false>), dim3(P), dim3(64), 0, st, N, ch, net->gd, nf, net->Ez,
-                     net->part, (uint32_t)MP_WE, -1);
-  hipLaunchKernelGGL((k_dense32<MP_H, MP_H, 0, false>), dim3(nw), dim3(64), 0, st, N, net->dOP1, net->dOPQ, nf,
-                     net->wb + MPB_HT, nf, nf, nu, net->dh);
-  for (int l = MP_NR - 1; l >= 0; l--) {
-    /* dzu = dh [zu > 0]: gradients of U, u and V */
-    hipLaunchKernelGGL((k_wgrad<MP_H, MP_H, MP_H, MP_H, true>), dim3(P), dim3(64), 0, st, N, ch, net->dh, net->ZU[l],
-                       net->H[l], net->part, (uint32_t)MP_U(l), (int)MP_UB(l));
-    hipLaunchKernelGGL((k_wgrad<MP_H, MP_H, MP_H, MP_H, true>), dim3(P), dim3(64), 0, st, N, ch, net->dh, net->ZU[l],
-                       net->M[l], net->part, (uint32_t)MP_V(l), -1);
-    /* dhn = dh + dzu U;  dm = (dzu V) / deg */
-    hipLaunchKernelGGL((k_dense32<MP_H, 0, 3, true>), dim3(nw), dim3(64), 0, st, N, net->dh, nf, net->ZU[l],
-                       net->wb + MPB_UT(l), nf, net->dh, nu, net->dhn);
-    hipLaunchKernelGGL((k_dense32<MP_H, 0, 4, true>), dim3(nw), dim3(64), 0, st, N, net->dh, nf, net->ZU[l],
-                       net->wb + MPB_VT(l), nf, nf, c->d.deg, net->dm);
+  const int L = MP_NR - 1;
+  hipLaunchKernelGGL(k_mp_head_bwd, dim3(P), dim3(MP_RB), 0, st, c->d, ch, net->ev, net->ideg, base, net->gbuf, net->wb,
+                     net->H[MP_NR], net->ZU[L], net->H[L], net->M[L], net->dhn, net->dm, net->part);
+  for (int l = L; l >= 0; l--) {
     hipLaunchKernelGGL(k_mp_message_bwd, dim3(P), dim3(MP_RB), 0, st, c->d, ch, net->ev, net->pos[l], net->words,
                        net->dm, (uint32_t)MP_C(l), (uint32_t)MP_CB(l), net->dP, net->dQ, net->part);
-    hipLaunchKernelGGL((k_wgrad<MP_H, MP_H, MP_H, MP_H, false>), dim3(P), dim3(64), 0, st, N, ch, net->dP, nf,
-                       net->H[l], net->part, (uint32_t)MP_A(l), -1);
-    hipLaunchKernelGGL((k_wgrad<MP_H, MP_H, MP_H, MP_H, false>), dim3(P), dim3(64), 0, st, N, ch, net->dQ, nf,
-                       net->H[l], net->part, (uint32_t)MP_B(l), -1);
-    /* dh = dhn + dP A + dQ B */
-    hipLaunchKernelGGL((k_dense32<MP_H, MP_H, 3, false>), dim3(nw), dim3(64), 0, st, N, net->dP, net->dQ, nf,
-                       net->wb + MPB_ABT(l), nf, net->dhn, nu, net->dh);
+    if (l > 0)
+      hipLaunchKernelGGL(k_mp_round_bwd<false>, dim3(P), dim3(MP_RB), 0, st, N, ch, l, net->ideg, net->wb, net->dP,
+                         net->dQ, net->H[l], net->ZU[l - 1], net->H[l - 1], net->M[l - 1], net->dhn, net->dm, net->part);
+    else
+      hipLaunchKernelGGL(k_mp_round_bwd<true>, dim3(P), dim3(MP_RB), 0, st, N, ch, l, net->ideg, net->wb, net->dP,
+                         net->dQ, net->H[0], net->Z0, net->X, nf, net->dhn, (float *)NULL, net->part);
   }
-  hipLaunchKernelGGL((k_wgrad<MP_H, MP_NIN, MP_H, MP_NIN, true>), dim3(P), dim3(64), 0, st, N, ch, net->dh, net->Z0,
-                     net->X, net->part, (uint32_t)MP_W0, (int)MP_B0);
-  hipLaunchKernelGGL(k_mp_grad_reduce, dim3(kf_blocks_for(MP_NPARAM, MP_RB)), dim3(MP_RB), 0, st, net->part, P,
-                     net->grad);
+  hipLaunchKernelGGL(k_mp_grad_reduce, dim3(kf_blocks_for(MP_NPARAM, 64)), dim3(1024), 0, st, net->part, P, net->grad);
   KF_LAUNCH_CHECK();
 }
 
@@ -1082,8 +1244,7 @@ extern "C" kf_mpnn *kf_mpnn_create(GEOMETRY *g, const float *theta_host, int nsl
   net->N = N;
   net->nslot = (uint32_t)nslot;
   uint32_t ch = (N + MP_PARTS - 1) / MP_PARTS;
-  ch = ((ch + 7u) / 8u) * 8u;
-  if (ch < 8) ch = 8;
+  ch = ((ch + 31u) / 32u) * 32u;   /* whole tiles of 32 vertices */
   net->chunk = ch;
   net->nparts = (N + ch - 1) / ch;
   net->nlblk = kf_blocks_for(N, MP_RB);
@@ -1115,15 +1276,11 @@ extern "C" kf_mpnn *kf_mpnn_create(GEOMETRY *g, const float *theta_host, int nsl
   }
   net->OP1 = mp_alloc<float>(NH);
   net->OPQ = mp_alloc<float>(NH);
-  net->dh = mp_alloc<float>(NH);
   net->dhn = mp_alloc<float>(NH);
   net->dm = mp_alloc<float>(NH);
   net->dP = mp_alloc<float>(NH);
   net->dQ = mp_alloc<float>(NH);
-  net->dOP1 = mp_alloc<float>(NH);
-  net->dOPQ = mp_alloc<float>(NH);
-  net->gd = mp_alloc<float>(4 * (size_t)N);
-  net->Ez = mp_alloc<float>(12 * (size_t)N);
+  net->ideg = mp_alloc<float>(N);
   net->dstore = mp_alloc<float>((size_t)nslot * 16 * N);
   net->isd = mp_alloc<float>(nslot);
   net->red = mp_alloc<double>(KF_NRED);
@@ -1168,7 +1325,8 @@ extern "C" kf_mpnn *kf_mpnn_create(GEOMETRY *g, const float *theta_host, int nsl
   float *ones = (float *)malloc(sizeof(float) * nslot);
   for (int i = 0; i < nslot; i++) ones[i] = 1.0f;
   KF_CHECK(hipMemcpyAsync(net->isd, ones, sizeof(float) * nslot, hipMemcpyHostToDevice, c->stream));
-  hipLaunchKernelGGL(k_mp_edge_vectors, dim3(kf_blocks_for(N, MP_RB)), dim3(MP_RB), 0, c->stream, c->d, net->ev);
+  hipLaunchKernelGGL(k_mp_edge_vectors, dim3(kf_blocks_for(N, MP_RB)), dim3(MP_RB), 0, c->stream, c->d, net->ev,
+                     net->ideg);
   KF_LAUNCH_CHECK();
   KF_CHECK(hipStreamSynchronize(c->stream));
   free(ones);
@@ -1198,8 +1356,8 @@ extern "C" void kf_mpnn_destroy(kf_mpnn *net)
   if (!net) return;
   KF_CHECK(hipStreamSynchronize(net->c->stream));
   void *bufs[] = {net->theta, net->am,   net->av,   net->grad,  net->part, net->sc,   net->gnorm, net->losses,
-                  net->wb,    net->ev,   net->X,    net->Z0,    net->OP1,  net->OPQ,  net->dh,    net->dhn,
-                  net->dm,    net->dP,   net->dQ,   net->dOP1,  net->dOPQ, net->gd,   net->Ez,    net->dstore,
+                  net->wb,    net->ev,   net->X,    net->Z0,    net->OP1,  net->OPQ,  net->ideg,  net->dhn,
+                  net->dm,    net->dP,   net->dQ,   net->dstore,
                   net->isd,   net->red,  net->tred, net->lpart, net->dl,   net->ebuf, net->ybuf,  net->gbuf,
                   net->tpos};
   for (void *p : bufs)
