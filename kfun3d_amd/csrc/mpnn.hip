@@ -357,13 +357,16 @@ __global__ __launch_bounds__(MP_RB) void k_mp_sumsq(size_t n, const T *__restric
   if (threadIdx.x == 0) part[blockIdx.x] = s;
 }
 
-/* One lane sums the KF_NRED partials in index order into *out = 1 / RMS
- * over `count` values (1 when zero or not finite). */
-__global__ void k_mp_finish(const double *__restrict__ part, double count, float *__restrict__ out)
+/* *out = 1 / RMS over `count` values from the KF_NRED partials (1 when zero or
+ * not finite) */
+__global__ __launch_bounds__(MP_RB) void k_mp_finish(const double *__restrict__ part, double count,
+                                                     float *__restrict__ out)
 {
-  if (threadIdx.x != 0) return;
+  __shared__ double sh[MP_RB];
   double a = 0.0;
-  for (int i = 0; i < KF_NRED; i++) a += part[i];
+  for (int i = threadIdx.x; i < KF_NRED; i += MP_RB) a += part[i];
+  a = mp_block_sum(a, sh);
+  if (threadIdx.x != 0) return;
   double s = sqrt(a / count);
   if (!(s > 0.0) || !isfinite(s)) s = 1.0;
   *out = (float)(1.0 / s);
@@ -578,32 +581,29 @@ __device__ __forceinline__ float4 ld4(const double *z, uint32_t v)
  * with zs_v = sum_u z_u and Ez_v[j][k] = sum_u z_u[j] e_vu[k] (the edge
  * blocks T_vu = P_v + b + Q_u + We e_vu factored), one thread per vertex.
  * OP1 = [S | P + b] (N x 32), OPQ = [Q | 0] (N x 32).  Output: FP64 out
- * (stored, or added when add) or, when outf is given, FP32 outf. */
+ * (stored, or added when add) or, when err is given, the FP32 error
+ * err = z + delta - target (formed in FP64; target NULL: z + delta).  Two
+ * neighbours' rows are in flight; the sums keep the edge order. */
 __global__ __launch_bounds__(MP_RB) void k_mp_apply(kf_dv d, const float4 *__restrict__ ev,
                                                     const float *__restrict__ OP1, const float *__restrict__ OPQ,
                                                     const float *__restrict__ theta, const double *__restrict__ z,
-                                                    double *__restrict__ out, int add, float *__restrict__ outf)
+                                                    double *__restrict__ out, int add,
+                                                    const double *__restrict__ target, float *__restrict__ err)
 {
   __shared__ float we[48];
   if (threadIdx.x < 48) we[threadIdx.x] = theta[MP_WE + threadIdx.x];
   __syncthreads();
-  const uint32_t v = blockIdx.x * MP_RB + threadIdx.x;
+  const uint32_t v = kf_xcd_block() * MP_RB + threadIdx.x;
   if (v >= d.N) return;
   const uint32_t deg = d.deg[v];
   size_t idx = (size_t)d.sell_ptr[v >> 6] * 64u + (v & 63u);
   float qz[4] = {0.0f, 0.0f, 0.0f, 0.0f}, zs[4] = {0.0f, 0.0f, 0.0f, 0.0f}, ez[12];
 #pragma unroll
   for (int i = 0; i < 12; i++) ez[i] = 0.0f;
-  for (uint32_t k = 0; k < deg; k++, idx += 64) {
-    const uint32_t u = d.sell_nbr[idx];
-    const float4 e = ev[idx], zu4 = ld4(z, u);
+  auto sum = [&](const float4 &e, const float4 &zu4, const float4 q[4]) {
     const float zu[4] = {zu4.x, zu4.y, zu4.z, zu4.w};
-    const float4 *q = (const float4 *)(OPQ + (size_t)u * MP_H);
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-      const float4 qi = q[i];
-      qz[i] += qi.x * zu[0] + qi.y * zu[1] + qi.z * zu[2] + qi.w * zu[3];
-    }
+    for (int i = 0; i < 4; i++) qz[i] += q[i].x * zu[0] + q[i].y * zu[1] + q[i].z * zu[2] + q[i].w * zu[3];
 #pragma unroll
     for (int j = 0; j < 4; j++) {
       zs[j] += zu[j];
@@ -611,6 +611,23 @@ __global__ __launch_bounds__(MP_RB) void k_mp_apply(kf_dv d, const float4 *__res
       ez[3 * j + 1] += zu[j] * e.y;
       ez[3 * j + 2] += zu[j] * e.z;
     }
+  };
+  uint32_t k = 0;
+  for (; k + 1 < deg; k += 2, idx += 128) {
+    const uint32_t ua = d.sell_nbr[idx], ub = d.sell_nbr[idx + 64];
+    const float4 ea = ev[idx], eb = ev[idx + 64];
+    const float4 za = ld4(z, ua), zb = ld4(z, ub);
+    const float4 *pa = (const float4 *)(OPQ + (size_t)ua * MP_H), *pb = (const float4 *)(OPQ + (size_t)ub * MP_H);
+    const float4 qa[4] = {pa[0], pa[1], pa[2], pa[3]}, qb[4] = {pb[0], pb[1], pb[2], pb[3]};
+    sum(ea, za, qa);
+    sum(eb, zb, qb);
+  }
+  if (k < deg) {
+    const uint32_t ua = d.sell_nbr[idx];
+    const float4 ea = ev[idx], za = ld4(z, ua);
+    const float4 *pa = (const float4 *)(OPQ + (size_t)ua * MP_H);
+    const float4 qa[4] = {pa[0], pa[1], pa[2], pa[3]};
+    sum(ea, za, qa);
   }
   const float4 zv4 = ld4(z, v);
   const float zv[4] = {zv4.x, zv4.y, zv4.z, zv4.w};
@@ -627,8 +644,9 @@ __global__ __launch_bounds__(MP_RB) void k_mp_apply(kf_dv d, const float4 *__res
            we[3 * (4 * i + j) + 2] * ez[3 * j + 2];
     }
     const float dl = sv + t * idg;
-    if (outf) outf[4 * (size_t)v + i] = dl;
-    else out[4 * (size_t)v + i] = add ? out[4 * (size_t)v + i] + (double)dl : (double)dl;
+    const size_t o = 4 * (size_t)v + i;
+    if (err) err[o] = (float)(z[o] + (double)dl - (target ? target[o] : 0.0));
+    else out[o] = add ? out[o] + (double)dl : (double)dl;
   }
 }
 
@@ -888,98 +906,140 @@ __global__ __launch_bounds__(MP_RB, 2) void k_mp_round_bwd(uint32_t N, uint32_t 
 
 /* ---- loss ---------------------------------------------------------------------------- */
 
-/* e = base + delta - target (target may be NULL: e = base + delta), FP32
- * computed in FP64 */
-__global__ __launch_bounds__(MP_RB) void k_mp_err(size_t n, const float *__restrict__ dl,
-                                                  const double *__restrict__ base, const double *__restrict__ target,
-                                                  float *__restrict__ e)
+/* The residual y the loss is formed of and, per workgroup, its sum of squares
+ * and the reference's: METRIC 0 y = e against |target|, 1 y = A e against |v|,
+ * 2 y = A e - v against |v|.  A quad of lanes per block row, lane c forming
+ * component c (as spmv.hip): the quad reads a whole 64-byte block at once,
+ * where one lane per row read 64 rows' blocks side by side (331,776 vertices:
+ * 91 us against 120 us for the product alone and 20 us for the rest). */
+template <int METRIC>
+__global__ __launch_bounds__(MP_RB) void k_mp_resid(uint32_t N, const uint32_t *__restrict__ rowptr,
+                                                    const uint32_t *__restrict__ col, const float *__restrict__ A,
+                                                    const float *__restrict__ e, const double *__restrict__ ref,
+                                                    float *__restrict__ y, double2 *__restrict__ lpart)
 {
-  const size_t k = (size_t)blockIdx.x * MP_RB + threadIdx.x;
-  if (k < n) e[k] = (float)(base[k] + (double)dl[k] - (target ? target[k] : 0.0));
-}
-
-/* y -= v (FP32 y, FP64 v) */
-__global__ __launch_bounds__(MP_RB) void k_mp_sub(size_t n, const double *__restrict__ v, float *__restrict__ y)
-{
-  const size_t k = (size_t)blockIdx.x * MP_RB + threadIdx.x;
-  if (k < n) y[k] = (float)((double)y[k] - v[k]);
-}
-
-/* y_i = sum over row i's blocks A(i, j) x_j (one thread per block row) */
-__global__ __launch_bounds__(MP_RB) void k_mp_bsr_mv(uint32_t N, const uint32_t *__restrict__ rowptr,
-                                                     const uint32_t *__restrict__ col, const float *__restrict__ A,
-                                                     const float *__restrict__ x, float *__restrict__ y)
-{
-  const uint32_t i = blockIdx.x * MP_RB + threadIdx.x;
-  if (i >= N) return;
-  float a0 = 0.0f, a1 = 0.0f, a2 = 0.0f, a3 = 0.0f;
-  for (uint32_t k = rowptr[i]; k < rowptr[i + 1]; k++) {
-    const float4 xv = *(const float4 *)(x + 4 * (size_t)col[k]);
-    const float *b = A + 16 * (size_t)k;
-    a0 += b[0] * xv.x + b[1] * xv.y + b[2] * xv.z + b[3] * xv.w;
-    a1 += b[4] * xv.x + b[5] * xv.y + b[6] * xv.z + b[7] * xv.w;
-    a2 += b[8] * xv.x + b[9] * xv.y + b[10] * xv.z + b[11] * xv.w;
-    a3 += b[12] * xv.x + b[13] * xv.y + b[14] * xv.z + b[15] * xv.w;
-  }
-  *(float4 *)(y + 4 * (size_t)i) = make_float4(a0, a1, a2, a3);
-}
-
-/* g_j = sum over row j's positions k (column i = col[k]) of A(i, j)^T y_i,
- * A(i, j) at tpos[k] (the pattern is structurally symmetric) */
-__global__ __launch_bounds__(MP_RB) void k_mp_bsr_mvt(uint32_t N, const uint32_t *__restrict__ rowptr,
-                                                      const uint32_t *__restrict__ col,
-                                                      const uint32_t *__restrict__ tpos, const float *__restrict__ A,
-                                                      const float *__restrict__ y, float *__restrict__ g)
-{
-  const uint32_t j = blockIdx.x * MP_RB + threadIdx.x;
-  if (j >= N) return;
-  float a0 = 0.0f, a1 = 0.0f, a2 = 0.0f, a3 = 0.0f;
-  for (uint32_t k = rowptr[j]; k < rowptr[j + 1]; k++) {
-    const float4 yv = *(const float4 *)(y + 4 * (size_t)col[k]);
-    const float *b = A + 16 * (size_t)tpos[k];
-    a0 += b[0] * yv.x + b[4] * yv.y + b[8] * yv.z + b[12] * yv.w;
-    a1 += b[1] * yv.x + b[5] * yv.y + b[9] * yv.z + b[13] * yv.w;
-    a2 += b[2] * yv.x + b[6] * yv.y + b[10] * yv.z + b[14] * yv.w;
-    a3 += b[3] * yv.x + b[7] * yv.y + b[11] * yv.z + b[15] * yv.w;
-  }
-  *(float4 *)(g + 4 * (size_t)j) = make_float4(a0, a1, a2, a3);
-}
-
-__global__ __launch_bounds__(MP_RB) void k_mp_sq4(uint32_t N, const float *__restrict__ x, double *__restrict__ lpart)
-{
-  __shared__ double sh[MP_RB];
-  const uint32_t n = blockIdx.x * MP_RB + threadIdx.x;
-  double acc = 0.0;
-  if (n < N) {
+  __shared__ double sh[2 * MP_RB / 64];
+  const uint32_t i = kf_xcd_block() * (MP_RB / 4) + (threadIdx.x >> 2), c = threadIdx.x & 3u;
+  double s = 0.0, t = 0.0;
+  if (i < N) {
+    const size_t o = 4 * (size_t)i + c;
+    float a;
+    if (METRIC == 0) {
+      a = e[o];
+    } else {
+      a = 0.0f;
+      const uint32_t j0 = rowptr[i], j1 = rowptr[i + 1];
+      for (uint32_t j = j0; j < j1; j += 4) {
+        float4 b[4], x[4];
 #pragma unroll
-    for (int o = 0; o < 4; o++) {
-      const double v = (double)x[4 * (size_t)n + o];
-      acc += v * v;
+        for (int q = 0; q < 4; q++) {
+          const uint32_t k = min(j + q, j1 - 1);
+          b[q] = *(const float4 *)(A + 16 * (size_t)k + 4 * c);
+          x[q] = *(const float4 *)(e + 4 * (size_t)col[k]);
+        }
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+          const float r = a + (b[q].x * x[q].x + b[q].y * x[q].y + b[q].z * x[q].z + b[q].w * x[q].w);
+          a = j + q < j1 ? r : a;
+        }
+      }
+      if (METRIC == 2) a = (float)((double)a - ref[o]);
+      y[o] = a;
+    }
+    s = (double)a * (double)a;
+    t = ref[o] * ref[o];
+  }
+#pragma unroll
+  for (int m = 32; m > 0; m >>= 1) {
+    s += __shfl_xor(s, m, 64);
+    t += __shfl_xor(t, m, 64);
+  }
+  if ((threadIdx.x & 63u) == 0) {
+    sh[2 * (threadIdx.x >> 6)] = s;
+    sh[2 * (threadIdx.x >> 6) + 1] = t;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < MP_RB / 64; w++) {
+      s += sh[2 * w];
+      t += sh[2 * w + 1];
+    }
+    lpart[kf_xcd_block()] = make_double2(s, t);
+  }
+}
+
+/* loss = sum of the residual's partials / sum of the reference's into out[0];
+ * the gradient scale 2 / the reference sum into sc[3] (one workgroup, each
+ * thread every 1024th partial, then a fixed tree; one lane walking them took
+ * 99 us) */
+__global__ __launch_bounds__(1024) void k_mp_loss_finish(const double2 *__restrict__ lpart, uint32_t nb,
+                                                         float *__restrict__ out, float *__restrict__ sc)
+{
+  __shared__ double sa[1024], st[1024];
+  const uint32_t i = threadIdx.x;
+  double a = 0.0, t = 0.0;
+  for (uint32_t b = i; b < nb; b += 1024) {
+    a += lpart[b].x;
+    t += lpart[b].y;
+  }
+  sa[i] = a;
+  st[i] = t;
+  __syncthreads();
+  for (uint32_t s = 512; s > 0; s >>= 1) {
+    if (i < s) {
+      sa[i] += sa[i + s];
+      st[i] += st[i + s];
+    }
+    __syncthreads();
+  }
+  if (i == 0) {
+    a = sa[0];
+    t = st[0];
+    out[0] = t > 0.0 ? (float)(a / t) : 0.0f;
+    sc[3] = t > 0.0 ? (float)(2.0 / t) : 0.0f;
+  }
+}
+
+/* g = sc[3] A^T y (TRANS; y for METRIC 0): g_j sums A(i, j)^T y_i over row
+ * j's positions k (column i = col[k], A(i, j) at tpos[k]; the pattern is
+ * structurally symmetric).  A quad of lanes per row, lane c reading column c
+ * of the blocks: four 16-byte runs a block (331,776 vertices: 107 us against
+ * 166 us with a lane per row, and a pass for the scale). */
+template <bool TRANS>
+__global__ __launch_bounds__(MP_RB) void k_mp_loss_grad(uint32_t N, const uint32_t *__restrict__ rowptr,
+                                                        const uint32_t *__restrict__ col,
+                                                        const uint32_t *__restrict__ tpos, const float *__restrict__ A,
+                                                        const float *__restrict__ y, const float *__restrict__ sc,
+                                                        float *__restrict__ g)
+{
+  const uint32_t i = kf_xcd_block() * (MP_RB / 4) + (threadIdx.x >> 2), c = threadIdx.x & 3u;
+  if (i >= N) return;
+  const size_t o = 4 * (size_t)i + c;
+  float a;
+  if (!TRANS) {
+    a = y[o];
+  } else {
+    a = 0.0f;
+    const uint32_t j0 = rowptr[i], j1 = rowptr[i + 1];
+    for (uint32_t j = j0; j < j1; j += 4) {
+      float4 x[4];
+      float b[4][4];
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        const uint32_t k = min(j + q, j1 - 1);
+        const float *p = A + 16 * (size_t)tpos[k] + c;
+#pragma unroll
+        for (int r = 0; r < 4; r++) b[q][r] = p[4 * r];
+        x[q] = *(const float4 *)(y + 4 * (size_t)col[k]);
+      }
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        const float r = a + (b[q][0] * x[q].x + b[q][1] * x[q].y + b[q][2] * x[q].z + b[q][3] * x[q].w);
+        a = j + q < j1 ? r : a;
+      }
     }
   }
-  const double s = mp_block_sum(acc, sh);
-  if (threadIdx.x == 0) lpart[blockIdx.x] = s;
-}
-
-/* loss = (block partials summed in order) / (reference partials summed in
- * order) into out[0]; the gradient scale 2 / that reference sum into sc[3] */
-__global__ void k_mp_loss_finish(const double *__restrict__ lpart, uint32_t nb, const double *__restrict__ tpart,
-                                 float *__restrict__ out, float *__restrict__ sc)
-{
-  if (threadIdx.x != 0) return;
-  double a = 0.0, t = 0.0;
-  for (uint32_t i = 0; i < nb; i++) a += lpart[i];
-  for (int i = 0; i < KF_NRED; i++) t += tpart[i];
-  out[0] = t > 0.0 ? (float)(a / t) : 0.0f;
-  sc[3] = t > 0.0 ? (float)(2.0 / t) : 0.0f;
-}
-
-/* g = f x, f = sc[3] */
-__global__ __launch_bounds__(MP_RB) void k_mp_scale(size_t n, const float *__restrict__ x,
-                                                    const float *__restrict__ sc, float *__restrict__ g)
-{
-  const size_t k = (size_t)blockIdx.x * MP_RB + threadIdx.x;
-  if (k < n) g[k] = x[k] * sc[3];
+  g[o] = a * sc[3];
 }
 
 /* A (FP64 or FP32 BSR values) as FP32 */
@@ -1068,7 +1128,7 @@ __global__ void k_mp_pack(const float *__restrict__ theta, unsigned short *__res
 
 struct kf_mpnn {
   kf_ctx *c;
-  uint32_t N, nparts, chunk, nslot, nlblk;
+  uint32_t N, nparts, chunk, nslot, nvblk, nlblk;   /* blocks of vertices, of block rows by quads */
   float *theta, *am, *av, *grad, *part, *sc, *gnorm, *losses;
   uint32_t nloss_cap, nloss;
   unsigned short *wb;
@@ -1080,8 +1140,9 @@ struct kf_mpnn {
   float *dhn, *dm, *dP, *dQ; /* backward: d h before the messages' part, d m / deg, d P, d Q */
   float *ideg;               /* 1 / max(degree, 1) */
   float *dstore, *isd;       /* per slot: FP32 [N][16] diagonal blocks, 1 / their RMS */
-  double *red, *tred, *lpart;
-  float *dl, *ebuf, *ybuf, *gbuf; /* loss: correction, error, A error, gradient (N x 4) */
+  double *red;
+  double2 *lpart;
+  float *ebuf, *ybuf, *gbuf; /* loss: error, A error, gradient (N x 4) */
   float **mslot;             /* per slot: the assembled Jacobian (FP32 BSR) or NULL */
   uint32_t *tpos;            /* BSR position of the transposed block */
   int t;                     /* Adam steps so far */
@@ -1146,8 +1207,6 @@ static void mp_loss_grad(kf_mpnn *net, int slot, const double *v, const double *
   kf_ctx *c = net->c;
   hipStream_t st = c->stream;
   const uint32_t N = net->N, P = net->nparts, ch = net->chunk, nb = net->nlblk;
-  const size_t n4 = 4 * (size_t)N;
-  const uint32_t nb4 = kf_blocks_for(n4, MP_RB);
   const float *nf = NULL;
   const int metric = net->metric;
   const float *A = net->mslot[slot];
@@ -1156,20 +1215,22 @@ static void mp_loss_grad(kf_mpnn *net, int slot, const double *v, const double *
     abort();
   }
   mp_context(net, slot);
-  hipLaunchKernelGGL(k_mp_apply, dim3(nb), dim3(MP_RB), 0, st, c->d, net->ev, net->OP1, net->OPQ, net->theta, base,
-                     (double *)NULL, 0, net->dl);
-  hipLaunchKernelGGL(k_mp_err, dim3(nb4), dim3(MP_RB), 0, st, n4, net->dl, base, metric == 2 ? NULL : target,
-                     net->ebuf);
-  hipLaunchKernelGGL(k_mp_sumsq<double>, dim3(KF_NRED), dim3(MP_RB), 0, st, n4, metric ? v : target, net->tred);
-  if (metric >= 1)
-    hipLaunchKernelGGL(k_mp_bsr_mv, dim3(nb), dim3(MP_RB), 0, st, N, c->d.rowptr, c->d.col, A, net->ebuf, net->ybuf);
-  if (metric == 2) hipLaunchKernelGGL(k_mp_sub, dim3(nb4), dim3(MP_RB), 0, st, n4, v, net->ybuf);
-  hipLaunchKernelGGL(k_mp_sq4, dim3(nb), dim3(MP_RB), 0, st, N, metric ? net->ybuf : net->ebuf, net->lpart);
-  hipLaunchKernelGGL(k_mp_loss_finish, dim3(1), dim3(64), 0, st, net->lpart, nb, net->tred, loss_dev, net->sc);
-  if (metric >= 1)
-    hipLaunchKernelGGL(k_mp_bsr_mvt, dim3(nb), dim3(MP_RB), 0, st, N, c->d.rowptr, c->d.col, net->tpos, A, net->ybuf,
-                       net->ebuf);
-  hipLaunchKernelGGL(k_mp_scale, dim3(nb4), dim3(MP_RB), 0, st, n4, net->ebuf, net->sc, net->gbuf);
+  hipLaunchKernelGGL(k_mp_apply, dim3(net->nvblk), dim3(MP_RB), 0, st, c->d, net->ev, net->OP1, net->OPQ, net->theta,
+                     base, (double *)NULL, 0, metric == 2 ? NULL : target, net->ebuf);
+#define MP_RESID(METRIC, REF)                                                                                      \
+  hipLaunchKernelGGL(k_mp_resid<METRIC>, dim3(nb), dim3(MP_RB), 0, st, N, c->d.rowptr, c->d.col, A, net->ebuf, REF, \
+                     net->ybuf, net->lpart)
+  if (metric == 0) MP_RESID(0, target);
+  else if (metric == 1) MP_RESID(1, v);
+  else MP_RESID(2, v);
+#undef MP_RESID
+  hipLaunchKernelGGL(k_mp_loss_finish, dim3(1), dim3(1024), 0, st, net->lpart, nb, loss_dev, net->sc);
+  if (metric == 0)
+    hipLaunchKernelGGL(k_mp_loss_grad<false>, dim3(nb), dim3(MP_RB), 0, st, N, c->d.rowptr, c->d.col, net->tpos, A,
+                       net->ebuf, net->sc, net->gbuf);
+  else
+    hipLaunchKernelGGL(k_mp_loss_grad<true>, dim3(nb), dim3(MP_RB), 0, st, N, c->d.rowptr, c->d.col, net->tpos, A,
+                       net->ybuf, net->sc, net->gbuf);
   const int L = MP_NR - 1;
   hipLaunchKernelGGL(k_mp_head_bwd, dim3(P), dim3(MP_RB), 0, st, c->d, ch, net->ev, net->ideg, base, net->gbuf, net->wb,
                      net->H[MP_NR], net->ZU[L], net->H[L], net->M[L], net->dhn, net->dm, net->part);
@@ -1247,7 +1308,8 @@ extern "C" kf_mpnn *kf_mpnn_create(GEOMETRY *g, const float *theta_host, int nsl
   ch = ((ch + 31u) / 32u) * 32u;   /* whole tiles of 32 vertices */
   net->chunk = ch;
   net->nparts = (N + ch - 1) / ch;
-  net->nlblk = kf_blocks_for(N, MP_RB);
+  net->nvblk = kf_blocks_for(N, MP_RB);
+  net->nlblk = kf_blocks_for(N, MP_RB / 4);
   net->theta = mp_alloc<float>(MP_NPARAM);
   net->am = mp_alloc<float>(MP_NPARAM);
   net->av = mp_alloc<float>(MP_NPARAM);
@@ -1284,9 +1346,7 @@ extern "C" kf_mpnn *kf_mpnn_create(GEOMETRY *g, const float *theta_host, int nsl
   net->dstore = mp_alloc<float>((size_t)nslot * 16 * N);
   net->isd = mp_alloc<float>(nslot);
   net->red = mp_alloc<double>(KF_NRED);
-  net->tred = mp_alloc<double>(KF_NRED);
-  net->lpart = mp_alloc<double>(net->nlblk);
-  net->dl = mp_alloc<float>(4 * (size_t)N);
+  net->lpart = mp_alloc<double2>(net->nlblk);
   net->ebuf = mp_alloc<float>(4 * (size_t)N);
   net->ybuf = mp_alloc<float>(4 * (size_t)N);
   net->gbuf = mp_alloc<float>(4 * (size_t)N);
@@ -1358,7 +1418,7 @@ extern "C" void kf_mpnn_destroy(kf_mpnn *net)
   void *bufs[] = {net->theta, net->am,   net->av,   net->grad,  net->part, net->sc,   net->gnorm, net->losses,
                   net->wb,    net->ev,   net->X,    net->Z0,    net->OP1,  net->OPQ,  net->ideg,  net->dhn,
                   net->dm,    net->dP,   net->dQ,   net->dstore,
-                  net->isd,   net->red,  net->tred, net->lpart, net->dl,   net->ebuf, net->ybuf,  net->gbuf,
+                  net->isd,   net->red,  net->lpart, net->ebuf, net->ybuf,  net->gbuf,
                   net->tpos};
   for (void *p : bufs)
     if (p) KF_CHECK(hipFree(p));
@@ -1391,7 +1451,7 @@ extern "C" void kf_mpnn_take_diag(kf_mpnn *net, int slot)
     hipLaunchKernelGGL(k_mp_take_diag<float>, dim3(nb), dim3(MP_RB), 0, st, N, c->d.diag, (const float *)c->a32, D);
   hipLaunchKernelGGL(k_mp_sumsq<float>, dim3(KF_NRED), dim3(MP_RB), 0, st, 16 * (size_t)N, (const float *)D,
                      net->red);
-  hipLaunchKernelGGL(k_mp_finish, dim3(1), dim3(64), 0, st, net->red, 16.0 * N, net->isd + slot);
+  hipLaunchKernelGGL(k_mp_finish, dim3(1), dim3(MP_RB), 0, st, net->red, 16.0 * N, net->isd + slot);
   KF_LAUNCH_CHECK();
   if (net->prepared == slot) net->prepared = -1;
 }
@@ -1434,7 +1494,7 @@ extern "C" void kf_mpnn_set_diag(kf_mpnn *net, int slot, const double *D_host)
   float *D = net->dstore + (size_t)slot * n;
   KF_CHECK(hipMemcpyAsync(D, tmp, sizeof(float) * n, hipMemcpyHostToDevice, c->stream));
   hipLaunchKernelGGL(k_mp_sumsq<float>, dim3(KF_NRED), dim3(MP_RB), 0, c->stream, n, (const float *)D, net->red);
-  hipLaunchKernelGGL(k_mp_finish, dim3(1), dim3(64), 0, c->stream, net->red, (double)n, net->isd + slot);
+  hipLaunchKernelGGL(k_mp_finish, dim3(1), dim3(MP_RB), 0, c->stream, net->red, (double)n, net->isd + slot);
   KF_LAUNCH_CHECK();
   KF_CHECK(hipStreamSynchronize(c->stream));
   free(tmp);
@@ -1455,8 +1515,8 @@ extern "C" void kf_mpnn_forward(kf_mpnn *net, int slot, const double *z, double 
 {
   mp_check_slot(net, slot);
   if (net->prepared != slot) mp_context(net, slot);
-  hipLaunchKernelGGL(k_mp_apply, dim3(net->nlblk), dim3(MP_RB), 0, net->c->stream, net->c->d, net->ev, net->OP1,
-                     net->OPQ, net->theta, z, out, add, (float *)NULL);
+  hipLaunchKernelGGL(k_mp_apply, dim3(net->nvblk), dim3(MP_RB), 0, net->c->stream, net->c->d, net->ev, net->OP1,
+                     net->OPQ, net->theta, z, out, add, (const double *)NULL, (float *)NULL);
   KF_LAUNCH_CHECK();
 }
 
