@@ -57,6 +57,54 @@ __device__ __forceinline__ T blk_mul(const T *A, const T *B, uint32_t r, uint32_
   return s;
 }
 
+/* value of lane I of this lane's quad: a quad holds one row of a 4x4 block,
+ * so these are the row's four entries */
+template <int I>
+__device__ __forceinline__ float quad_bcast(float v)
+{
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), I * 0x55, 0xf, 0xf, true));
+}
+
+template <int I>
+__device__ __forceinline__ double quad_bcast(double v)
+{
+  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), I * 0x55, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), I * 0x55, 0xf, 0xf, true);
+  return __hiloint2double(hi, lo);
+}
+
+/* blk_mul with the left block in registers (one entry per lane) and column c
+ * of the right block in b: the same sum in the same order */
+template <typename T>
+__device__ __forceinline__ T row_mul(T a, const T b[4])
+{
+  T s = T(0);
+  s += quad_bcast<0>(a) * b[0];
+  s += quad_bcast<1>(a) * b[1];
+  s += quad_bcast<2>(a) * b[2];
+  s += quad_bcast<3>(a) * b[3];
+  return s;
+}
+
+/* column c of the 4x4 block at p */
+template <typename T>
+__device__ __forceinline__ void blk_col(const T *p, uint32_t c, T b[4])
+{
+#pragma unroll
+  for (int k = 0; k < 4; k++) b[k] = p[4 * k + c];
+}
+
+__device__ __forceinline__ float lane_get(float v, int l)
+{
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
+}
+
+__device__ __forceinline__ double lane_get(double v, int l)
+{
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), l),
+                          __builtin_amdgcn_readlane(__double2loint(v), l));
+}
+
 /* EXACT: the reference's one-thread sweep bit for bit.  Each block it forms
  * ends with the product of the last common pair of its merge (matrix/ilu.cpp:
  * 71-86): subtracted, then added back, which rounds.  For a lower block (i,k)
@@ -188,242 +236,412 @@ __global__ __launch_bounds__(64) void k_ilu(kf_dv d, const uint32_t *__restrict_
  * maxrow blocks per row, maxlow lower blocks per row, maxmatch update pairs
  * per row. */
 struct ilu_layout {
-  uint32_t scol, sa, sa0, sldg, smoff, sjm, slo, stage, bytes;
+  uint32_t sa, sa0, ssrc, smoff, slo, stage, bytes;
   __host__ __device__ ilu_layout(uint32_t maxrow, uint32_t maxlow, uint32_t maxmatch, uint32_t tsize, bool exact)
   {
     uint32_t o = 0;
     auto take = [&o](uint32_t n) { const uint32_t r = o; o += (n + 15u) & ~15u; return r; };
-    scol = take(4 * maxrow);
     sa = take(16 * tsize * maxrow);
     sa0 = exact ? take(16 * tsize * maxrow) : 0;
-    sldg = take(4 * maxlow);
+    ssrc = take(4 * ((exact ? 2 : 1) * maxlow + maxmatch));
     smoff = take(4 * (maxlow + 1));
-    sjm = take(4 * maxmatch);
-    slo = take(2 * maxmatch);
-    stage = take(16 * tsize * ((exact ? 3 : 1) * maxlow + maxmatch));
+    slo = take(2 * (maxmatch + 8));   /* 8 spare pairs, see the elimination */
+    stage = take(16 * tsize * ((exact ? 3 : 1) * maxlow + maxmatch + 8));
     bytes = o;
   }
 };
 
 #define ILU_Q 4    /* values per lane per load round before the wait */
 #define ILU_QB 12  /* values per lane per staging round after the wait */
+#define ILU_GMAX 8 /* wavefronts per workgroup at most */
+#define ILU_RING 4 /* batches of tickets a workgroup knows of */
+
+/* The tickets of a workgroup.  One atomic on the launch's counter draws a
+ * batch of B consecutive tickets (they serialise at about 12 ns each: with 4
+ * to an atomic they bounded the FP32 factors of 2.65M vertices at 8.1 ms, with
+ * 8 those take 4.6), and the workgroup's wavefronts take them one by one from
+ * LDS, in order and without waiting for one another.  B is the number of
+ * wavefronts: more rows of one level to a wavefront take it longer, fewer
+ * serialise.  The wavefront that takes the first of batch k
+ * draws batch k + 2 (after k + 1 has been stored, so that a workgroup's
+ * batches ascend), and stores it once it is back, before it waits for any
+ * row: entry k % ILU_RING of the ring is k << 32 | first ticket, `read`
+ * counts the tickets taken of it.
+ * No wait can deadlock: a wavefront takes its next ticket when the row it
+ * holds needs no other row any more, so the oldest unfinished ticket of the
+ * launch is held by a running wavefront whose dependences are all finished,
+ * and the wavefront that is to store a batch stores it without waiting for a
+ * row.  The counter advances by kf_ticket_advance_ring(). */
+struct ilu_ring {
+  unsigned long long entry[ILU_RING];
+  uint32_t read[ILU_RING], head;
+};
+
+static inline uint32_t kf_ticket_advance_ring(uint32_t ntask, uint32_t nb, uint32_t B)
+{
+  return B * ((ntask + B - 1) / B + 2 * nb);
+}
+
+template <typename V>
+__device__ __forceinline__ V lds_load(V *p)
+{
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+template <typename V>
+__device__ __forceinline__ void lds_store(V *p, V v)
+{
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+/* a row's schedule, the same for the whole wavefront */
+struct ilu_row {
+  uint32_t i, j0, L, nlow, mbeg, mcnt;
+};
+
+/* the end of the pairs of lower block p - 1, from the register that holds
+ * moff by lane (its lanes past the row's lower blocks hold the pair count) */
+__device__ __forceinline__ uint32_t step_end(uint32_t moreg, const uint32_t *smoff, uint32_t p)
+{
+  if (p < 64) return __builtin_amdgcn_readlane(moreg, p);
+  return __builtin_amdgcn_readfirstlane(smoff[p]);
+}
 
 /* k_ilu with the row's schedule precomputed on the host (kf_plan_ilu): a
  * record per ticket, the diagonal position of every row it reads from and
- * the list of update pairs (U(m,k) block, position of k in row i).  The wave
- * loads, in one round, its row, those tables and its L_old blocks, then
- * stages inv(U(m,m)), U(m,m) and the U(m,k) blocks in LDS from the
- * published copies (apub, udpub), retrying values that still hold the
+ * the list of update pairs (U(m,k) block, position of k in row i).  The
+ * wavefront stages inv(U(m,m)), U(m,m) and the U(m,k) blocks in LDS from the
+ * published copies (apub), retrying values that still hold the
  * call's sentinel (handoff.h): no flags, no fences.  The rest runs from
- * LDS; the row then stores its factors in place and publishes its diagonal
- * inverse, upper blocks and U(i,i).  Arithmetic and its order are those of
- * k_ilu. */
+ * LDS; the row then publishes its upper blocks, U(i,i) and diagonal inverse
+ * and stores its factors in place.  Arithmetic and its order are those of
+ * k_ilu.
+ *
+ * Bound by rows in flight times the time a wavefront spends on one: the
+ * round trip for the published blocks (2.4 us under load), the chain of the
+ * elimination and the inverse.  So the next row's record and blocks are
+ * loaded while this one computes, what its chain does not need is formed
+ * while the published blocks are on their way, and their places are one
+ * table, so that all of a lane's loads go out together.  Against a version
+ * that took each block's place from one of three tables on its own branch,
+ * formed L(i,m) on 16 lanes through LDS and loaded each row when its
+ * predecessor was done: FP64 (exact) 2.05 -> 1.65 ms on 331,776 vertices and
+ * 12.7 -> 10.0 ms on 2.65M, FP32 1.36 -> 1.22 and 8.1 -> 4.6 ms. */
 template <typename T, bool EXACT>
-__global__ __launch_bounds__(256) void k_ilu_rows(kf_dv d, const uint32_t *__restrict__ rec, uint32_t nrows,
-                                                 uint32_t *ticket, uint32_t base, T *apub, T *udpub,
-                                                 typename sentinel<T>::bits snt, T *a, T *lold,
-                                                 const uint32_t *__restrict__ ldiag,
-                                                 const uint32_t *__restrict__ moff, const uint32_t *__restrict__ mjm,
-                                                 const uint16_t *__restrict__ mlo, uint32_t maxrow, uint32_t maxlow,
-                                                 uint32_t maxmatch)
+__global__ __launch_bounds__(64 * ILU_GMAX, sizeof(T) == 8 ? 2 : 3)
+void k_ilu_rows(kf_dv d, const uint32_t *__restrict__ rec, uint32_t nrows, uint32_t *ticket, uint32_t base, uint32_t B,
+                uint32_t nnzb, T *apub, typename sentinel<T>::bits snt, T *a, T *lold, const uint32_t *__restrict__ ldiag,
+                const uint32_t *__restrict__ moff, const uint32_t *__restrict__ mjm, const uint16_t *__restrict__ mlo,
+                uint32_t maxrow, uint32_t maxlow, uint32_t maxmatch)
 {
   extern __shared__ __align__(16) unsigned char ilu_lds_all[];
-  __shared__ uint32_t sbatch;
+  __shared__ ilu_ring ring;
   const ilu_layout lay(maxrow, maxlow, maxmatch, sizeof(T), EXACT);
-  const uint32_t G = blockDim.x >> 6, wv = threadIdx.x >> 6;
-  unsigned char *ilu_lds = ilu_lds_all + (size_t)wv * lay.bytes;   /* this wave's region */
-  uint32_t *scol = (uint32_t *)(ilu_lds + lay.scol);
+  unsigned char *ilu_lds = ilu_lds_all + (size_t)(threadIdx.x >> 6) * lay.bytes;   /* this wave's region */
   T *sa = (T *)(ilu_lds + lay.sa);
   T *sa0 = (T *)(ilu_lds + lay.sa0);
-  uint32_t *sldg = (uint32_t *)(ilu_lds + lay.sldg);
+  uint32_t *ssrc = (uint32_t *)(ilu_lds + lay.ssrc);
   uint32_t *smoff = (uint32_t *)(ilu_lds + lay.smoff);
-  uint32_t *sjm = (uint32_t *)(ilu_lds + lay.sjm);
   uint16_t *slo = (uint16_t *)(ilu_lds + lay.slo);
   T *stage = (T *)(ilu_lds + lay.stage);
   const uint32_t lane = threadIdx.x & 63u;
   const uint32_t e = lane & 15, er = e >> 2, ec = e & 3, grp = lane >> 4;
   bool aborted = false;
-  /* G consecutive tickets per atomic, one row per wavefront; the workgroup
-   * takes the next G when all its rows are done (sync.h) */
-  if (threadIdx.x == 0) sbatch = atomicAdd(ticket, G) - base;
-  __syncthreads();
-  uint32_t bstart = sbatch;
-  for (;;) {
-    if (bstart >= nrows) break;   /* uniform over the workgroup */
-    uint32_t nxt = 0;
-    if (threadIdx.x == 0) nxt = atomicAdd(ticket, G);
-    const uint32_t t = bstart + wv;
-    if (t < nrows) {
-    const uint32_t rv = lane < 6 ? rec[8 * (size_t)t + lane] : 0;
-    const uint32_t i = __shfl(rv, 0, 64), j0 = __shfl(rv, 1, 64), L = __shfl(rv, 2, 64);
-    const uint32_t nlow = __shfl(rv, 3, 64), mbeg = __shfl(rv, 4, 64), mcnt = __shfl(rv, 5, 64);
-    const uint32_t pd = nlow;
-    /* staged slots: [0, nlow) inv(U(m,m)); EXACT: [nlow, 2 nlow) U(m,m),
-     * [2 nlow, 3 nlow) L_old; then the U(m,k) blocks of the update pairs */
-    const uint32_t mbase = EXACT ? 3 * nlow : nlow;
-    /* one round of loads: row i, the tables, L_old (rows beyond the
-     * register round take the loops below) */
-    {
-      T av[ILU_Q], lv[ILU_Q];
-      uint32_t cv = 0, gv = 0, mo = 0, jv = 0;
-      uint16_t ov = 0;
+  /* the cofactor expression of this lane's entry: 18 factor positions of 4
+   * bits and the signs, kept in registers (three words and a byte) */
+  uint32_t cof[3];
 #pragma unroll
-      for (int q = 0; q < ILU_Q; q++) {
-        const uint32_t k = lane + 64 * q;
-        if (k < 16 * L) av[q] = a[16 * (size_t)j0 + k];
-        if (EXACT && k < 16 * nlow) {
-          const uint32_t pp = k >> 4, ee = k & 15;
-          lv[q] = pp == 0 ? a[16 * ((size_t)j0 + nlow - 1) + ee] : lold[16 * ((size_t)j0 + pp) + ee];
-        }
-      }
-      if (lane < L) cv = d.col[j0 + lane];
-      if (lane < nlow) { gv = ldiag[j0 + lane]; mo = moff[j0 + lane]; }
-      if (lane < mcnt) { jv = mjm[mbeg + lane]; ov = mlo[mbeg + lane]; }
+  for (int w = 0; w < 3; w++) {
+    cof[w] = 0;
 #pragma unroll
-      for (int q = 0; q < ILU_Q; q++) {
-        const uint32_t k = lane + 64 * q;
-        if (k < 16 * L) {
-          sa[k] = av[q];
-          if (EXACT) sa0[k] = av[q];
-        }
-        if (EXACT && k < 16 * nlow) stage[32 * nlow + k] = lv[q];
-      }
-      if (lane < L) scol[lane] = cv;
-      if (lane < nlow) { sldg[lane] = gv; smoff[lane] = mo; }
-      if (lane < mcnt) { sjm[lane] = jv; slo[lane] = ov; }
-      if (lane == 0) smoff[nlow] = mcnt;
-      for (uint32_t k = lane + 64 * ILU_Q; k < 16 * L; k += 64) {
-        const T v = a[16 * (size_t)j0 + k];
-        sa[k] = v;
-        if (EXACT) sa0[k] = v;
-      }
-      if (EXACT)
-        for (uint32_t k = lane + 64 * ILU_Q; k < 16 * nlow; k += 64)
-          stage[32 * nlow + k] = lold[16 * ((size_t)j0 + (k >> 4)) + (k & 15)];
-      for (uint32_t k = lane + 64; k < L; k += 64) scol[k] = d.col[j0 + k];
-      for (uint32_t k = lane + 64; k < nlow; k += 64) { sldg[k] = ldiag[j0 + k]; smoff[k] = moff[j0 + k]; }
-      for (uint32_t k = lane + 64; k < mcnt; k += 64) { sjm[k] = mjm[mbeg + k]; slo[k] = mlo[mbeg + k]; }
+    for (int q = 0; q < 6; q++) cof[w] |= (uint32_t)kf_cof_idx[e][2 * w + q / 3][q % 3] << (4 * q);
+  }
+  const uint32_t neg = kf_cof_neg[e];
+
+  if (threadIdx.x == 0) {
+    /* batches 0 and 1, one after the other: a workgroup's batches ascend */
+    for (uint32_t k = 0; k < ILU_RING; k++) {
+      ring.entry[k] = k < 2 ? (unsigned long long)k << 32 | (atomicAdd(ticket, B) - base) : ~0ull;
+      ring.read[k] = k < 2 ? 0u : B;
     }
+    ring.head = 0;
+  }
+  __syncthreads();
+
+  /* the wavefront's next ticket; a drawn batch is in `drawn` until put() */
+  uint32_t put_k = 0, drawn = 0;
+  auto entry = [&](uint32_t k) -> uint32_t {   /* batch k's first ticket, once it is stored */
+    unsigned long long en = lds_load(&ring.entry[k % ILU_RING]);
+    for (uint32_t n = 0; (uint32_t)(en >> 32) != k; n++) {
+      if (n > KF_SPIN_LIMIT) {
+        if (lane == 0) atomicOr(d.err, KF_ERR_SPIN_LIMIT);
+        return nrows;
+      }
+      __builtin_amdgcn_s_sleep(1);
+      en = lds_load(&ring.entry[k % ILU_RING]);
+    }
+    return __builtin_amdgcn_readfirstlane((uint32_t)en);
+  };
+  auto take = [&]() -> uint32_t {
+    uint32_t q = 0;
+    if (lane == 0) q = atomicAdd(&ring.head, 1u);
+    q = __builtin_amdgcn_readfirstlane(q);
+    const uint32_t k = q / B, j = q % B, r = k % ILU_RING;
+    const uint32_t start = entry(k);
+    if (lane == 0) atomicAdd(&ring.read[r], 1u);
+    if (j == 0) {
+      entry(k + 1);   /* drawn and back: k + 2 is drawn after it */
+      put_k = k + 2;
+      drawn = nrows;
+      if (start < nrows && lane == 0) drawn = atomicAdd(ticket, B) - base;
+    }
+    return start + j;
+  };
+  auto put = [&]() {
+    if (!put_k) return;
+    const uint32_t r = put_k % ILU_RING;
+    for (uint32_t n = 0; lds_load(&ring.read[r]) != B && n <= KF_SPIN_LIMIT; n++) __builtin_amdgcn_s_sleep(1);
+    if (lane == 0) {
+      lds_store(&ring.read[r], 0u);
+      lds_store(&ring.entry[r], (unsigned long long)put_k << 32 | drawn);
+    }
+    put_k = 0;
+  };
+
+  /* a row's record, then its blocks, tables and L_old in one round of loads
+   * (what lies beyond the round is loaded in load_rest) */
+  uint32_t rv = 0, cv = 0, gv = 0, mo = 0, jv = 0;
+  uint16_t ov = 0;
+  T av[ILU_Q], lv[ILU_Q];
+  ilu_row w;
+  auto load_rec = [&](uint32_t t) { rv = t < nrows && lane < 6 ? rec[8 * (size_t)t + lane] : 0u; };
+  auto load_row = [&]() {
+    w.i = __builtin_amdgcn_readlane(rv, 0);
+    w.j0 = __builtin_amdgcn_readlane(rv, 1);
+    w.L = __builtin_amdgcn_readlane(rv, 2);
+    w.nlow = __builtin_amdgcn_readlane(rv, 3);
+    w.mbeg = __builtin_amdgcn_readlane(rv, 4);
+    w.mcnt = __builtin_amdgcn_readlane(rv, 5);
+    if (lane < w.nlow) {
+      gv = ldiag[w.j0 + lane];
+      mo = moff[w.j0 + lane];
+      if (EXACT) cv = d.col[w.j0 + lane];
+    } else {
+      mo = w.mcnt;
+    }
+    if (lane < w.mcnt) { jv = mjm[w.mbeg + lane]; ov = mlo[w.mbeg + lane]; }
+#pragma unroll
+    for (int q = 0; q < ILU_Q; q++) {
+      const uint32_t k = lane + 64 * q;
+      if (k < 16 * w.L) av[q] = a[16 * (size_t)w.j0 + k];
+      if (EXACT && k < 16 * w.nlow) {
+        const uint32_t pp = k >> 4, ee = k & 15;
+        lv[q] = pp == 0 ? a[16 * ((size_t)w.j0 + w.nlow - 1) + ee] : lold[16 * ((size_t)w.j0 + pp) + ee];
+      }
+    }
+  };
+
+  uint32_t t = take();
+  load_rec(t);
+  put();
+  load_row();
+  while (t < nrows) {
+    const uint32_t i = w.i, j0 = w.j0, L = w.L, nlow = w.nlow, mcnt = w.mcnt, pd = w.nlow, moreg = mo;
+    /* staged blocks: [0, nlow) inv(U(m,m)); EXACT: [nlow, 2 nlow) U(m,m);
+     * from mbase the U(m,k) of the update pairs; from lbase (EXACT) L_old.
+     * ssrc: where the published ones stand, in blocks of apub (the U(m,m)
+     * follow its nnzb blocks). */
+    const uint32_t mbase = EXACT ? 2 * nlow : nlow, nsrc = mbase + mcnt, lbase = nsrc + 8;
+    for (uint32_t k = lane, first = 1; k < nlow; k += 64, first = 0) {
+      ssrc[k] = first ? gv : ldiag[j0 + k];
+      smoff[k] = first ? mo : moff[j0 + k];
+      if (EXACT) ssrc[nlow + k] = nnzb + (first ? cv : d.col[j0 + k]);
+    }
+    for (uint32_t k = lane, first = 1; k < mcnt; k += 64, first = 0) {
+      ssrc[mbase + k] = first ? jv : mjm[w.mbeg + k];
+      slo[k] = 16 * (first ? ov : mlo[w.mbeg + k]);
+    }
+    if (lane < 8) slo[mcnt + lane] = 0;
+    if (lane == 0) smoff[nlow] = mcnt;
     wave_lds_sync();
-    /* staging from the published copies, ILU_QB values per lane per round;
-     * a value still holding the sentinel is loaded again */
-    {
-      const uint32_t npre = EXACT ? 2 * nlow : nlow;
-      const uint32_t tot = 16 * (npre + mcnt);
-      for (uint32_t b0 = 0; b0 < tot; b0 += 64 * ILU_QB) {
-        uint32_t need = 0;
+    /* the published blocks, ILU_QB values per lane per round (a lane past the
+     * end reads the last block and drops it); a value still holding the
+     * sentinel is loaded again.  While the first round is on its way the
+     * row's own blocks go to LDS. */
+    const uint32_t tot = 16 * nsrc;
+    for (uint32_t b0 = 0; b0 == 0 || b0 < tot; b0 += 64 * ILU_QB) {
+      uint32_t need = 0, blk[ILU_QB];
+      T v[ILU_QB];
+      if (tot) {
+#pragma unroll
+        for (int q = 0; q < ILU_QB; q++) blk[q] = ssrc[min(b0 / 16 + grp + 4 * q, nsrc - 1)];
+#pragma unroll
+        for (int q = 0; q < ILU_QB; q++) {
+          v[q] = ld_coherent(apub + 16 * (size_t)blk[q] + e);
+          if (b0 + lane + 64 * q < tot) need |= 1u << q;
+        }
+      }
+      if (b0 == 0) {
+#pragma unroll
+        for (int q = 0; q < ILU_Q; q++) {
+          const uint32_t k = lane + 64 * q;
+          if (k < 16 * L) {
+            sa[k] = av[q];
+            if (EXACT) sa0[k] = av[q];
+          }
+          if (EXACT && k < 16 * nlow) stage[16 * lbase + k] = lv[q];
+        }
+        for (uint32_t k = lane + 64 * ILU_Q; k < 16 * L; k += 64) {
+          const T x = a[16 * (size_t)j0 + k];
+          sa[k] = x;
+          if (EXACT) sa0[k] = x;
+        }
+        if (EXACT) {
+          for (uint32_t k = lane + 64 * ILU_Q; k < 16 * nlow; k += 64)
+            stage[16 * lbase + k] = lold[16 * ((size_t)j0 + (k >> 4)) + (k & 15)];
+          wave_lds_sync();
+          /* I A(i,k) of the upper blocks (in place: a group's lanes read
+           * the whole block before they store it) */
+          for (uint32_t p = pd + grp; p < L; p += 4) {
+            const T *a0 = sa0 + 16 * p;
+            T dq = T(0);
+#pragma unroll
+            for (int k = 0; k < 4; k++) dq += (er == (uint32_t)k ? T(1) : T(0)) * a0[4 * k + ec];
+            sa0[16 * p + e] = dq;
+          }
+        }
+      }
+      for (uint32_t n = 0;; n++) {
 #pragma unroll
         for (int q = 0; q < ILU_QB; q++)
-          if (b0 + lane + 64 * q < tot) need |= 1u << q;
-        for (uint32_t n = 0; need && !aborted; n++) {
-          if (n > 0) {
-            if (n > KF_SPIN_LIMIT) {
-              atomicOr(d.err, KF_ERR_SPIN_LIMIT);
-              aborted = true;
-              break;
-            }
-            for (uint32_t z = 0; z < d.spin_sleep; z++) __builtin_amdgcn_s_sleep(1);
+          if ((need & (1u << q)) && sentinel<T>::raw(v[q]) != snt) {
+            stage[b0 + lane + 64 * q] = v[q];
+            need &= ~(1u << q);
           }
-          T v[ILU_QB];
-#pragma unroll
-          for (int q = 0; q < ILU_QB; q++)
-            if (need & (1u << q)) {
-              const uint32_t k = b0 + lane + 64 * q, sl = k >> 4, ee = k & 15;
-              const T *src;
-              if (sl < nlow) src = apub + 16 * (size_t)sldg[sl];
-              else if (EXACT && sl < 2 * nlow) src = udpub + 16 * (size_t)scol[sl - nlow];
-              else src = apub + 16 * (size_t)sjm[sl - npre];
-              v[q] = ld_coherent(src + ee);
-            }
-#pragma unroll
-          for (int q = 0; q < ILU_QB; q++)
-            if ((need & (1u << q)) && sentinel<T>::raw(v[q]) != snt) {
-              const uint32_t k = b0 + lane + 64 * q, sl = k >> 4;
-              stage[16 * (sl < npre ? sl : sl - npre + mbase) + (k & 15)] = v[q];
-              need &= ~(1u << q);
-            }
+        if (!need || aborted) break;
+        if (n >= KF_SPIN_LIMIT) {
+          atomicOr(d.err, KF_ERR_SPIN_LIMIT);
+          aborted = true;
+          break;
         }
+        for (uint32_t z = 0; z < d.spin_sleep; z++) __builtin_amdgcn_s_sleep(1);
+#pragma unroll
+        for (int q = 0; q < ILU_QB; q++)
+          if (need & (1u << q)) v[q] = ld_coherent(apub + 16 * (size_t)blk[q] + e);
       }
-      aborted = __any(aborted);   /* a wave gives up at most once per launch */
     }
+    aborted = __any(aborted);   /* a wave gives up at most once per launch */
+    /* nothing is waited for from here to the row's end: take the next ticket */
+    t = take();
+    load_rec(t);
     wave_lds_sync();
 
-    for (uint32_t p = 0; p < nlow; p++) {
-      if (EXACT) {
-        /* a(i,m) = (a - L_old U(m,m)) + L_old U(m,m) */
-        if (lane < 16) {
-          const T dq = blk_mul(stage + 16 * (2 * nlow + p), stage + 16 * (nlow + p), er, ec);
-          T v = sa[16 * p + e];
+    if (EXACT) {
+      /* L_old(i,m) U(m,m) of all lower blocks, four at a time, into L_old's place */
+      for (uint32_t p = grp; p < nlow; p += 4) {
+        T *q = stage + 16 * (lbase + p);
+        const T dq = blk_mul(q, stage + 16 * (nlow + p), er, ec);
+        q[e] = dq;
+      }
+      wave_lds_sync();
+    }
+    /* The elimination.  The row's chain is a(i,m) -> L(i,m) -> the updates
+     * of row i -> the next a(i,m): every group of 16 lanes forms L(i,m) by
+     * itself (its quads hold the block's rows, so the product needs no
+     * exchange through LDS), and all operands of a step are read at once,
+     * without a branch: the pairs' bounds are scalars, their targets are
+     * known one step ahead, and a lane past the step's pairs works on some
+     * other pair (the table ends in 8 spare ones) and does not store. */
+    {
+      uint32_t i0 = 0, i1 = step_end(moreg, smoff, 1);
+      uint32_t o0 = slo[grp], o1 = slo[grp + 4];
+      for (uint32_t p = 0; p < nlow; p++) {
+        const bool on0 = i0 + grp < i1, on1 = i0 + grp + 4 < i1, two = i1 - i0 > 4;
+        T v = sa[16 * p + e], dq = T(0), bi[4], u0[4], u1[4];
+        if (EXACT) dq = stage[16 * (lbase + p) + e];
+        const T t0 = sa[o0 + e], t1 = sa[o1 + e];
+        blk_col(stage + 16 * p, ec, bi);
+        blk_col(stage + 16 * (mbase + i0 + grp), ec, u0);
+        if (two) blk_col(stage + 16 * (mbase + i0 + grp + 4), ec, u1);
+        const uint32_t i2 = step_end(moreg, smoff, p + 2 < nlow ? p + 2 : nlow);
+        const uint32_t n0 = slo[i1 + grp], n1 = slo[i1 + grp + 4];
+        if (EXACT) {
+          /* a(i,m) = (a - L_old U(m,m)) + L_old U(m,m) */
           v = T(-1) * dq + v;
           v = T(1) * dq + v;
-          sa[16 * p + e] = v;
+        }
+        const T lw = row_mul(v, bi);   /* L(i,m) = a(i,m) inv(U(m,m)) */
+        if (grp == 0) sa[16 * p + e] = lw;
+        /* a(i,k) -= L(i,m) U(m,k) for the update pairs of m (distinct k) */
+        const T s0 = t0 - row_mul(lw, u0);
+        if (on0) sa[o0 + e] = s0;
+        if (two) {
+          const T s1 = t1 - row_mul(lw, u1);
+          if (on1) sa[o1 + e] = s1;
+          for (uint32_t x = i0 + 8; x < i1; x += 4) {
+            const uint32_t o2 = slo[x + grp];
+            T u2[4];
+            blk_col(stage + 16 * (mbase + x + grp), ec, u2);
+            const T s2 = sa[o2 + e] - row_mul(lw, u2);
+            if (x + grp < i1) sa[o2 + e] = s2;
+          }
         }
         wave_lds_sync();
+        i0 = i1;
+        i1 = i2;
+        o0 = n0;
+        o1 = n1;
       }
-      /* L(i,m) = a(i,m) inv(U(m,m)) */
-      T lv = T(0);
-      if (lane < 16) lv = blk_mul(sa + 16 * p, stage + 16 * p, er, ec);
-      wave_lds_sync();
-      if (lane < 16) sa[16 * p + e] = lv;
-      wave_lds_sync();
-      /* a(i,k) -= L(i,m) U(m,k) for the update pairs of m (distinct k) */
-      for (uint32_t idx = smoff[p] + grp; idx < smoff[p + 1]; idx += 4) {
-        const uint32_t lo = slo[idx];
-        const T s = blk_mul(sa + 16 * p, stage + 16 * (size_t)(mbase + idx), er, ec);
-        sa[16 * lo + e] = sa[16 * lo + e] - s;
-      }
-      wave_lds_sync();
     }
 
     if (EXACT) {
       /* upper blocks: a = (a - I A(i,k)) + I A(i,k), A = the fill's block */
       for (uint32_t p = pd + grp; p < L; p += 4) {
-        const T *a0 = sa0 + 16 * p;
-        T dq = T(0);
-#pragma unroll
-        for (int k = 0; k < 4; k++) dq += (er == (uint32_t)k ? T(1) : T(0)) * a0[4 * k + ec];
+        const T dq = sa0[16 * p + e];
         T v = sa[16 * p + e];
         v = T(-1) * dq + v;
         v = T(1) * dq + v;
         sa[16 * p + e] = v;
       }
       wave_lds_sync();
-      if (lane < 16) st_coherent(udpub + 16 * (size_t)i + e, canon(sa[16 * pd + e]));
+      if (lane < 16) st_coherent(apub + 16 * ((size_t)nnzb + i) + e, canon(sa[16 * pd + e]));
     }
-
+    /* published copies of what later rows read, as soon as they are final:
+     * U(i,k) before the diagonal's inverse, both before this row's own stores */
+    for (uint32_t k = 16 + lane; k < 16 * (L - pd); k += 64)
+      st_coherent(apub + 16 * ((size_t)j0 + pd) + k, canon(sa[16 * pd + k]));
     {
       const T *s = sa + 16 * pd;
-      const uint8_t neg = kf_cof_neg[e];
-      T acc = s[kf_cof_idx[e][0][0]];
+      T f[18];
+#pragma unroll
+      for (int q = 0; q < 18; q++) f[q] = s[(cof[q / 6] >> (4 * (q % 6))) & 15u];
+      const T s0 = s[0], s1 = s[1], s2 = s[2], s3 = s[3];
+      T acc = f[0];
       if (neg & 1u) acc = -acc;
-      acc = acc * s[kf_cof_idx[e][0][1]] * s[kf_cof_idx[e][0][2]];
+      acc = acc * f[1] * f[2];
 #pragma unroll
       for (int tt = 1; tt < 6; tt++) {
-        const T pr = s[kf_cof_idx[e][tt][0]] * s[kf_cof_idx[e][tt][1]] * s[kf_cof_idx[e][tt][2]];
+        const T pr = f[3 * tt] * f[3 * tt + 1] * f[3 * tt + 2];
         acc = (neg & (1u << tt)) ? acc - pr : acc + pr;
       }
-      const T d0 = __shfl(acc, 0, 16), d4 = __shfl(acc, 4, 16), d8 = __shfl(acc, 8, 16), d12 = __shfl(acc, 12, 16);
-      T det = s[0] * d0 + s[1] * d4 + s[2] * d8 + s[3] * d12;
+      const T d0 = lane_get(acc, 0), d4 = lane_get(acc, 4), d8 = lane_get(acc, 8), d12 = lane_get(acc, 12);
+      T det = s0 * d0 + s1 * d4 + s2 * d8 + s3 * d12;
       det = T(1) / det;
       acc *= det;
       wave_lds_sync();
       if (lane < 16) {
+        st_coherent(apub + 16 * ((size_t)j0 + pd) + e, canon(acc));
         if (!isfinite((double)acc)) atomicOr(d.err, KF_ERR_NONFINITE_PIVOT);
         sa[16 * pd + e] = acc;
       }
     }
+    put();
+    if (t < nrows) load_row();
     wave_lds_sync();
     for (uint32_t k = lane; k < 16 * L; k += 64) a[16 * (size_t)j0 + k] = sa[k];
     if (EXACT)
       for (uint32_t k = lane; k < 16 * nlow; k += 64) lold[16 * (size_t)j0 + k] = sa[k];
-    /* published copies of what later rows read: inv(U(i,i)) and U(i,k) */
-    for (uint32_t k = lane; k < 16 * (L - pd); k += 64)
-      st_coherent(apub + 16 * ((size_t)j0 + pd) + k, canon(sa[16 * pd + k]));
-    }
-    __syncthreads();   /* every row of the batch done; sbatch free */
-    if (threadIdx.x == 0) sbatch = nxt - base;
-    __syncthreads();
-    bstart = sbatch;
+    wave_lds_sync();
   }
 }
 
@@ -435,36 +653,45 @@ static uint32_t persistent_waves(uint32_t work, uint32_t cap)
 template <typename T, bool EXACT>
 static void launch_ilu(kf_ctx *c, T *a, T *lold, T *ud)
 {
-  /* the context's setting, else 2048 waves for FP64 and 3072 for the
-   * single-precision factors (8.8 -> 8.1 ms per factorisation on the
-   * 2.65M-vertex lattice; FP64 is flat from 2048 to 4096) */
-  const uint32_t nw = persistent_waves(c->d.N, c->ilu_waves ? c->ilu_waves : (sizeof(T) == 8 ? 2048u : 3072u));
+  /* the context's setting, else what fits the registers: 2048 waves in FP64
+   * (221 VGPRs, two per SIMD; capped at three the exact sweep spills and
+   * takes twice as long), and for the single-precision factors (127 VGPRs)
+   * 4096 where the schedule has that many rows to a level, 3072 below, where
+   * waves that wait for later levels only crowd the polls (2.65M vertices:
+   * 5.3 -> 4.6 ms; 161K: 0.87 against 0.90 ms) */
+  const bool wide = (uint64_t)c->d.N >= 3072ull * (c->nlev_l ? c->nlev_l : 1);
+  const uint32_t nw =
+      persistent_waves(c->d.N, c->ilu_waves ? c->ilu_waves : sizeof(T) == 8 ? 2048u : wide ? 4096u : 3072u);
   const ilu_layout lay(c->ilu_maxrow, c->ilu_maxlow, c->ilu_maxmatch, sizeof(T), EXACT);
-  /* wavefronts per workgroup: as asked, within 4 and 64 KB of LDS */
+  /* wavefronts per workgroup and rows per batch: as asked, within the LDS */
   uint32_t G = c->ilu_group;
-  const size_t lds_cap = c->lds_max < 64 * 1024 ? c->lds_max : 64 * 1024;
+  const size_t lds_cap = c->lds_max - sizeof(ilu_ring);
   while (G > 1 && G * (size_t)lay.bytes > lds_cap) G--;
   if (lay.bytes <= lds_cap) {
     const uint32_t nb = (nw + G - 1) / G;
-    /* published copies, preset to this call's sentinel */
-    const size_t na = 16 * c->nnzb, nu = 16 * (size_t)c->d.N;
-    if (!c->ilu_apub) KF_CHECK(hipMalloc(&c->ilu_apub, na * sizeof(double)));
-    if (EXACT && !c->ilu_udpub) KF_CHECK(hipMalloc(&c->ilu_udpub, nu * sizeof(double)));
+    /* published copies (the blocks of A, then the U(i,i)), preset to this
+     * call's sentinel */
+    const size_t na = 16 * (c->nnzb + (EXACT ? (size_t)c->d.N : 0));
+    if (c->ilu_napub < na) {
+      KF_CHECK(hipStreamSynchronize(c->stream));
+      if (c->ilu_apub) KF_CHECK(hipFree(c->ilu_apub));
+      KF_CHECK(hipMalloc(&c->ilu_apub, na * sizeof(double)));
+      c->ilu_napub = na;
+    }
     const typename sentinel<T>::bits snt = sentinel<T>::of(++c->icall);
-    T *apub = (T *)c->ilu_apub, *udpub = EXACT ? (T *)c->ilu_udpub : NULL;
+    T *apub = (T *)c->ilu_apub;
     hipLaunchKernelGGL((k_fill_bits<T>), dim3(kf_blocks_for(na, 256)), dim3(256), 0, c->stream, apub, na, snt);
     KF_LAUNCH_CHECK();
-    if (EXACT) {
-      hipLaunchKernelGGL((k_fill_bits<T>), dim3(kf_blocks_for(nu, 256)), dim3(256), 0, c->stream, udpub, nu, snt);
-      KF_LAUNCH_CHECK();
-    }
+    if (G * (size_t)lay.bytes > 64 * 1024)
+      KF_CHECK(hipFuncSetAttribute((const void *)k_ilu_rows<T, EXACT>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                   (int)(G * lay.bytes)));
     const int s = kf_prof_begin(c, KP_ILU);
     hipLaunchKernelGGL((k_ilu_rows<T, EXACT>), dim3(nb), dim3(64 * G), G * lay.bytes, c->stream, c->d, c->ilu_rec,
-                       c->d.N, c->ticket + 2, c->ticket_base[2], apub, udpub, snt, a, lold, c->ilu_ldiag, c->ilu_moff,
-                       c->ilu_mjm, c->ilu_mlo, c->ilu_maxrow, c->ilu_maxlow, c->ilu_maxmatch);
+                       c->d.N, c->ticket + 2, c->ticket_base[2], G, (uint32_t)c->nnzb, apub, snt, a, lold, c->ilu_ldiag,
+                       c->ilu_moff, c->ilu_mjm, c->ilu_mlo, c->ilu_maxrow, c->ilu_maxlow, c->ilu_maxmatch);
     KF_LAUNCH_CHECK();
     kf_prof_end(c, s);
-    c->ticket_base[2] += kf_ticket_advance_groups(c->d.N, nb, G);
+    c->ticket_base[2] += kf_ticket_advance_ring(c->d.N, nb, G);
   } else {
     const uint32_t epoch = ++c->epoch;
     const int s = kf_prof_begin(c, KP_ILU);

@@ -114,7 +114,8 @@ struct kf_ctx {
   uint32_t *ilu_rec, *ilu_ldiag, *ilu_moff, *ilu_mjm;
   uint16_t *ilu_mlo;
   uint32_t ilu_maxrow, ilu_maxlow, ilu_maxmatch;
-  void *ilu_apub, *ilu_udpub; /* published diagonal inverses and U blocks, U(i,i) */
+  void *ilu_apub;             /* published diagonal inverses and U blocks, then U(i,i) */
+  size_t ilu_napub;           /* ... values it holds */
   uint64_t icall;             /* ILU calls so far (sentinel numbering) */
   uint32_t trsv_waves, ilu_waves;   /* persistent wavefronts per launch (trsv: 0 = sized) */
   uint32_t trsv_auto;               /* triangular solves: waves for ~3.5 task levels in flight */

@@ -8,9 +8,10 @@
  * dispatch order of workgroups.
  *
  * One atomic on a single counter serialises at the memory side (about
- * 11 ns each on MI355X), so the planned kernels take G consecutive tickets
+ * 11 ns each on MI355X), so the triangular solves take G consecutive tickets
  * per atomic for a workgroup of G wavefronts, one ticket each, and the
- * group's next G once all G are done.  Every ticket below the oldest
+ * group's next G once all G are done (the planned ILU hands a batch out one
+ * by one, ilu.hip).  Every ticket below the oldest
  * unfinished one is finished and every ticket of a running group is being
  * worked on, so the oldest unfinished ticket of the launch belongs to a
  * running wave whose dependences are all finished: no wait can deadlock.
