@@ -252,7 +252,6 @@ struct ilu_layout {
 };
 
 #define ILU_Q 4    /* values per lane per load round before the wait */
-#define ILU_QB 12  /* values per lane per staging round after the wait */
 #define ILU_GMAX 8 /* wavefronts per workgroup at most */
 #define ILU_RING 4 /* batches of tickets a workgroup knows of */
 
@@ -327,13 +326,60 @@ __device__ __forceinline__ uint32_t step_end(uint32_t moreg, const uint32_t *smo
  * formed L(i,m) on 16 lanes through LDS and loaded each row when its
  * predecessor was done: FP64 (exact) 2.05 -> 1.65 ms on 331,776 vertices and
  * 12.7 -> 10.0 ms on 2.65M, FP32 1.36 -> 1.22 and 8.1 -> 4.6 ms. */
-template <typename T, bool EXACT>
-__global__ __launch_bounds__(64 * ILU_GMAX, sizeof(T) == 8 ? 2 : 3)
+/* where a row's factors go beside a: the BF16 copy (TS = uint16_t) and, with
+ * Jacobi sweeps, the sweeps' sliced copy (val; layout at k_jac_lower_sl), in
+ * TS.  Written from the row in LDS, they cost their own stores; as passes
+ * after the factorisation the two read and wrote the factors again (1.12M
+ * vertices and seven coarse levels: 1.08 ms of 8.0). */
+struct ilu_out {
+  uint16_t *abf;
+  void *val;
+  uint32_t K, nslice;
+};
+
+__device__ __forceinline__ void ilu_cvt(double v, double *o) { *o = v; }
+__device__ __forceinline__ void ilu_cvt(float v, float *o) { *o = v; }
+__device__ __forceinline__ void ilu_cvt(float v, uint16_t *o)   /* round to nearest even */
+{
+  uint32_t u = __float_as_uint(v);
+  u += 0x7FFFu + ((u >> 16) & 1u);
+  *o = (uint16_t)(u >> 16);
+}
+
+__device__ __forceinline__ void ilu_ld4(const float *p, float x[4])
+{
+  const float4 v = *reinterpret_cast<const float4 *>(p);
+  x[0] = v.x; x[1] = v.y; x[2] = v.z; x[3] = v.w;
+}
+__device__ __forceinline__ void ilu_ld4(const double *p, double x[4])
+{
+  const double2 u = reinterpret_cast<const double2 *>(p)[0], v = reinterpret_cast<const double2 *>(p)[1];
+  x[0] = u.x; x[1] = u.y; x[2] = v.x; x[3] = v.y;
+}
+__device__ __forceinline__ void ilu_st4(double *p, const double x[4])
+{
+  reinterpret_cast<double2 *>(p)[0] = make_double2(x[0], x[1]);
+  reinterpret_cast<double2 *>(p)[1] = make_double2(x[2], x[3]);
+}
+__device__ __forceinline__ void ilu_st4(float *p, const float x[4])
+{
+  *reinterpret_cast<float4 *>(p) = make_float4(x[0], x[1], x[2], x[3]);
+}
+__device__ __forceinline__ void ilu_st4(uint16_t *p, const uint16_t x[4])
+{
+  *reinterpret_cast<uint2 *>(p) = make_uint2(x[0] | (uint32_t)x[1] << 16, x[2] | (uint32_t)x[3] << 16);
+}
+
+template <typename T, bool EXACT, typename TS>
+__global__ __launch_bounds__(64 * ILU_GMAX, sizeof(T) == 8 ? 2 : 4)
 void k_ilu_rows(kf_dv d, const uint32_t *__restrict__ rec, uint32_t nrows, uint32_t *ticket, uint32_t base, uint32_t B,
                 uint32_t nnzb, T *apub, typename sentinel<T>::bits snt, T *a, T *lold, const uint32_t *__restrict__ ldiag,
                 const uint32_t *__restrict__ moff, const uint32_t *__restrict__ mjm, const uint16_t *__restrict__ mlo,
-                uint32_t maxrow, uint32_t maxlow, uint32_t maxmatch)
+                uint32_t maxrow, uint32_t maxlow, uint32_t maxmatch, ilu_out out)
 {
+  /* values per lane and staging round: one round covers the 45 (EXACT) or 38
+   * blocks of a lattice row */
+  constexpr int QB = EXACT ? 12 : 10;
   extern __shared__ __align__(16) unsigned char ilu_lds_all[];
   __shared__ ilu_ring ring;
   const ilu_layout lay(maxrow, maxlow, maxmatch, sizeof(T), EXACT);
@@ -464,19 +510,19 @@ void k_ilu_rows(kf_dv d, const uint32_t *__restrict__ rec, uint32_t nrows, uint3
     if (lane < 8) slo[mcnt + lane] = 0;
     if (lane == 0) smoff[nlow] = mcnt;
     wave_lds_sync();
-    /* the published blocks, ILU_QB values per lane per round (a lane past the
+    /* the published blocks, QB values per lane per round (a lane past the
      * end reads the last block and drops it); a value still holding the
      * sentinel is loaded again.  While the first round is on its way the
      * row's own blocks go to LDS. */
     const uint32_t tot = 16 * nsrc;
-    for (uint32_t b0 = 0; b0 == 0 || b0 < tot; b0 += 64 * ILU_QB) {
-      uint32_t need = 0, blk[ILU_QB];
-      T v[ILU_QB];
+    for (uint32_t b0 = 0; b0 == 0 || b0 < tot; b0 += 64 * QB) {
+      uint32_t need = 0, blk[QB];
+      T v[QB];
       if (tot) {
 #pragma unroll
-        for (int q = 0; q < ILU_QB; q++) blk[q] = ssrc[min(b0 / 16 + grp + 4 * q, nsrc - 1)];
+        for (int q = 0; q < QB; q++) blk[q] = ssrc[min(b0 / 16 + grp + 4 * q, nsrc - 1)];
 #pragma unroll
-        for (int q = 0; q < ILU_QB; q++) {
+        for (int q = 0; q < QB; q++) {
           v[q] = ld_coherent(apub + 16 * (size_t)blk[q] + e);
           if (b0 + lane + 64 * q < tot) need |= 1u << q;
         }
@@ -513,7 +559,7 @@ void k_ilu_rows(kf_dv d, const uint32_t *__restrict__ rec, uint32_t nrows, uint3
       }
       for (uint32_t n = 0;; n++) {
 #pragma unroll
-        for (int q = 0; q < ILU_QB; q++)
+        for (int q = 0; q < QB; q++)
           if ((need & (1u << q)) && sentinel<T>::raw(v[q]) != snt) {
             stage[b0 + lane + 64 * q] = v[q];
             need &= ~(1u << q);
@@ -526,7 +572,7 @@ void k_ilu_rows(kf_dv d, const uint32_t *__restrict__ rec, uint32_t nrows, uint3
         }
         for (uint32_t z = 0; z < d.spin_sleep; z++) __builtin_amdgcn_s_sleep(1);
 #pragma unroll
-        for (int q = 0; q < ILU_QB; q++)
+        for (int q = 0; q < QB; q++)
           if (need & (1u << q)) v[q] = ld_coherent(apub + 16 * (size_t)blk[q] + e);
       }
     }
@@ -638,11 +684,47 @@ void k_ilu_rows(kf_dv d, const uint32_t *__restrict__ rec, uint32_t nrows, uint3
     put();
     if (t < nrows) load_row();
     wave_lds_sync();
-    for (uint32_t k = lane; k < 16 * L; k += 64) a[16 * (size_t)j0 + k] = sa[k];
-    if (EXACT)
-      for (uint32_t k = lane; k < 16 * nlow; k += 64) lold[16 * (size_t)j0 + k] = sa[k];
+    /* the factors, a block row of 4 values per lane and store */
+    for (uint32_t k = lane; k < 4 * L; k += 64) {
+      T x[4];
+      ilu_ld4(sa + 4 * k, x);
+      ilu_st4(a + 16 * (size_t)j0 + 4 * k, x);
+      if (EXACT && k < 4 * nlow) ilu_st4(lold + 16 * (size_t)j0 + 4 * k, x);
+      TS y[4];
+#pragma unroll
+      for (int q = 0; q < 4; q++) ilu_cvt(x[q], y + q);
+      if (sizeof(TS) == 2) ilu_st4(reinterpret_cast<TS *>(out.abf) + 16 * (size_t)j0 + 4 * k, y);
+      if (out.val) {
+        /* slot p of L, slot p - nlow - 1 of U, or the diagonal */
+        const uint32_t p = k >> 2, u = p > nlow ? p - nlow - 1 : p;
+        const size_t slot = (size_t)(i >> 4) * out.K + u + (p > nlow ? (size_t)out.nslice * out.K : 0);
+        TS *o = static_cast<TS *>(out.val) + 16 * (i & 15u) + 4 * (k & 3u);
+        o += 256 * (p == nlow ? 2 * (size_t)out.nslice * out.K + (i >> 4) : slot);
+        if (p == nlow || u < out.K) ilu_st4(o, y);
+      }
+    }
     wave_lds_sync();
   }
+}
+
+/* the slots other rows read -- each row's blocks from the diagonal on, and
+ * with nu the U(i,i) after the nnzb blocks -- preset to the call's sentinel:
+ * 16 lanes per row, 16 bytes each (all of A's blocks were preset before,
+ * nearly twice the bytes) */
+template <typename T>
+__global__ __launch_bounds__(256) void k_ilu_preset(uint32_t N, const uint32_t *__restrict__ rowptr,
+                                                    const uint32_t *__restrict__ diag, uint32_t nnzb, bool nu,
+                                                    T *__restrict__ apub, typename sentinel<T>::bits snt)
+{
+  const uint32_t i = blockIdx.x * 16u + (threadIdx.x >> 4), l = threadIdx.x & 15u;
+  if (i >= N) return;
+  constexpr uint32_t V = 16 / sizeof(T);   /* values per store */
+  union { typename sentinel<T>::bits b[V]; uint4 q; } w;
+#pragma unroll
+  for (uint32_t k = 0; k < V; k++) w.b[k] = snt;
+  const size_t j = 16 * (size_t)diag[i], n = 16 * (size_t)rowptr[i + 1] - j;
+  for (size_t k = V * l; k < n; k += 16 * V) *reinterpret_cast<uint4 *>(apub + j + k) = w.q;
+  if (nu && V * l < 16) *reinterpret_cast<uint4 *>(apub + 16 * ((size_t)nnzb + i) + V * l) = w.q;
 }
 
 static uint32_t persistent_waves(uint32_t work, uint32_t cap)
@@ -650,8 +732,9 @@ static uint32_t persistent_waves(uint32_t work, uint32_t cap)
   return work < cap ? (work ? work : 1) : cap;
 }
 
-template <typename T, bool EXACT>
-static void launch_ilu(kf_ctx *c, T *a, T *lold, T *ud)
+/* true: the planned kernel ran, and wrote what `out` asks for */
+template <typename T, bool EXACT, typename TS>
+static bool launch_ilu(kf_ctx *c, T *a, T *lold, T *ud, const ilu_out &out)
 {
   /* the context's setting, else what fits the registers: 2048 waves in FP64
    * (221 VGPRs, two per SIMD; capped at three the exact sweep spills and
@@ -680,18 +763,20 @@ static void launch_ilu(kf_ctx *c, T *a, T *lold, T *ud)
     }
     const typename sentinel<T>::bits snt = sentinel<T>::of(++c->icall);
     T *apub = (T *)c->ilu_apub;
-    hipLaunchKernelGGL((k_fill_bits<T>), dim3(kf_blocks_for(na, 256)), dim3(256), 0, c->stream, apub, na, snt);
+    hipLaunchKernelGGL(k_ilu_preset<T>, dim3(kf_blocks_for(c->d.N, 16)), dim3(256), 0, c->stream, c->d.N, c->d.rowptr,
+                       c->d.diag, (uint32_t)c->nnzb, EXACT, apub, snt);
     KF_LAUNCH_CHECK();
     if (G * (size_t)lay.bytes > 64 * 1024)
-      KF_CHECK(hipFuncSetAttribute((const void *)k_ilu_rows<T, EXACT>, hipFuncAttributeMaxDynamicSharedMemorySize,
+      KF_CHECK(hipFuncSetAttribute((const void *)k_ilu_rows<T, EXACT, TS>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                    (int)(G * lay.bytes)));
     const int s = kf_prof_begin(c, KP_ILU);
-    hipLaunchKernelGGL((k_ilu_rows<T, EXACT>), dim3(nb), dim3(64 * G), G * lay.bytes, c->stream, c->d, c->ilu_rec,
+    hipLaunchKernelGGL((k_ilu_rows<T, EXACT, TS>), dim3(nb), dim3(64 * G), G * lay.bytes, c->stream, c->d, c->ilu_rec,
                        c->d.N, c->ticket + 2, c->ticket_base[2], G, (uint32_t)c->nnzb, apub, snt, a, lold, c->ilu_ldiag,
-                       c->ilu_moff, c->ilu_mjm, c->ilu_mlo, c->ilu_maxrow, c->ilu_maxlow, c->ilu_maxmatch);
+                       c->ilu_moff, c->ilu_mjm, c->ilu_mlo, c->ilu_maxrow, c->ilu_maxlow, c->ilu_maxmatch, out);
     KF_LAUNCH_CHECK();
     kf_prof_end(c, s);
     c->ticket_base[2] += kf_ticket_advance_ring(c->d.N, nb, G);
+    return true;
   } else {
     const uint32_t epoch = ++c->epoch;
     const int s = kf_prof_begin(c, KP_ILU);
@@ -700,6 +785,7 @@ static void launch_ilu(kf_ctx *c, T *a, T *lold, T *ud)
     KF_LAUNCH_CHECK();
     kf_prof_end(c, s);
     c->ticket_base[2] += c->d.N + nw;
+    return false;
   }
 }
 
@@ -716,29 +802,34 @@ __global__ __launch_bounds__(256) void k_to_bf16(size_t n, const float *__restri
 
 void kf_launch_ilu(kf_ctx *c)
 {
-  c->jsl_fresh = 0;   /* the Jacobi sweeps' sliced copy is now stale */
   if (c->maxrow > ILU_MAXROW) {
     fprintf(stderr, "kf: ILU supports at most %d blocks per row (mesh has %u)\n", ILU_MAXROW, c->maxrow);
     abort();
   }
+  const size_t n = 16 * c->nnzb;
+  if (c->opt.prec == KF_PREC_BF16 && !c->abf) KF_CHECK(hipMalloc((void **)&c->abf, n * sizeof(uint16_t)));
+  ilu_out out = {c->abf, NULL, 0, 0};
+  if (c->opt.jacobi_sweeps > 0) out.val = kf_jac_slices(c, &out.K, &out.nslice);
+  bool wrote;
   if (c->opt.prec == KF_PREC_FP64) {
     if (c->opt.ilu_exact) {
       if (!c->lold) {
-        KF_CHECK(hipMalloc((void **)&c->lold, 16 * c->nnzb * sizeof(double)));
-        KF_CHECK(hipMemset(c->lold, 0, 16 * c->nnzb * sizeof(double)));
+        KF_CHECK(hipMalloc((void **)&c->lold, n * sizeof(double)));
+        KF_CHECK(hipMemset(c->lold, 0, n * sizeof(double)));
         KF_CHECK(hipMalloc((void **)&c->ud, 16 * (size_t)c->d.N * sizeof(double)));
       }
-      launch_ilu<double, true>(c, c->a64, c->lold, c->ud);
+      wrote = launch_ilu<double, true, double>(c, c->a64, c->lold, c->ud, out);
     } else {
-      launch_ilu<double, false>(c, c->a64, NULL, NULL);
+      wrote = launch_ilu<double, false, double>(c, c->a64, NULL, NULL, out);
     }
+  } else if (c->opt.prec == KF_PREC_FP32) {
+    wrote = launch_ilu<float, false, float>(c, c->a32, NULL, NULL, out);
   } else {
-    launch_ilu<float, false>(c, c->a32, NULL, NULL);
-    if (c->opt.prec == KF_PREC_BF16) {
-      const size_t n = 16 * c->nnzb;
-      if (!c->abf) KF_CHECK(hipMalloc((void **)&c->abf, n * sizeof(uint16_t)));
+    wrote = launch_ilu<float, false, uint16_t>(c, c->a32, NULL, NULL, out);
+    if (!wrote) {
       hipLaunchKernelGGL(k_to_bf16, dim3(kf_blocks_for(n, 256)), dim3(256), 0, c->stream, n, c->a32, c->abf);
       KF_LAUNCH_CHECK();
     }
   }
+  c->jsl_fresh = wrote && out.val;   /* else the sweeps pack the copy when they need it */
 }

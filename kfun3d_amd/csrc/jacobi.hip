@@ -193,8 +193,8 @@ __global__ __launch_bounds__(JAC_WG) void k_jac_upper(uint32_t N, const uint32_t
  * the CSR kernels' to the bit.  Entries past slot K (rows longer than K,
  * none on a lattice) are read from the CSR array.  K is the most held
  * entries of the triangular solves (7, or 8 when a row has more than 7 on a
- * side).  Packed after each factorisation, on the first sweep that needs
- * it. */
+ * side).  The factorisation writes it while jacobi_sweeps is set; else it is
+ * packed by the first sweep that needs it (k_jac_pack). */
 template <typename TM, typename TV>
 __device__ __forceinline__ void jld4(const TM *p, TV m[4])
 {
@@ -567,8 +567,6 @@ static void jacobi_solve_sl(kf_ctx *c, const TM *a, const TB *b, double *x, TV *
   kf_prof_end(c, s);
 }
 
-/* the sliced copy of the current factors, packed now unless the last
- * factorisation's is already there (kf_launch_ilu marks it stale) */
 template <typename TM>
 static void jsl_pack_as(kf_ctx *c, const TM *a, uint32_t nslice)
 {
@@ -583,33 +581,53 @@ static void jsl_pack_as(kf_ctx *c, const TM *a, uint32_t nslice)
   KF_LAUNCH_CHECK();
 }
 
-static jsl_view jsl_pack(kf_ctx *c)
+static void jsl_pack_now(kf_ctx *c, uint32_t nslice)
 {
-  const uint32_t nslice = (c->d.N + 15) / 16;
+  if (c->jsl_esize == 8) jsl_pack_as<double>(c, c->a64, nslice);
+  else if (c->jsl_esize == 4) jsl_pack_as<float>(c, c->a32, nslice);
+  else jsl_pack_as<uint16_t>(c, c->abf, nslice);
+}
+
+/* the sliced copy's memory in the context's precision.  A new one is packed
+ * from whatever the factor array holds: that writes the columns and the
+ * zeros of the empty slots, which the factorisation leaves alone when it
+ * writes the copy itself (ilu.hip). */
+void *kf_jac_slices(kf_ctx *c, uint32_t *K, uint32_t *nslice)
+{
+  const uint32_t ns = (c->d.N + 15) / 16;
   const size_t es = c->opt.prec == KF_PREC_FP64 ? 8 : c->opt.prec == KF_PREC_FP32 ? 4 : 2;
   c->jsl_k = c->trsv_pf;   /* 7 or 8 */
-  const size_t nk = (size_t)nslice * c->jsl_k;
+  const size_t nk = (size_t)ns * c->jsl_k;
   if (c->jsl_val && c->jsl_esize != es) {   /* the precision changed */
     KF_CHECK(hipStreamSynchronize(c->stream));
     KF_CHECK(hipFree(c->jsl_val));
     c->jsl_val = NULL;
   }
+  if (!c->jsl_col) KF_CHECK(hipMalloc((void **)&c->jsl_col, 2 * nk * 16 * sizeof(uint32_t)));
   if (!c->jsl_val) {
-    KF_CHECK(hipMalloc(&c->jsl_val, (2 * nk + nslice) * 256 * es));
+    KF_CHECK(hipMalloc(&c->jsl_val, (2 * nk + ns) * 256 * es));
     c->jsl_esize = es;
     c->jsl_fresh = 0;
+    jsl_pack_now(c, ns);
   }
-  if (!c->jsl_col) KF_CHECK(hipMalloc((void **)&c->jsl_col, 2 * nk * 16 * sizeof(uint32_t)));
+  *K = c->jsl_k;
+  *nslice = ns;
+  return c->jsl_val;
+}
+
+/* the sliced copy of the current factors, packed now unless the last
+ * factorisation wrote it */
+static jsl_view jsl_pack(kf_ctx *c)
+{
+  uint32_t K, nslice;
+  jsl_view v;
+  v.val = kf_jac_slices(c, &K, &nslice);
+  v.nslice = nslice;
+  v.col = c->jsl_col;
   if (!c->jsl_fresh) {
-    if (es == 8) jsl_pack_as<double>(c, c->a64, nslice);
-    else if (es == 4) jsl_pack_as<float>(c, c->a32, nslice);
-    else jsl_pack_as<uint16_t>(c, c->abf, nslice);
+    jsl_pack_now(c, nslice);
     c->jsl_fresh = 1;
   }
-  jsl_view v;
-  v.nslice = nslice;
-  v.val = c->jsl_val;
-  v.col = c->jsl_col;
   return v;
 }
 

@@ -258,6 +258,9 @@ void kf_launch_jacobi(kf_ctx *c, const double *b, double *x);
 /* the multilevel preconditioner's fine solve: the sweeps on t (FP64 with FP64
  * factors, else FP32), then x += P z_c fused into the last sweep */
 void kf_launch_jacobi_ml(kf_ctx *c, const void *t, double *x, const uint32_t *agg, const double *zc);
+/* the sweeps' sliced copy of the factors (jacobi.hip): its memory, slots per
+ * row and side, slices of 16 rows */
+void *kf_jac_slices(kf_ctx *c, uint32_t *K, uint32_t *nslice);
 /* at context creation, with the context's device current: the device
  * address of kf_sptrsv_jacobi_noalloc's fixed work array (jacobi.hip) */
 void kf_noalloc_setup(kf_ctx *c);
