@@ -200,6 +200,7 @@ extern "C" void kf_ctx_create(GEOMETRY *g, const kf_prep *p, const kf_options *o
   d.sell_wy = dupload(wy, ne);
   d.sell_wz = dupload(wz, ne);
   free(sptr); free(deg); free(nbr); free(ent); free(blk); free(wx); free(wy); free(wz);
+  kf_sell_records(c, ne);
   kf_grad_setup(c);
   kf_phase("LSQ moments (device)");
 
@@ -315,7 +316,7 @@ extern "C" void kf_ctx_destroy(GEOMETRY *g)
     KF_CHECK(hipStreamDestroy(c->fstream));
   }
   kf_dv &d = c->d;
-  void *ptrs[] = {d.en, d.egeo, d.x, d.y, d.z, d.xyzw, d.sell_ptr, d.deg, d.sell_nbr, d.sell_ent,
+  void *ptrs[] = {d.en, d.egeo, d.sell_geo, d.x, d.y, d.z, d.xyzw, d.sell_ptr, d.deg, d.sell_nbr, d.sell_ent,
                   d.sell_blk, d.sell_wx, d.sell_wy, d.sell_wz, d.lsq, d.sell_nbs, d.sf0, d.sf1, d.sf2, d.color, d.sfptr, d.sfent, d.snx, d.sny,
                   d.snz, d.snptr, d.snent, d.fnx, d.fny, d.fnz, d.fnptr, d.fnent, d.rowptr, d.col, d.diag, d.eres,
                   d.red, d.scal, d.err, c->lrows, c->rdone,
@@ -596,7 +597,6 @@ extern "C" void ComputeA(GEOMETRY *g)
 {
   kf_ctx *c = kf_ctx_of(g);
   kf_launch_fill(c);
-  if (c->opt.bsr_operator) kf_keep_jacobian(c);   /* the ILU factors the fill's array in place */
 }
 
 /* y = A x with the Jacobian of the last ComputeA (kept when bsr_operator is

@@ -183,31 +183,97 @@ __device__ __forceinline__ void freestream_block(T xn, T yn, T zn, T U, T V, T p
   v[15] = ln * (wb * unbw + unb * wbw + zn * pbw);
 }
 
+/* Blocks are stored by the whole wavefront through its own LDS: each lane
+ * puts its block into its row (padded by 16 bytes, which say what to store
+ * and keep the rows apart in the banks), then 8 lanes together store one
+ * 128-byte line.  A lane storing its whole block by itself made 64 write
+ * requests of 16 bytes an instruction, and those, 29 million at 496K
+ * vertices, were what the kernel waited for.  An FP32 block is half a line,
+ * and lines written in halves go to memory at 2.5 TB/s: a block waits in its
+ * row for the other half of its line, which is the next incidence's wherever
+ * edges ascend with their ends. */
 template <typename T>
-__device__ __forceinline__ void store_block(T *__restrict__ a, uint32_t blk, const T v[16]);
+struct fill_rows {
+  static constexpr int PC = sizeof(T), STRIDE = 9;   /* 16-byte pieces of a block, of a row */
+  float4 w[64 * STRIDE];
+};
 
-template <>
-__device__ __forceinline__ void store_block<double>(double *__restrict__ a, uint32_t blk, const double v[16])
+#define FILL_NONE 0xffffffffu
+
+/* the rows' lines: line in units of 128 bytes, FILL_NONE for no line, and the
+ * halves that are there */
+template <typename T>
+__device__ __forceinline__ void store_lines(fill_rows<T> &rows, T *__restrict__ a, T *__restrict__ keep, uint32_t line,
+                                            uint32_t halves)
 {
-  double2 *o = reinterpret_cast<double2 *>(a + 16 * (size_t)blk);
+  constexpr int STRIDE = fill_rows<T>::STRIDE;
+  const uint32_t lane = threadIdx.x & 63u, piece = lane & 7u;
+  float4 *o = rows.w + lane * STRIDE + 8;
+  o->x = __uint_as_float(line);
+  o->y = __uint_as_float(halves);
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   /* the wavefront's own rows: in order, no barrier */
+  __builtin_amdgcn_wave_barrier();
+#pragma unroll
+  for (int i = 0; i < 8; i++) {
+    const float4 *in = rows.w + (i * 8 + lane / 8) * STRIDE;
+    const float4 val = in[piece];
+    const float2 w = *reinterpret_cast<const float2 *>(in + 8);
+    const uint32_t n = __float_as_uint(w.x);
+    if (n != FILL_NONE && (__float_as_uint(w.y) >> (piece >> 2) & 1u)) {
+      reinterpret_cast<float4 *>(a + (128 / sizeof(T)) * (size_t)n)[piece] = val;
+      if (keep) reinterpret_cast<float4 *>(keep + (128 / sizeof(T)) * (size_t)n)[piece] = val;
+    }
+  }
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+/* FP64: a block is a line */
+__device__ __forceinline__ void store_blocks(fill_rows<double> &rows, double *__restrict__ a,
+                                             double *__restrict__ keep, uint32_t blk, const double v[16], uint32_t &,
+                                             uint32_t &)
+{
+  double2 *o = reinterpret_cast<double2 *>(rows.w + (threadIdx.x & 63u) * fill_rows<double>::STRIDE);
 #pragma unroll
   for (int k = 0; k < 8; k++) o[k] = make_double2(v[2 * k], v[2 * k + 1]);
+  store_lines<double>(rows, a, keep, blk, 3u);
 }
 
-template <>
-__device__ __forceinline__ void store_block<float>(float *__restrict__ a, uint32_t blk, const float v[16])
+/* FP32: line, halves: what waits in the lane's row */
+__device__ __forceinline__ void store_blocks(fill_rows<float> &rows, float *__restrict__ a, float *__restrict__ keep,
+                                             uint32_t blk, const float v[16], uint32_t &line, uint32_t &halves)
 {
-  float4 *o = reinterpret_cast<float4 *>(a + 16 * (size_t)blk);
+  const bool other = blk != FILL_NONE && line != blk >> 1;   /* also when nothing waits */
+  store_lines<float>(rows, a, keep, other ? line : FILL_NONE, halves);
+  if (other) { line = blk >> 1; halves = 0u; }
+  if (blk != FILL_NONE) {
+    float4 *o = rows.w + (threadIdx.x & 63u) * fill_rows<float>::STRIDE + 4 * (blk & 1u);
 #pragma unroll
-  for (int k = 0; k < 4; k++) o[k] = make_float4(v[4 * k], v[4 * k + 1], v[4 * k + 2], v[4 * k + 3]);
+    for (int k = 0; k < 4; k++) o[k] = make_float4(v[4 * k], v[4 * k + 1], v[4 * k + 2], v[4 * k + 3]);
+    halves |= 1u << (blk & 1u);
+  }
 }
 
+/* Bound by memory: the records of the incidences once (36 bytes each, dense)
+ * and the blocks once, at the rate of a copy.  173x61x47 (496K vertices), FP32
+ * with the kept copy: 0.303 ms, 4.4 TB/s (0.379 ms and a copy of 0.126 ms with
+ * lanes storing their own blocks and gathered edge records; 0.374 ms with
+ * lines in halves); 144x48x48 FP64: 0.327 -> 0.190 ms.  More or fewer
+ * wavefronts (2 to 4 a SIMD) make no difference.
+ * keep: a second copy of the matrix, or NULL; a copy afterwards reads back
+ * what was just written */
 template <typename T>
 __global__ __launch_bounds__(128) void k_fill(kf_dv d, const double *__restrict__ q, const double *__restrict__ cdt,
-                                              T *__restrict__ a)
+                                              T *__restrict__ a, T *__restrict__ keep)
 {
-  const uint32_t r = kf_xcd_block() * 128u + threadIdx.x;
-  if (r >= d.N) return;
+  __shared__ fill_rows<T> srows[2];
+  fill_rows<T> &rows = srows[threadIdx.x >> 6];
+  const uint32_t t = kf_xcd_block() * 128u + threadIdx.x;
+  const uint32_t slice = __builtin_amdgcn_readfirstlane(t >> 6);
+  if (slice >= d.nslice) return;
+  const uint32_t base = d.sell_ptr[slice], width = d.sell_ptr[slice + 1] - base;
+  /* lanes behind the last row go along with no incidence */
+  const uint32_t r = min(t, d.N - 1), deg = t < d.N ? d.deg[r] : 0u;
   const T zero = T(0), mone = T(-1);
   T dg[16];
 #pragma unroll
@@ -216,37 +282,63 @@ __global__ __launch_bounds__(128) void k_fill(kf_dv d, const double *__restrict_
   dg[0] += cd; dg[5] += cd; dg[10] += cd; dg[15] += cd;
   const double *qr = q + 4 * (size_t)r;
   const T ur = (T)qr[1], vr = (T)qr[2], wr = (T)qr[3];
-  const uint32_t deg = d.deg[r];
-  size_t idx = (size_t)d.sell_ptr[r >> 6] * 64u + (r & 63u);
-  for (uint32_t k = 0; k < deg; k++, idx += 64) {
-    const uint32_t ent = d.sell_ent[idx], e = ent >> 1, nb = d.sell_nbr[idx];
-    const double *qn = q + 4 * (size_t)nb;
-    const T un = (T)qn[1], vn = (T)qn[2], wn = (T)qn[3];
-    T v0[16], v1[16], off[16];
-    const kf_egeo eg = kf_edge_geo(d.egeo, e);
-    if (ent & 1u) {   /* r is n1: (n1,n0) -= v0, (n1,n1) -= v1 */
-      edge_blocks<T>((T)eg.xn, (T)eg.yn, (T)eg.zn, (T)eg.ln, un, vn, wn, ur, vr, wr, v0, v1);
-#pragma unroll
-      for (int j = 0; j < 16; j++) { off[j] = zero + mone * v0[j]; dg[j] += mone * v1[j]; }
-    } else {          /* r is n0: (n0,n0) += v0, (n0,n1) += v1 */
-      edge_blocks<T>((T)eg.xn, (T)eg.yn, (T)eg.zn, (T)eg.ln, ur, vr, wr, un, vn, wn, v0, v1);
-#pragma unroll
-      for (int j = 0; j < 16; j++) { off[j] = zero + v1[j]; dg[j] += v0[j]; }
+  /* The next incidence is loaded before this one is stored: loads behind
+   * stores come back behind them, since one counter waits for both. */
+  size_t idx = (size_t)base * 64u + (t & 63u);
+  uint32_t nbs = 0, nbs1 = 0, blk1 = 0;   /* this incidence's, the next one's */
+  uint32_t line = FILL_NONE, halves = 0;
+  double qn[3];
+  kf_egeo eg;
+  if (width) {
+    nbs = d.sell_nbs[idx];
+    nbs1 = d.sell_nbs[width > 1 ? idx + 64 : idx];
+    blk1 = d.sell_blk[idx];
+    eg = kf_edge_geo(d.sell_geo, idx);
+    const double *p = q + 4 * (size_t)(nbs & 0x7fffffffu);
+    qn[0] = p[1]; qn[1] = p[2]; qn[2] = p[3];
+  }
+  for (uint32_t k = 0; k < width; k++, idx += 64) {
+    T off[16];
+    const T un = (T)qn[0], vn = (T)qn[1], wn = (T)qn[2];
+    const T xn = (T)eg.xn, yn = (T)eg.yn, zn = (T)eg.zn, ln = (T)eg.ln;
+    const bool side1 = nbs >> 31;
+    const uint32_t blk = k < deg ? blk1 : FILL_NONE;
+    if (k + 1 < width) {
+      const double *p = q + 4 * (size_t)(nbs1 & 0x7fffffffu);
+      qn[0] = p[1]; qn[1] = p[2]; qn[2] = p[3];
+      eg = kf_edge_geo(d.sell_geo, idx + 64);
+      nbs = nbs1;
+      blk1 = d.sell_blk[idx + 64];
+      nbs1 = d.sell_nbs[k + 2 < width ? idx + 128 : idx + 64];
     }
-    store_block<T>(a, d.sell_blk[idx], off);
-  }
-  for (uint32_t s = d.snptr[r]; s < d.snptr[r + 1]; s++) {   /* matrix/matrix.cpp:282-296 */
-    const uint32_t i = d.snent[s];
-    dg[4] += (T)d.snx[i]; dg[8] += (T)d.sny[i]; dg[12] += (T)d.snz[i];
-  }
-  for (uint32_t s = d.fnptr[r]; s < d.fnptr[r + 1]; s++) {
-    const uint32_t i = d.fnent[s];
-    T v[16];
-    freestream_block<T>((T)d.fnx[i], (T)d.fny[i], (T)d.fnz[i], (T)d.U, (T)d.V, (T)qr[0], ur, vr, wr, v);
+    if (k < deg) {
+      /* r is n1: (n1,n0) -= v0, (n1,n1) -= v1; r is n0: (n0,n0) += v0, (n0,n1) += v1 */
+      T v0[16], v1[16];
+      edge_blocks<T>(xn, yn, zn, ln, side1 ? un : ur, side1 ? vn : vr, side1 ? wn : wr, side1 ? ur : un,
+                     side1 ? vr : vn, side1 ? wr : wn, v0, v1);
 #pragma unroll
-    for (int j = 0; j < 16; j++) dg[j] += v[j];
+      for (int j = 0; j < 16; j++) {
+        off[j] = zero + (side1 ? mone * v0[j] : v1[j]);
+        dg[j] += side1 ? mone * v1[j] : v0[j];
+      }
+    }
+    store_blocks(rows, a, keep, blk, off, line, halves);
   }
-  store_block<T>(a, d.diag[r], dg);
+  if (t < d.N) {
+    for (uint32_t s = d.snptr[r]; s < d.snptr[r + 1]; s++) {   /* matrix/matrix.cpp:282-296 */
+      const uint32_t i = d.snent[s];
+      dg[4] += (T)d.snx[i]; dg[8] += (T)d.sny[i]; dg[12] += (T)d.snz[i];
+    }
+    for (uint32_t s = d.fnptr[r]; s < d.fnptr[r + 1]; s++) {
+      const uint32_t i = d.fnent[s];
+      T v[16];
+      freestream_block<T>((T)d.fnx[i], (T)d.fny[i], (T)d.fnz[i], (T)d.U, (T)d.V, (T)qr[0], ur, vr, wr, v);
+#pragma unroll
+      for (int j = 0; j < 16; j++) dg[j] += v[j];
+    }
+  }
+  store_blocks(rows, a, keep, t < d.N ? d.diag[r] : FILL_NONE, dg, line, halves);
+  if (sizeof(T) == 4) store_lines<T>(rows, a, keep, line, halves);
 }
 
 static void ensure_f32(kf_ctx *c)
@@ -254,15 +346,36 @@ static void ensure_f32(kf_ctx *c)
   if (!c->a32) KF_CHECK(hipMalloc((void **)&c->a32, 16 * c->nnzb * sizeof(float)));
 }
 
+/* the copy of the assembled Jacobian that the BSR operator reads (the ILU
+ * factors the fill's array in place): room for it in the fill's precision */
+static void ensure_kept(kf_ctx *c, bool f64)
+{
+  const size_t n = 16 * c->nnzb;
+  if (f64 ? c->jop32 != NULL : c->jop64 != NULL) {
+    /* the precision changed: drop the other copy (its last reader is done
+     * once the stream is) */
+    KF_CHECK(hipStreamSynchronize(c->stream));
+    KF_CHECK(hipFree(f64 ? (void *)c->jop32 : (void *)c->jop64));
+    c->jop32 = NULL;
+    c->jop64 = NULL;
+  }
+  if (f64 && !c->jop64) KF_CHECK(hipMalloc((void **)&c->jop64, n * sizeof(double)));
+  if (!f64 && !c->jop32) KF_CHECK(hipMalloc((void **)&c->jop32, n * sizeof(float)));
+}
+
 void kf_launch_fill(kf_ctx *c)
 {
   const uint32_t nb = kf_blocks_for(c->d.N, 128);
+  const bool f64 = c->opt.prec == KF_PREC_FP64, keep = c->opt.bsr_operator;
+  if (keep) ensure_kept(c, f64);
   const int s = kf_prof_begin(c, KP_FILL);
-  if (c->opt.prec == KF_PREC_FP64) {
-    hipLaunchKernelGGL(k_fill<double>, dim3(nb), dim3(128), 0, c->stream, c->d, c->q, c->cdt, c->a64);
+  if (f64) {
+    hipLaunchKernelGGL(k_fill<double>, dim3(nb), dim3(128), 0, c->stream, c->d, c->q, c->cdt, c->a64,
+                       keep ? c->jop64 : (double *)NULL);
   } else {
     ensure_f32(c);
-    hipLaunchKernelGGL(k_fill<float>, dim3(nb), dim3(128), 0, c->stream, c->d, c->q, c->cdt, c->a32);
+    hipLaunchKernelGGL(k_fill<float>, dim3(nb), dim3(128), 0, c->stream, c->d, c->q, c->cdt, c->a32,
+                       keep ? c->jop32 : (float *)NULL);
   }
   KF_LAUNCH_CHECK();
   kf_prof_end(c, s);

@@ -91,8 +91,8 @@ __device__ __forceinline__ void edge_vector(const d4 &cv, const d4 &cn, bool sid
 
 /* Per-vertex moments (src/weights.c:103-366): three passes over the
  * incidences in ascending edge id, each reading only the vertex's own sums
- * of the earlier passes, then the magnitudes.  Also writes sell_nbs. */
-__global__ __launch_bounds__(256) void k_lsq_moments(kf_dv d, double *__restrict__ m, uint32_t *__restrict__ nbs)
+ * of the earlier passes, then the magnitudes. */
+__global__ __launch_bounds__(256) void k_lsq_moments(kf_dv d, double *__restrict__ m)
 {
   const uint32_t v = blockIdx.x * 256u + threadIdx.x;
   if (v >= d.N) return;
@@ -103,9 +103,7 @@ __global__ __launch_bounds__(256) void k_lsq_moments(kf_dv d, double *__restrict
   /* w00, w01, w02: src/weights.c:237-297 (r = x(nb) - x(v) from either end) */
   for (uint32_t k = 0; k < deg; k++) {
     const size_t idx = base + 64 * (size_t)k;
-    const uint32_t nb = d.sell_nbr[idx], side = d.sell_ent[idx] & 1u;
-    nbs[idx] = nb | side << 31;
-    const d4 cn = ld4(d.xyzw, nb);
+    const d4 cn = ld4(d.xyzw, d.sell_nbr[idx]);
     const double rx = cn.p - cv.p, ry = cn.u - cv.u, rz = cn.v - cv.v;
     w0 += rx * rx; w1 += rx * ry; w2 += rx * rz;
   }
@@ -194,6 +192,40 @@ __global__ __launch_bounds__(256) void k_lsq_check(kf_dv d, const double *__rest
   if (!ok) atomicOr(bad, 1u);
 }
 
+/* neighbour | side << 31 and the edge's (unit normal, area) of every
+ * incidence, in sliced-ELL order (zeros in its padding): the vertex kernels
+ * read them as dense lines, where the per-edge records are gathers of 32
+ * bytes */
+__global__ __launch_bounds__(256) void k_sell_records(kf_dv d, uint32_t *__restrict__ nbs, double *__restrict__ geo)
+{
+  const uint32_t v = blockIdx.x * 256u + threadIdx.x, slice = v >> 6;
+  if (slice >= d.nslice) return;
+  const uint32_t width = d.sell_ptr[slice + 1] - d.sell_ptr[slice], deg = v < d.N ? d.deg[v] : 0u;
+  size_t idx = (size_t)d.sell_ptr[slice] * 64u + (v & 63u);
+  for (uint32_t k = 0; k < width; k++, idx += 64) {
+    uint32_t s = 0;
+    kf_egeo eg = {0.0, 0.0, 0.0, 0.0};
+    if (k < deg) {
+      const uint32_t ent = d.sell_ent[idx];
+      eg = kf_edge_geo(d.egeo, ent >> 1);
+      s = d.sell_nbr[idx] | ent << 31;
+    }
+    nbs[idx] = s;
+    st4(geo, idx, eg.xn, eg.yn, eg.zn, eg.ln);
+  }
+}
+
+void kf_sell_records(kf_ctx *c, size_t ne)
+{
+  kf_dv &d = c->d;
+  KF_CHECK(hipMalloc((void **)&d.sell_nbs, (ne + 1) * sizeof(uint32_t)));
+  KF_CHECK(hipMalloc((void **)&d.sell_geo, (4 * ne + 4) * sizeof(double)));
+  if (!d.N) return;
+  hipLaunchKernelGGL(k_sell_records, dim3(kf_blocks_for(d.N, 256)), dim3(256), 0, c->stream, d, d.sell_nbs, d.sell_geo);
+  KF_LAUNCH_CHECK();
+  KF_CHECK(hipStreamSynchronize(c->stream));
+}
+
 /* k_grad's LSQ terms from per-vertex moments (56 bytes a vertex, and the
  * neighbour's coordinates beside its state) rather than 24 bytes per
  * incidence, once every incidence's terms are shown bit-identical to the
@@ -204,15 +236,12 @@ void kf_grad_setup(kf_ctx *c)
   const char *ev = getenv("KF_GRAD_MOMENTS");
   c->grad_mom = 0;
   if ((ev && atoi(ev) == 0) || d.N == 0 || d.N > 0x7fffffffu) return;
-  uint32_t nslice_rows;
-  KF_CHECK(hipMemcpy(&nslice_rows, d.sell_ptr + d.nslice, sizeof(uint32_t), hipMemcpyDeviceToHost));
   KF_CHECK(hipMalloc((void **)&d.lsq, 7 * (size_t)d.N * sizeof(double)));
-  KF_CHECK(hipMalloc((void **)&d.sell_nbs, (size_t)nslice_rows * 64 * sizeof(uint32_t) + sizeof(uint32_t)));
   uint32_t *bad;
   KF_CHECK(hipMalloc((void **)&bad, sizeof(uint32_t)));
   KF_CHECK(hipMemsetAsync(bad, 0, sizeof(uint32_t), c->stream));
   const dim3 gv(kf_blocks_for(d.N, 256)), b(256);
-  hipLaunchKernelGGL(k_lsq_moments, gv, b, 0, c->stream, d, d.lsq, d.sell_nbs);
+  hipLaunchKernelGGL(k_lsq_moments, gv, b, 0, c->stream, d, d.lsq);
   KF_LAUNCH_CHECK();
   hipLaunchKernelGGL(k_lsq_check, gv, b, 0, c->stream, d, (const double *)d.lsq, bad);
   KF_LAUNCH_CHECK();
@@ -222,9 +251,7 @@ void kf_grad_setup(kf_ctx *c)
   KF_CHECK(hipFree(bad));
   if (hbad) {
     KF_CHECK(hipFree(d.lsq));
-    KF_CHECK(hipFree(d.sell_nbs));
     d.lsq = NULL;
-    d.sell_nbs = NULL;
     return;
   }
   KF_CHECK(hipFree(d.sell_wx));
@@ -632,11 +659,9 @@ __global__ __launch_bounds__(256) void k_timestep(kf_dv d, const double *__restr
   size_t idx = (size_t)d.sell_ptr[v >> 6] * 64u + (v & 63u);
   const d4 qv = ld4(q, v);
   for (uint32_t k = 0; k < deg; k++, idx += 64) {
-    const uint32_t ent = d.sell_ent[idx], e = ent >> 1;
-    const d4 qn = ld4(q, d.sell_nbr[idx]);
-    const d4 qa = (ent & 1u) ? qn : qv, qb = (ent & 1u) ? qv : qn;   /* (n0, n1) */
-    const kf_egeo eg = kf_edge_geo(d.egeo, e);
-    acc = acc + spectral_term(qa, qb, eg.xn, eg.yn, eg.zn, eg.ln);
+    const d4 qn = ld4(q, d.sell_nbs[idx] & 0x7fffffffu);
+    const kf_egeo eg = kf_edge_geo(d.sell_geo, idx);
+    acc = acc + spectral_term(qv, qn, eg.xn, eg.yn, eg.zn, eg.ln);   /* the same from either end */
   }
   cdt[v] = spectral_boundary(d, v, qv, acc) / cfl;
 }

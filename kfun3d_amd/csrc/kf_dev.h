@@ -53,11 +53,11 @@
 #define KF_ERR_SPIN_LIMIT 2u
 
 /* everything a kernel reads, passed by value */
-/* an edge's (unit normal, area) record */
+/* an edge's (unit normal, area): record i of a list of them */
 struct kf_egeo { double xn, yn, zn, ln; };
-__device__ __forceinline__ kf_egeo kf_edge_geo(const double *__restrict__ egeo, uint32_t e)
+__device__ __forceinline__ kf_egeo kf_edge_geo(const double *__restrict__ geo, size_t i)
 {
-  const double2 *p = reinterpret_cast<const double2 *>(egeo + 4 * (size_t)e);
+  const double2 *p = reinterpret_cast<const double2 *>(geo + 4 * i);
   const double2 lo = p[0], hi = p[1];
   return {lo.x, lo.y, hi.x, hi.y};
 }
@@ -74,7 +74,8 @@ struct kf_dv {
   uint32_t *sell_nbr, *sell_ent, *sell_blk;
   double *sell_wx, *sell_wy, *sell_wz;   /* the LSQ terms per incidence (NULL once lsq is verified) */
   double *lsq;                  /* 7 x N: per-vertex LSQ moments w00 w01 w02 w11 w12 w22 w33 (one array each) */
-  uint32_t *sell_nbs;           /* neighbour | side << 31 per incidence (with lsq) */
+  uint32_t *sell_nbs;           /* neighbour | side << 31 per incidence */
+  double *sell_geo;             /* the edge's unit normal (x, y, z) and dual-face area per incidence */
   uint32_t *sf0, *sf1, *sf2;
   uint32_t *color, ncolor;    /* solid-face colour offsets */
   uint32_t *sfptr, *sfent;
@@ -228,6 +229,7 @@ void kf_prof_end(kf_ctx *c, int slot);
 
 /* launches (defined in the .hip files) */
 /* sr != NULL: also the time-step sums of the state q (see k_residual) */
+void kf_sell_records(kf_ctx *c, size_t ne);
 void kf_grad_setup(kf_ctx *c);
 /* fd: iJacVec's combination formed by the residual's last kernel, whose
  * state q is then fd->w (k_residual<false, true>) */
@@ -251,7 +253,6 @@ struct kf_fdb {
 void kf_launch_sptrsv(kf_ctx *c, const double *b, double *x, const kf_fdb *fd);
 /* y = A x with the kept copy of the assembled Jacobian (spmv.hip) */
 void kf_launch_spmv(kf_ctx *c, const double *x, double *y);
-void kf_keep_jacobian(kf_ctx *c);
 bool kf_trsv_capped(const kf_ctx *c);
 /* x ~ U^-1 L^-1 b by opt.jacobi_sweeps Jacobi sweeps each way (jacobi.hip) */
 void kf_launch_jacobi(kf_ctx *c, const double *b, double *x);

@@ -392,8 +392,8 @@ __global__ __launch_bounds__(MP_RB) void k_mp_edge_vectors(kf_dv d, float4 *__re
   if (v >= d.N) return;
   size_t idx = (size_t)d.sell_ptr[v >> 6] * 64u + (v & 63u);
   for (uint32_t k = 0; k < d.deg[v]; k++, idx += 64) {
-    const uint32_t ent = d.sell_ent[idx], e = ent >> 1, u = d.sell_nbr[idx];
-    const kf_egeo eg = kf_edge_geo(d.egeo, e);
+    const uint32_t ent = d.sell_ent[idx], u = d.sell_nbr[idx];
+    const kf_egeo eg = kf_edge_geo(d.sell_geo, idx);
     const double ar = (ent & 1u) ? -eg.ln : eg.ln;
     const size_t ui = (size_t)d.sell_ptr[u >> 6] * 64u + (u & 63u);
     uint32_t kr = 0;

@@ -94,26 +94,3 @@ void kf_launch_spmv(kf_ctx *c, const double *x, double *y)
   KF_LAUNCH_CHECK();
   kf_prof_end(c, s);
 }
-
-/* after a fill: the operator's copy of the assembled Jacobian (the ILU then
- * factors the fill's array in place) */
-void kf_keep_jacobian(kf_ctx *c)
-{
-  const size_t n = 16 * c->nnzb;
-  const bool f64 = c->opt.prec == KF_PREC_FP64;
-  if ((f64 && c->jop32) || (!f64 && c->jop64)) {
-    /* the precision changed: drop the other copy (its last reader is done
-     * once the stream is) */
-    KF_CHECK(hipStreamSynchronize(c->stream));
-    KF_CHECK(hipFree(f64 ? (void *)c->jop32 : (void *)c->jop64));
-    c->jop32 = f64 ? NULL : c->jop32;
-    c->jop64 = f64 ? c->jop64 : NULL;
-  }
-  if (f64) {
-    if (!c->jop64) KF_CHECK(hipMalloc((void **)&c->jop64, n * sizeof(double)));
-    KF_CHECK(hipMemcpyAsync(c->jop64, c->a64, n * sizeof(double), hipMemcpyDeviceToDevice, c->stream));
-  } else {
-    if (!c->jop32) KF_CHECK(hipMalloc((void **)&c->jop32, n * sizeof(float)));
-    KF_CHECK(hipMemcpyAsync(c->jop32, c->a32, n * sizeof(float), hipMemcpyDeviceToDevice, c->stream));
-  }
-}
