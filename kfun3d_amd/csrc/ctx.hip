@@ -200,7 +200,14 @@ extern "C" void kf_ctx_create(GEOMETRY *g, const kf_prep *p, const kf_options *o
   d.sell_wy = dupload(wy, ne);
   d.sell_wz = dupload(wz, ne);
   free(sptr); free(deg); free(nbr); free(ent); free(blk); free(wx); free(wy); free(wz);
+  {
+    uint32_t *pos = (uint32_t *)kf_xmalloc((E + 1) * sizeof(uint32_t));
+    c->neres = kf_place_edges(g, p, pos);
+    d.edge_pos = dupload(pos, E);
+    free(pos);
+  }
   kf_sell_records(c, ne);
+  kf_phase("places of the fluxes, records");
   kf_grad_setup(c);
   kf_phase("LSQ moments (device)");
 
@@ -229,7 +236,7 @@ extern "C" void kf_ctx_create(GEOMETRY *g, const kf_prep *p, const kf_options *o
   c->q = dalloc<double>(4 * N);
   c->cdt = dalloc<double>(N);
   KF_CHECK(hipMemset(c->cdt, 0, N * sizeof(double)));
-  d.eres = dalloc<double>(4 * E + 8);
+  d.eres = dalloc<double>(4 * c->neres + 8);
   d.red = dalloc<double>(2 * KF_NRED);   /* two sets of partial sums (fused MGS) */
   c->mgs_part = dalloc<double>(2 * (size_t)KF_MGS_MAXV * KF_NRED);
   c->mgs_sync = dalloc<uint32_t>(4);
@@ -316,7 +323,7 @@ extern "C" void kf_ctx_destroy(GEOMETRY *g)
     KF_CHECK(hipStreamDestroy(c->fstream));
   }
   kf_dv &d = c->d;
-  void *ptrs[] = {d.en, d.egeo, d.sell_geo, d.x, d.y, d.z, d.xyzw, d.sell_ptr, d.deg, d.sell_nbr, d.sell_ent,
+  void *ptrs[] = {d.en, d.egeo, d.edge_pos, d.sell_geo, d.sell_pos, d.x, d.y, d.z, d.xyzw, d.sell_ptr, d.deg, d.sell_nbr, d.sell_ent,
                   d.sell_blk, d.sell_wx, d.sell_wy, d.sell_wz, d.lsq, d.sell_nbs, d.sf0, d.sf1, d.sf2, d.color, d.sfptr, d.sfent, d.snx, d.sny,
                   d.snz, d.snptr, d.snent, d.fnx, d.fny, d.fnz, d.fnptr, d.fnent, d.rowptr, d.col, d.diag, d.eres,
                   d.red, d.scal, d.err, c->lrows, c->rdone,

@@ -192,25 +192,28 @@ __global__ __launch_bounds__(256) void k_lsq_check(kf_dv d, const double *__rest
   if (!ok) atomicOr(bad, 1u);
 }
 
-/* neighbour | side << 31 and the edge's (unit normal, area) of every
- * incidence, in sliced-ELL order (zeros in its padding): the vertex kernels
- * read them as dense lines, where the per-edge records are gathers of 32
- * bytes */
-__global__ __launch_bounds__(256) void k_sell_records(kf_dv d, uint32_t *__restrict__ nbs, double *__restrict__ geo)
+/* neighbour | side << 31, the edge's (unit normal, area) and the place of its
+ * flux << 1 | side of every incidence, in sliced-ELL order (zeros in its
+ * padding): the vertex kernels read them as dense lines, where the per-edge
+ * records are gathers of 32 bytes */
+__global__ __launch_bounds__(256) void k_sell_records(kf_dv d, uint32_t *__restrict__ nbs, double *__restrict__ geo,
+                                                      uint32_t *__restrict__ spos)
 {
   const uint32_t v = blockIdx.x * 256u + threadIdx.x, slice = v >> 6;
   if (slice >= d.nslice) return;
   const uint32_t width = d.sell_ptr[slice + 1] - d.sell_ptr[slice], deg = v < d.N ? d.deg[v] : 0u;
   size_t idx = (size_t)d.sell_ptr[slice] * 64u + (v & 63u);
   for (uint32_t k = 0; k < width; k++, idx += 64) {
-    uint32_t s = 0;
+    uint32_t s = 0, at = 0;
     kf_egeo eg = {0.0, 0.0, 0.0, 0.0};
     if (k < deg) {
       const uint32_t ent = d.sell_ent[idx];
       eg = kf_edge_geo(d.egeo, ent >> 1);
       s = d.sell_nbr[idx] | ent << 31;
+      at = d.edge_pos[ent >> 1] << 1 | (ent & 1u);
     }
     nbs[idx] = s;
+    spos[idx] = at;
     st4(geo, idx, eg.xn, eg.yn, eg.zn, eg.ln);
   }
 }
@@ -219,9 +222,11 @@ void kf_sell_records(kf_ctx *c, size_t ne)
 {
   kf_dv &d = c->d;
   KF_CHECK(hipMalloc((void **)&d.sell_nbs, (ne + 1) * sizeof(uint32_t)));
+  KF_CHECK(hipMalloc((void **)&d.sell_pos, (ne + 1) * sizeof(uint32_t)));
   KF_CHECK(hipMalloc((void **)&d.sell_geo, (4 * ne + 4) * sizeof(double)));
   if (!d.N) return;
-  hipLaunchKernelGGL(k_sell_records, dim3(kf_blocks_for(d.N, 256)), dim3(256), 0, c->stream, d, d.sell_nbs, d.sell_geo);
+  hipLaunchKernelGGL(k_sell_records, dim3(kf_blocks_for(d.N, 256)), dim3(256), 0, c->stream, d, d.sell_nbs, d.sell_geo,
+                     d.sell_pos);
   KF_LAUNCH_CHECK();
   KF_CHECK(hipStreamSynchronize(c->stream));
 }
@@ -332,6 +337,28 @@ __global__ __launch_bounds__(256) void k_grad(kf_dv d, const double *__restrict_
   st4(gz, v, a2[0], a2[1], a2[2], a2[3]);
 }
 
+__device__ __forceinline__ uint32_t dpp_swap(uint32_t v)   /* the other lane of the pair's */
+{
+  return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0xB1, 0xf, 0xf, true);
+}
+__device__ __forceinline__ double dpp_swap(double v)
+{
+  return __hiloint2double((int)dpp_swap((uint32_t)__double2hiint(v)), (int)dpp_swap((uint32_t)__double2loint(v)));
+}
+
+/* st4 by pairs of lanes, all lanes of the wavefront active: a store
+ * instruction writes whole records */
+__device__ __forceinline__ void st4_pair(double *__restrict__ a, uint32_t i, double p, double u, double v, double w)
+{
+  const bool odd = threadIdx.x & 1u;
+  const double s0 = dpp_swap(odd ? p : v), s1 = dpp_swap(odd ? u : w);
+  const uint32_t io = dpp_swap(i);
+  double2 *r0 = reinterpret_cast<double2 *>(a + 4 * (size_t)(odd ? io : i)) + (odd ? 1 : 0);
+  double2 *r1 = reinterpret_cast<double2 *>(a + 4 * (size_t)(odd ? i : io)) + (odd ? 1 : 0);
+  *r0 = odd ? make_double2(s0, s1) : make_double2(p, u);   /* the even lane's record */
+  *r1 = odd ? make_double2(v, w) : make_double2(s0, s1);   /* the odd lane's */
+}
+
 /* ---- Roe-type edge flux: src/flux.c:151-448, one thread per edge --------- */
 
 /* edge term of the local time step (src/timestep.c:58-101), from the states
@@ -375,7 +402,12 @@ __device__ __forceinline__ double spectral_boundary(const kf_dv &d, uint32_t v, 
  * The end points' coordinates come from the interleaved copy (one 32-byte
  * gather each instead of three; 0.507 -> 0.479 ms on the 2.65M-vertex
  * lattice).  Interleaving the gradient too (12 values per vertex) made the
- * gradient kernel's stores slower than the gathers it saved here. */
+ * gradient kernel's stores slower than the gathers it saved here.
+ * Bound by memory and by the L1's lookups (83 % of its cycles).  The fluxes go
+ * to their places in sliced-ELL order, where k_residual finds one end's share
+ * of its incidences as dense lines: its loads fall from 1.6 to 1.1 GB at
+ * 288x96x96 (0.310 -> 0.199 ms), the scattered stores here cost 0.05 ms of that
+ * (0.505 -> 0.551 ms; stored lane by lane 0.569). */
 template <bool SPECTRAL>
 __global__ __launch_bounds__(256) void k_edge_flux(kf_dv d, const double *__restrict__ q,
                                                    const double *__restrict__ gx, const double *__restrict__ gy,
@@ -462,8 +494,10 @@ __global__ __launch_bounds__(256) void k_edge_flux(kf_dv d, const double *__rest
   const double res2 = 0.5 * (fluxp2 + fluxm2 - ln * t2);
   const double res3 = 0.5 * (fluxp3 + fluxm3 - ln * t3);
   const double res4 = 0.5 * (fluxp4 + fluxm4 - ln * t4);
-  st4(eres, i, res1, res2, res3, res4);
-  if (SPECTRAL) eterm[i] = spectral_term(q0, q1, xn, yn, zn, ln);
+  const uint32_t at = d.edge_pos[i];
+  if (__ballot(1) == ~0ull) st4_pair(eres, at, res1, res2, res3, res4);
+  else st4(eres, at, res1, res2, res3, res4);
+  if (SPECTRAL) eterm[at] = spectral_term(q0, q1, xn, yn, zn, ln);
 }
 
 /* ---- slip-wall face pressure terms: src/flux.c:477-537 ------------------- */
@@ -567,7 +601,7 @@ __global__ __launch_bounds__(256) void k_residual(kf_dv d, const double *__restr
     double et[RC];
 #pragma unroll
     for (uint32_t i = 0; i < RC; i++)
-      if (k0 + i < deg) ent[i] = d.sell_ent[idx0 + 64u * (k0 + i)];
+      if (k0 + i < deg) ent[i] = d.sell_pos[idx0 + 64u * (k0 + i)];
 #pragma unroll
     for (uint32_t i = 0; i < RC; i++)
       if (k0 + i < deg) {
@@ -623,7 +657,7 @@ void kf_launch_flux(kf_ctx *c, const double *q, double *gx, double *gy, double *
   KF_LAUNCH_CHECK();
   kf_prof_end(c, s);
   s = kf_prof_begin(c, KP_EDGE);
-  if (sr && !c->eterm) KF_CHECK(hipMalloc((void **)&c->eterm, (size_t)d.E * sizeof(double)));
+  if (sr && !c->eterm) KF_CHECK(hipMalloc((void **)&c->eterm, (c->neres + 1) * sizeof(double)));
   if (sr) hipLaunchKernelGGL(k_edge_flux<true>, ge, b, 0, c->stream, d, q, gx, gy, gz, d.eres, c->eterm);
   else hipLaunchKernelGGL(k_edge_flux<false>, ge, b, 0, c->stream, d, q, gx, gy, gz, d.eres, (double *)NULL);
   KF_LAUNCH_CHECK();

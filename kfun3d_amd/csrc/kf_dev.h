@@ -76,6 +76,7 @@ struct kf_dv {
   double *lsq;                  /* 7 x N: per-vertex LSQ moments w00 w01 w02 w11 w12 w22 w33 (one array each) */
   uint32_t *sell_nbs;           /* neighbour | side << 31 per incidence */
   double *sell_geo;             /* the edge's unit normal (x, y, z) and dual-face area per incidence */
+  uint32_t *edge_pos, *sell_pos;   /* place of an edge's flux in eres; the same << 1 | side per incidence */
   uint32_t *sf0, *sf1, *sf2;
   uint32_t *color, ncolor;    /* solid-face colour offsets */
   uint32_t *sfptr, *sfent;
@@ -84,7 +85,7 @@ struct kf_dv {
   double *fnx, *fny, *fnz;
   uint32_t *fnptr, *fnent;
   uint32_t *rowptr, *col, *diag;
-  double *eres;
+  double *eres;                 /* 4 doubles an edge, at its place (and scratch between two evaluations) */
   double *red, *scal;
   uint32_t *err;
 };
@@ -181,6 +182,7 @@ struct kf_ctx {
   size_t jsl_esize;         /* bytes per packed value */
   uint32_t jsl_k;           /* slots per row and side */
   int jsl_fresh;            /* 1: packed from the current factors */
+  size_t neres;             /* places in eres and eterm */
   double *eterm, *sr;       /* per-edge time-step terms, per-vertex time-step sums */
   /* forces overlapped with the next pseudo-time step (kf_forces_async) */
   hipStream_t fstream;      /* default priority, like the main stream */

@@ -88,6 +88,9 @@ typedef struct kf_sell {
 void kf_build_sell(const GEOMETRY *g, const kf_prep *p, kf_sell *out);
 /* the device's per-edge records: (n0, n1) pairs and (unit normal, area) */
 void kf_edge_records(const GEOMETRY *g, uint32_t *en, double *egeo);
+/* pos[e]: where edge e's flux is kept, in sliced-ELL order of lists of which
+ * each edge is in one of its ends'; returns the places, padding included */
+size_t kf_place_edges(const GEOMETRY *g, const kf_prep *p, uint32_t *pos);
 
 /* .msh reader (src/mesh.c:22-154 without the device part) */
 void kf_read_msh(const char *fpath, GEOMETRY *g);

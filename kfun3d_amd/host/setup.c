@@ -537,6 +537,67 @@ void kf_build_sell(const GEOMETRY *g, const kf_prep *p, kf_sell *out)
   out->wx = wx; out->wy = wy; out->wz = wz;
 }
 
+/* own[e]: the side whose end has edge e.  deg: how many each vertex then has.
+ * Returns the entries of the sliced lists. */
+static size_t edge_slots(size_t N, size_t E, const uint32_t *n0, const uint32_t *n1, const unsigned char *own,
+                         uint32_t *deg)
+{
+  memset(deg, 0, N * sizeof(uint32_t));
+  for (size_t e = 0; e < E; e++) deg[own[e] ? n1[e] : n0[e]]++;
+  size_t rows = 0;
+  for (size_t s = 0; s < N; s += 64) {
+    uint32_t l = 0;
+    for (size_t v = s; v < N && v < s + 64; v++)
+      if (deg[v] > l) l = deg[v];
+    rows += l;
+  }
+  return rows * 64;
+}
+
+/* The edges' places, by one of the two ends: its n0, or the end that has fewer
+ * edges so far where that fills the slices better (on a lattice numbered along
+ * its axes every vertex is the n0 of as many edges as the next; on other
+ * numberings one is the n0 of none of its edges, the next of all). */
+size_t kf_place_edges(const GEOMETRY *g, const kf_prep *p, uint32_t *pos)
+{
+  const size_t N = p->N, E = g->e->sz;
+  const uint32_t *n0 = g->e->eptr->n0, *n1 = g->e->eptr->n1;
+  const size_t nslice = (N + 63) / 64;
+  unsigned char *own = (unsigned char *)kf_xcalloc(E + 1, 1);
+  uint32_t *deg = (uint32_t *)kf_xcalloc(N + 1, sizeof(uint32_t));
+  size_t n = edge_slots(N, E, n0, n1, own, deg);
+  if (8 * n > 9 * E) {
+    memset(deg, 0, N * sizeof(uint32_t));
+    for (size_t e = 0; e < E; e++) {
+      own[e] = deg[n1[e]] < deg[n0[e]];
+      deg[own[e] ? n1[e] : n0[e]]++;
+    }
+    const size_t even = edge_slots(N, E, n0, n1, own, deg);
+    if (even >= n) {
+      memset(own, 0, E);
+      edge_slots(N, E, n0, n1, own, deg);
+    } else n = even;
+  }
+  size_t row = 0;
+  for (size_t s = 0; s < nslice; s++) {
+    uint32_t l = 0;
+    for (size_t v = s * 64; v < N && v < s * 64 + 64; v++) {
+      size_t at = row * 64 + (v & 63);
+      for (uint32_t k = p->vptr[v]; k < p->vptr[v + 1]; k++) {
+        const uint32_t e = p->vent[k] >> 1;
+        if (own[e] != (p->vent[k] & 1u)) continue;
+        pos[e] = (uint32_t)at;
+        at += 64;
+      }
+      if (deg[v] > l) l = deg[v];
+    }
+    row += l;
+  }
+  free(own);
+  free(deg);
+  return n;
+}
+
 void kf_free_prep(kf_prep *p)
 {
   free(p->rowptr); free(p->col); free(p->diag); free(p->vptr); free(p->vent); free(p->vblk);
