@@ -16,6 +16,8 @@
 #include "handoff.h"
 
 #define RB 256
+#define MGS_WG (2 * RB)        /* k_mgs_res's workgroup */
+static_assert(KF_MGS_ROW == RB, "k_mgs_res folds four blocks to a workgroup");
 
 /* The fixed tree over the block's RB values: at each halving s, value t
  * becomes v[t] + v[t + s].  The levels s >= 64 pair threads of different
@@ -39,6 +41,38 @@ __device__ __forceinline__ double block_sum(double v, double *sh)
   const double r = sh[0];
   __syncthreads();   /* every thread has read sh[0] before sh is reused */
   return r;
+}
+
+/* the same tree by 16 lanes, from all RB values in LDS: lane t of a row forms
+ * the levels s >= 16 of value t by itself, the rest are shifts within the row;
+ * the sum is in the row's first lane */
+__device__ __forceinline__ double row_tree(const double *sh)
+{
+  const double *p = sh + (threadIdx.x & 15u);
+  double v[16];
+#pragma unroll
+  for (int m = 0; m < 16; m++) v[m] = p[16 * m];
+#pragma unroll
+  for (int s = 8; s > 0; s >>= 1)
+#pragma unroll
+    for (int m = 0; m < s; m++) v[m] = v[m] + v[m + s];
+  double x = v[0];
+#define KF_ROW_SHL(n) __hiloint2double(__builtin_amdgcn_mov_dpp(__double2hiint(x), 0x100 + n, 0xf, 0xf, true), \
+                                       __builtin_amdgcn_mov_dpp(__double2loint(x), 0x100 + n, 0xf, 0xf, true))
+  x = x + KF_ROW_SHL(8);
+  x = x + KF_ROW_SHL(4);
+  x = x + KF_ROW_SHL(2);
+  x = x + KF_ROW_SHL(1);
+#undef KF_ROW_SHL
+  return x;
+}
+
+__device__ __forceinline__ double lane_value(double v, int k)
+{
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_readlane((int)(b & 0xffffffffll), k);
+  const int hi = __builtin_amdgcn_readlane((int)(b >> 32), k);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
 }
 
 /* elements i, i + 1 of x: one 16-byte load when the vector is 16-byte
@@ -101,13 +135,6 @@ __global__ __launch_bounds__(RB) void k_red_final(const double *__restrict__ par
  * src/kernel.c:133-134) into an OpenMP reduction copy that starts at zero and
  * is then added to 0.  One wavefront forms 64 products at a time and adds
  * them lane by lane; every lane carries the same running sum. */
-__device__ __forceinline__ double lane_value(double v, int k)
-{
-  const long long b = __double_as_longlong(v);
-  const int lo = __builtin_amdgcn_readlane((int)(b & 0xffffffffll), k);
-  const int hi = __builtin_amdgcn_readlane((int)(b >> 32), k);
-  return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
-}
 
 __global__ __launch_bounds__(64) void k_dot_seq(size_t n, const double *__restrict__ x, const double *__restrict__ y,
                                                 double *__restrict__ out, int take_sqrt)
@@ -235,9 +262,9 @@ __device__ __forceinline__ void publish_flag(double *p, double v)
                      __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-/* A partial sum published by another workgroup of the launch: polled until
- * it no longer holds the call's sentinel (bounded; a thread that gives up
- * records KF_ERR_SPIN_LIMIT and stops waiting for the rest of the launch). */
+/* A sum published by another workgroup of the launch: polled until it no
+ * longer holds the call's sentinel (bounded; a thread that gives up records
+ * KF_ERR_SPIN_LIMIT and stops waiting for the rest of the launch). */
 __device__ __forceinline__ double poll_part(const double *p, unsigned long long s, uint32_t *err, bool &aborted,
                                             uint32_t sleep)
 {
@@ -259,9 +286,15 @@ __device__ __forceinline__ double poll_part(const double *p, unsigned long long 
  * itself, see below), w held in registers throughout (src/kernel.c:129-141
  * and the closing norm, src/kernel.c:138-141).
  *
- * The grid is k_dot_part's KF_NRED x RB threads folded two to one: thread t
- * of workgroup b plays thread t of blocks 2b and 2b + 1 (the virtual sets
- * 0 and 1), owns exactly the element pairs those threads walk (pairs
+ * The grid is k_dot_part's KF_NRED x RB threads folded four to one:
+ * workgroup b plays blocks b + RB {0, 1, 2, 3}, whose partials are just those
+ * that thread b of k_red_final adds first, so it publishes their sum, and a
+ * step's table row is RB values and not KF_NRED (every workgroup polls all of
+ * them: their traffic, and four polls after one another, bounded a step).
+ * Blocks that own no pair of a short vector have partials of +0, which leave
+ * the sums' bits, and are not launched.  Thread t of half h plays thread t of
+ * the blocks 2 h and 2 h + 1 (the virtual sets 0 and 1), owns exactly the
+ * element pairs those threads walk (pairs
  * g, g + S, g + 2S, ... with S = KF_NRED RB, and the half pair of an odd
  * length), and keeps them in registers, at most MP pairs per set.  Step k:
  *   the partials of <w, V_k> (of <w, w> after the last vector), summed per
@@ -273,9 +306,13 @@ __device__ __forceinline__ double poll_part(const double *p, unsigned long long 
  * k_dot_part / k_mgs_step / k_red_final sequence.  The update reuses the
  * V_k values the dot loaded: from registers (HOLDV), else from LDS for the
  * first NL slots and from memory again for the rest; w is read once and
- * written once. */
+ * written once.
+ * Bound by a step's hand-off: a sum's way to memory and back.  About 15
+ * vectors a call, as a solve makes them: 12K vertices 80 -> 43 us, 332K
+ * 99 -> 81 us (two sets a workgroup, 1024 values to a row, twelve barriers a
+ * step and V_k loaded in the step: before). */
 template <int MP, bool HOLDV>
-__global__ __launch_bounds__(RB, 2) void k_mgs_res(size_t n, int nv, const double *__restrict__ vbase, size_t vstride,
+__global__ __launch_bounds__(MGS_WG, 2) void k_mgs_res(size_t n, int nv, const double *__restrict__ vbase, size_t vstride,
                                                    double *__restrict__ w, double *__restrict__ hslot, double *part,
                                                    unsigned long long sent, uint32_t *err, uint32_t sleep, int unit,
                                                    uint32_t *sync, int force_abort, double *part_next,
@@ -284,10 +321,13 @@ __global__ __launch_bounds__(RB, 2) void k_mgs_res(size_t n, int nv, const doubl
                                                    const double *__restrict__ qstate, double *__restrict__ wpert)
 {
   /* without HOLDV the first NL slots of V_k are kept in LDS between the dot
-   * and the update (72 KB for NL = 9: two workgroups still fit a CU) */
+   * and the update (144 KB for NL = 9: one workgroup to a CU) */
   constexpr int NL = HOLDV ? 0 : (MP < 9 ? MP : 9);
-  __shared__ double sh[RB];
-  __shared__ double2 vl[2][NL > 0 ? NL : 1][RB];
+  /* two barriers a step: the sets' values (dsh) are read before the one
+   * behind the polled sums (psh), and these before the next step's first */
+  __shared__ double dsh[4][RB], psh[RB];
+  __shared__ double2 vl[2][NL > 0 ? NL : 1][NL > 0 ? MGS_WG : 1];
+  const uint32_t t = threadIdx.x % RB, upper = threadIdx.x / RB;
   /* np = q S + r: every virtual thread owns pairs m < q, those with g < r
    * also pair q, and the thread g == r the half pair of an odd length.
    * Every lane walks MP >= q + (r > 0) pair slots without branching: a slot
@@ -302,11 +342,11 @@ __global__ __launch_bounds__(RB, 2) void k_mgs_res(size_t n, int nv, const doubl
    * per-step kernels); on go block 0 leaves hslot[nv + 1] = 0. */
   /* The tables alternate between calls: the other one (last used by the
    * previous launch, which has finished) is made ready for the next call --
-   * every workgroup presets its own two columns of it, block 0 its arrival
-   * words -- so no separate preset launch is needed. */
-  if (threadIdx.x < 2 * KF_MGS_MAXV)
-    part_next[(size_t)(threadIdx.x >> 1) * KF_NRED + 2 * blockIdx.x + (threadIdx.x & 1)] =
-        sentinel<double>::val(sent_next);
+   * every workgroup presets columns of it, block 0 its arrival words -- so no
+   * separate preset launch is needed. */
+  if (threadIdx.x < KF_MGS_MAXV)
+    for (uint32_t col = blockIdx.x; col < RB; col += gridDim.x)
+      part_next[(size_t)threadIdx.x * RB + col] = sentinel<double>::val(sent_next);
   if (blockIdx.x == 0 && threadIdx.x < 2) sync_next[threadIdx.x] = 0;
   __shared__ uint32_t decision;
   if (threadIdx.x == 0) {
@@ -345,13 +385,31 @@ __global__ __launch_bounds__(RB, 2) void k_mgs_res(size_t n, int nv, const doubl
   double wr[2][MP][2], wt[2] = {0.0, 0.0};
 #pragma unroll
   for (int v = 0; v < 2; v++) {
-    const uint32_t g = (2 * blockIdx.x + v) * RB + threadIdx.x;
+    const uint32_t g = (blockIdx.x + RB * (2 * upper + v)) * RB + t;
     ext[v] = g < r;
     tail[v] = (n & 1) && g == r;
     voff[v] = 16u * g;
   }
   /* whether set v owns slot m, and the slot's byte offset: a uniform base
    * plus one 32-bit per-lane offset */
+  /* the four blocks' partials, a row of lanes of the first wavefront each, and
+   * their sum as k_red_final's thread forms it */
+#define KF_PUBLISH(k)                                                                                      \
+  do {                                                                                                     \
+    __syncthreads();                                                                                       \
+    if (threadIdx.x < 64) {                                                                                \
+      const double x = row_tree(dsh[threadIdx.x >> 4]);                                                    \
+      double s = 0.0;                                                                                      \
+      for (int b = 0; b < 4; b++) s += canon(lane_value(x, 16 * b));                                       \
+      if (threadIdx.x == 0) st_coherent(part + (size_t)(k) * RB + blockIdx.x, canon(s));                   \
+    }                                                                                                      \
+  } while (0)
+  /* the sum over the table's row, by every wavefront */
+#define KF_COLLECT(k, h)                                                                                   \
+  if (!upper)                                                                                             \
+    psh[t] = t < gridDim.x ? poll_part(part + (size_t)(k) * RB + t, sent, err, aborted, sleep) : 0.0;      \
+  __syncthreads();                                                                                         \
+  const double h = lane_value(row_tree(psh), 0)
 #define KF_ON(m, v) ((m) < q || ((m) == q && ext[v]))
 #define KF_PAIR(x, m, v)                                                                                   \
   (*reinterpret_cast<const double2 *>(reinterpret_cast<const char *>(x) +                                  \
@@ -368,6 +426,20 @@ __global__ __launch_bounds__(RB, 2) void k_mgs_res(size_t n, int nv, const doubl
   }
   bool aborted = false;
   double nrm2 = 0.0;
+  /* HOLDV: V_k's pairs, and the next vector's, which are loaded while the
+   * step waits for the other workgroups' sums (3 us a step, 1 of them a load) */
+  double vr[2][HOLDV ? MP : 1][2], vn[2][HOLDV ? MP : 1][2];
+  double vt[2] = {0.0, 0.0}, vtn[2] = {0.0, 0.0};
+#define KF_LOAD_NEXT(u)                                                                                    \
+  _Pragma("unroll") for (int v = 0; v < 2; v++) {                                                          \
+    _Pragma("unroll") for (int m = 0; m < MP; m++) {                                                       \
+      const double2 t2 = KF_PAIR(u, m, v);                                                                 \
+      vn[v][HOLDV ? m : 0][0] = t2.x;                                                                      \
+      vn[v][HOLDV ? m : 0][1] = t2.y;                                                                      \
+    }                                                                                                      \
+    if (tail[v]) vtn[v] = (u)[n - 1];                                                                      \
+  }
+  if (HOLDV && nv > 0) KF_LOAD_NEXT(vbase);
   for (int k = 0; k <= nv; k++) {
     /* the offsets pass through an empty asm each step, so the pair
      * addresses are formed where they are used instead of being kept in
@@ -375,8 +447,17 @@ __global__ __launch_bounds__(RB, 2) void k_mgs_res(size_t n, int nv, const doubl
     asm volatile("" : "+v"(voff[0]), "+v"(voff[1]));
     const bool self = k == nv;
     const double *u = vbase + (size_t)k * vstride;
-    double vr[2][HOLDV ? MP : 1][2];
-    double vt[2] = {0.0, 0.0};
+    if (HOLDV) {
+#pragma unroll
+      for (int v = 0; v < 2; v++) {
+#pragma unroll
+        for (int m = 0; m < MP; m++) {
+          vr[v][HOLDV ? m : 0][0] = vn[v][HOLDV ? m : 0][0];
+          vr[v][HOLDV ? m : 0][1] = vn[v][HOLDV ? m : 0][1];
+        }
+        vt[v] = vtn[v];
+      }
+    }
 #pragma unroll
     for (int v = 0; v < 2; v++) {
       double acc = 0.0;
@@ -388,6 +469,14 @@ __global__ __launch_bounds__(RB, 2) void k_mgs_res(size_t n, int nv, const doubl
           acc += KF_ON(m, v) ? p1 : 0.0;
         }
         if (tail[v]) acc += wt[v] * wt[v];
+      } else if (HOLDV) {
+#pragma unroll
+        for (int m = 0; m < MP; m++) {
+          const double p0 = wr[v][m][0] * vr[v][HOLDV ? m : 0][0], p1 = wr[v][m][1] * vr[v][HOLDV ? m : 0][1];
+          acc += KF_ON(m, v) ? p0 : 0.0;
+          acc += KF_ON(m, v) ? p1 : 0.0;
+        }
+        if (tail[v]) acc += wt[v] * vt[v];
       } else {
         /* chunks of four pairs: a chunk's loads are in flight together */
 #pragma unroll
@@ -407,29 +496,22 @@ __global__ __launch_bounds__(RB, 2) void k_mgs_res(size_t n, int nv, const doubl
               const double p0 = wr[v][m][0] * uu[j][0], p1 = wr[v][m][1] * uu[j][1];
               acc += KF_ON(m, v) ? p0 : 0.0;
               acc += KF_ON(m, v) ? p1 : 0.0;
-              if (HOLDV) {
-                vr[v][HOLDV ? m : 0][0] = uu[j][0];
-                vr[v][HOLDV ? m : 0][1] = uu[j][1];
-              } else if (m < NL) {
-                vl[v][m < NL ? m : 0][threadIdx.x] = make_double2(uu[j][0], uu[j][1]);
-              }
+              if (m < NL) vl[v][m < NL ? m : 0][threadIdx.x] = make_double2(uu[j][0], uu[j][1]);
             }
           }
-          if (!HOLDV) __builtin_amdgcn_sched_barrier(0);   /* one chunk's loads live at a time */
+          __builtin_amdgcn_sched_barrier(0);   /* one chunk's loads live at a time */
         }
         if (tail[v]) {
           vt[v] = u[n - 1];
           acc += wt[v] * vt[v];
         }
       }
-      const double s = block_sum(acc, sh);
-      if (threadIdx.x == 0) st_coherent(part + (size_t)k * KF_NRED + 2 * blockIdx.x + v, canon(s));
+      dsh[2 * upper + v][t] = acc;
     }
-    /* h_k (or |w|^2) from row k, in k_red_final's tree */
-    double acc = 0.0;
-    for (int j = threadIdx.x; j < KF_NRED; j += RB)
-      acc += poll_part(part + (size_t)k * KF_NRED + j, sent, err, aborted, sleep);
-    const double h = block_sum(acc, sh);
+    KF_PUBLISH(k);
+    if (HOLDV && k + 1 < nv) KF_LOAD_NEXT(u + vstride);
+    /* h_k (or |w|^2) from row k, in k_red_final's tree, by every wavefront */
+    KF_COLLECT(k, h);
     /* whether any thread of this workgroup gave up a wait (its h_k hold a
      * placeholder then); uniform: self is the same for every thread */
     const int gaveup = self ? __syncthreads_or(aborted ? 1 : 0) : 0;
@@ -511,13 +593,10 @@ __global__ __launch_bounds__(RB, 2) void k_mgs_res(size_t n, int nv, const doubl
         acc += KF_ON(m, v) ? p1 : 0.0;
       }
       if (tail[v]) acc += wt[v] * wt[v];
-      const double s = block_sum(acc, sh);
-      if (threadIdx.x == 0) st_coherent(part + (size_t)(nv + 1) * KF_NRED + 2 * blockIdx.x + v, canon(s));
+      dsh[2 * upper + v][t] = acc;
     }
-    double acc = 0.0;
-    for (int j = threadIdx.x; j < KF_NRED; j += RB)
-      acc += poll_part(part + (size_t)(nv + 1) * KF_NRED + j, sent, err, aborted, sleep);
-    const double h = block_sum(acc, sh);
+    KF_PUBLISH(nv + 1);
+    KF_COLLECT(nv + 1, h);
     const double xn = sqrt(h);
     if (blockIdx.x == 0 && threadIdx.x == 0) *xnorm_out = xn;
     /* wpert: the next iJacVec's perturbed state, as k_fd_perturb forms it:
@@ -567,6 +646,9 @@ __global__ __launch_bounds__(RB, 2) void k_mgs_res(size_t n, int nv, const doubl
   }
 #undef KF_PAIR
 #undef KF_ON
+#undef KF_PUBLISH
+#undef KF_COLLECT
+#undef KF_LOAD_NEXT
 }
 
 /* a partial table preset to a call's sentinel, and its arrival counter and
@@ -598,7 +680,7 @@ static const void *mgs_kernel(int i)
 }
 
 /* One launch of k_mgs_res when w and the basis are 16-byte aligned, the
- * pairs fit a variant and the occupancy of its KF_NRED / 2 workgroups allows
+ * pairs fit a variant and the occupancy of its RB workgroups allows
  * them all on this device at once; false (nothing launched) otherwise.  The
  * launch is an ordinary one -- co-residency is checked by the kernel itself,
  * which writes the abort flag to scal[slot + nv + 1] -- because a
@@ -618,16 +700,16 @@ static bool mgs_resident(kf_ctx *c, size_t n, const double *vbase, size_t stride
     int nb = 0, dev = 0, ncu = 0;
     KF_CHECK(hipGetDevice(&dev));
     KF_CHECK(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
-    KF_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, fn, RB, 0));
-    c->mgs_ok[vi] = ((size_t)nb * (size_t)ncu >= KF_NRED / 2) ? 1 : 0;
+    KF_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, fn, MGS_WG, 0));
+    c->mgs_ok[vi] = ((size_t)nb * (size_t)ncu >= RB) ? 1 : 0;
   }
   if (!c->mgs_ok[vi]) return false;
   /* this call's table and arrival words (preset by the previous launch, or
    * at set-up for the first), and the other parity's, for the next call */
   const uint64_t k = c->mcall;
   const unsigned long long sent = sentinel<double>::of(k), sent_next = sentinel<double>::of(k + 1);
-  double *part = c->mgs_part + (k & 1) * (size_t)KF_MGS_MAXV * KF_NRED;
-  double *part_next = c->mgs_part + ((k + 1) & 1) * (size_t)KF_MGS_MAXV * KF_NRED;
+  double *part = c->mgs_part + (k & 1) * (size_t)KF_MGS_MAXV * RB;
+  double *part_next = c->mgs_part + ((k + 1) & 1) * (size_t)KF_MGS_MAXV * RB;
   uint32_t *sync = c->mgs_sync + 2 * (k & 1), *sync_next = c->mgs_sync + 2 * ((k + 1) & 1);
   double *hslot = c->d.scal + slot;
   uint32_t *err = c->d.err;
@@ -639,10 +721,13 @@ static bool mgs_resident(kf_ctx *c, size_t n, const double *vbase, size_t stride
                                         nothing written) or 2 (a wait expired: the values are not valid) */
   const double *qstate = c->q;
   if (!xnorm_out || n != 4 * (size_t)c->d.N || !aligned16(wpert)) wpert = NULL;   /* needs the norm round */
+  /* of k_dot_part's blocks 0 .. RB - 1 those that own a pair (or the half pair) */
+  const size_t na = (np + (n & 1) + RB - 1) / RB;
+  const uint32_t nwg = na < RB ? (uint32_t)na : RB;
   void *args[] = {&n,   &nv,    &vbase, &stride, &w,           &hslot,     &part,      (void *)&sent,
                   &err, &sleep, &unit,  &sync,   (void *)&force_abort, &part_next, (void *)&sent_next, &sync_next,
                   &xnorm_out, &hhost, &fd_h, &qstate, &wpert};
-  KF_CHECK(hipLaunchKernel(fn, dim3(KF_NRED / 2), dim3(RB), args, 0, c->stream));
+  KF_CHECK(hipLaunchKernel(fn, dim3(nwg), dim3(MGS_WG), args, 0, c->stream));
   c->mcall++;
   return true;
 }
@@ -650,7 +735,7 @@ static bool mgs_resident(kf_ctx *c, size_t n, const double *vbase, size_t stride
 /* the first resident launch's table and arrival words (call 0, parity 0) */
 void kf_mgs_setup(kf_ctx *c)
 {
-  const size_t rows = (size_t)KF_MGS_MAXV * KF_NRED;
+  const size_t rows = (size_t)KF_MGS_MAXV * RB;
   hipLaunchKernelGGL(k_mgs_preset, dim3(kf_blocks_for(rows, RB)), dim3(RB), 0, c->stream, c->mgs_part, rows,
                      sentinel<double>::of(0), c->mgs_sync);
   KF_LAUNCH_CHECK();

@@ -238,7 +238,7 @@ extern "C" void kf_ctx_create(GEOMETRY *g, const kf_prep *p, const kf_options *o
   KF_CHECK(hipMemset(c->cdt, 0, N * sizeof(double)));
   d.eres = dalloc<double>(4 * c->neres + 8);
   d.red = dalloc<double>(2 * KF_NRED);   /* two sets of partial sums (fused MGS) */
-  c->mgs_part = dalloc<double>(2 * (size_t)KF_MGS_MAXV * KF_NRED);
+  c->mgs_part = dalloc<double>(2 * (size_t)KF_MGS_MAXV * KF_MGS_ROW);
   c->mgs_sync = dalloc<uint32_t>(4);
   c->mgs_res = (ev = getenv("KF_MGS_RESIDENT")) ? atoi(ev) : 1;
   if (c->mgs_res == 2) c->mgs_res = 1;

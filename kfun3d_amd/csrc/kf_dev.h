@@ -43,6 +43,7 @@
 #define KF_NRED 1024          /* partial sums of a deterministic reduction */
 #define KF_NSCAL 256          /* device scalar slots */
 #define KF_MGS_MAXV 64        /* basis vectors + 1 of one resident MGS launch, at most */
+#define KF_MGS_ROW (KF_NRED / 4)   /* its workgroups at most, and sums to a row of its table */
 #define KF_MGS_ARRIVE 4096    /* polls a resident MGS workgroup waits for the others to arrive */
 #define KF_GROUP 16           /* rows per triangular-solve group */
 #define KF_SLOT_FASYNC (KF_NSCAL - 6)   /* scalar slots of the overlapped forces (3) */
@@ -147,7 +148,7 @@ struct kf_ctx {
   uint64_t tcall;           /* triangular solves so far (sentinel numbering) */
   /* modified Gram-Schmidt with w resident in registers (one launch per
    * orthogonalisation): per-step partial sums handed over through sentinel
-   * slots, two tables (by call parity) of KF_MGS_MAXV rows of KF_NRED */
+   * slots, two tables (by call parity) of KF_MGS_MAXV rows of KF_MGS_ROW */
   double *mgs_part;
   uint64_t mcall;            /* resident MGS launches so far (sentinel numbering) */
   uint32_t *mgs_sync;        /* per parity: arrival counter and go/abort decision of the launch */
