@@ -27,11 +27,11 @@
  * Kernels (a quad of lanes per block row, lane c forming component c, as
  * spmv.hip; workgroups remapped XCD by XCD):
  *   k_gather_sum   a block = the sum of listed blocks in ascending position:
- *                  A P from the fine blocks, then P^T A P from A P
+ *                  A P from the fine blocks (with its BF16 copy, with a BF16
+ *                  preconditioner), then P^T A P from A P
  *   k_restrict     coarse vector = sum of the aggregate's members, ascending
  *   k_coarse_resid t = b - (A P) z_c (FP32 where the fine solve is FP32
- *                  sweeps); k_coarse_resid_sl the same over a sliced BF16
- *                  copy of A P with a BF16 preconditioner
+ *                  sweeps)
  *   k_prolong_add  x += P z_c (with Jacobi sweeps: inside their last sweep)
  * Every sum runs in a fixed order, so the preconditioner is deterministic.
  */
@@ -47,14 +47,13 @@ struct kf_coarse {
   size_t cnnzb, nap;
   uint32_t *agg;       /* [N] aggregate of each fine vertex */
   uint32_t *mptr, *mlist;   /* members of each aggregate */
-  uint32_t *aprp, *apcol;   /* A P pattern: per fine row, its aggregates */
+  uint32_t *aprp;      /* A P pattern: where a fine row's blocks would start row by row */
+  uint32_t *appos, *apcol;      /* ... the place of each, and the aggregates by place */
   uint32_t *apgptr, *apglist;   /* fine block positions of each A P block */
-  uint32_t *gptr, *glist;   /* A P positions of each coarse block */
-  double *ap64;        /* A P values (FP64 preconditioner) ... */
+  uint32_t *gptr, *glist;   /* A P places of each coarse block */
+  double *ap64;        /* A P values by place (FP64 preconditioner) ... */
   float *ap32;         /* ... or FP32 */
-  void *apsl;          /* A P packed per 16-row slice and slot in BF16, for the
-                          remainder product with a BF16 preconditioner */
-  uint32_t *apsl_col;  /* ... the slots' aggregates */
+  uint16_t *apbf;      /* ... and in BF16, for the remainder product with a BF16 preconditioner */
   double *rc, *zc;     /* coarse right-hand side and solution, 4 nc */
   double *t;           /* the fine remainder b - A z, 4 N */
   float *t32;          /* ... in FP32, where the fine solve is FP32 sweeps */
@@ -69,27 +68,72 @@ static T *cupload(const T *h, size_t n)
   return p;
 }
 
+/* four values of a block row */
+template <typename T>
+struct cg_row { T v[4]; };
+
+__device__ __forceinline__ cg_row<float> cg_ld(const float *p)
+{
+  const float4 t = *reinterpret_cast<const float4 *>(p);
+  return {{t.x, t.y, t.z, t.w}};
+}
+__device__ __forceinline__ cg_row<double> cg_ld(const double *p)
+{
+  const double2 lo = reinterpret_cast<const double2 *>(p)[0], hi = reinterpret_cast<const double2 *>(p)[1];
+  return {{lo.x, lo.y, hi.x, hi.y}};
+}
+__device__ __forceinline__ void cg_st(float *p, const cg_row<float> &r)
+{
+  *reinterpret_cast<float4 *>(p) = make_float4(r.v[0], r.v[1], r.v[2], r.v[3]);
+}
+__device__ __forceinline__ void cg_st(double *p, const cg_row<double> &r)
+{
+  reinterpret_cast<double2 *>(p)[0] = make_double2(r.v[0], r.v[1]);
+  reinterpret_cast<double2 *>(p)[1] = make_double2(r.v[2], r.v[3]);
+}
+
+/* rounded to nearest even */
+__device__ __forceinline__ uint32_t cg_bf16(float v)
+{
+  uint32_t u = __float_as_uint(v);
+  u += 0x7FFFu + ((u >> 16) & 1u);
+  return u >> 16;
+}
+
+/* pos: where block b goes (NULL: to b); bf: the BF16 copy, or NULL.
+ * The lists' blocks are loaded GB at a time, before their sums: A P of
+ * 216x72x72 with its BF16 copy 0.36 ms (0.47 ms, and 0.34 ms for the copy,
+ * with one block at a time and a kernel of its own). */
 template <typename T>
 __global__ __launch_bounds__(CG_WG) void k_gather_sum(uint32_t nb, const uint32_t *__restrict__ gptr,
                                                     const uint32_t *__restrict__ glist, const T *__restrict__ a,
-                                                    T *__restrict__ ac)
+                                                    T *__restrict__ ac, const uint32_t *__restrict__ pos,
+                                                    uint16_t *__restrict__ bf)
 {
+  constexpr uint32_t GB = 4;
   const uint32_t b = kf_xcd_block() * (CG_WG / 4) + (threadIdx.x >> 2);
   const int c = threadIdx.x & 3;
   if (b >= nb) return;
-  T s0 = T(0), s1 = T(0), s2 = T(0), s3 = T(0);
-  for (uint32_t k = gptr[b]; k < gptr[b + 1]; k++) {
-    const T *p = a + 16 * (size_t)glist[k] + 4 * c;
-    s0 += p[0];
-    s1 += p[1];
-    s2 += p[2];
-    s3 += p[3];
+  const uint32_t k1 = gptr[b + 1];
+  const size_t at = pos ? pos[b] : b;
+  cg_row<T> s = {{T(0), T(0), T(0), T(0)}};
+  for (uint32_t k = gptr[b]; k < k1; k += GB) {
+    uint32_t j[GB];
+    cg_row<T> p[GB];
+#pragma unroll
+    for (uint32_t i = 0; i < GB; i++) j[i] = glist[min(k + i, k1 - 1u)];
+#pragma unroll
+    for (uint32_t i = 0; i < GB; i++) p[i] = cg_ld(a + 16 * (size_t)j[i] + 4 * c);
+#pragma unroll
+    for (uint32_t i = 0; i < GB; i++)
+#pragma unroll
+      for (int m = 0; m < 4; m++) s.v[m] = k + i < k1 ? s.v[m] + p[i].v[m] : s.v[m];
   }
-  T *o = ac + 16 * (size_t)b + 4 * c;
-  o[0] = s0;
-  o[1] = s1;
-  o[2] = s2;
-  o[3] = s3;
+  cg_st(ac + 16 * at + 4 * c, s);
+  if constexpr (sizeof(T) == 4)
+    if (bf)
+      *reinterpret_cast<uint2 *>(bf + 16 * at + 4 * c) =
+          make_uint2(cg_bf16(s.v[0]) | cg_bf16(s.v[1]) << 16, cg_bf16(s.v[2]) | cg_bf16(s.v[3]) << 16);
 }
 
 __global__ __launch_bounds__(CG_WG) void k_restrict(uint32_t nc, const uint32_t *__restrict__ mptr,
@@ -104,138 +148,131 @@ __global__ __launch_bounds__(CG_WG) void k_restrict(uint32_t nc, const uint32_t 
   rc[4 * (size_t)I + c] = s;
 }
 
-template <typename T>
-__device__ __forceinline__ void cg_row4(const T *a, size_t j, int c, double &a0, double &a1, double &a2, double &a3)
+/* ---- A P by places ------------------------------------------------------------
+ *
+ * A slice of 16 rows is a wavefront's: its blocks lie together, first all the
+ * rows' first blocks, then the second ones of the rows that have one, and so
+ * on, so that a load instruction reads one contiguous run and nothing is
+ * padded (a lattice row has 5 or 8 A P blocks).  A wavefront finds its rows'
+ * places by counting lanes: no index is loaded. */
+
+/* the places of row by row positions, and the aggregates by place */
+__global__ __launch_bounds__(CG_WG) void k_ap_places(uint32_t N, const uint32_t *__restrict__ aprp,
+                                                     const uint32_t *__restrict__ col, uint32_t *__restrict__ pos,
+                                                     uint32_t *__restrict__ pcol)
 {
-  const T *p = a + 16 * j + 4 * c;
-  a0 = (double)p[0];
-  a1 = (double)p[1];
-  a2 = (double)p[2];
-  a3 = (double)p[3];
+  const uint32_t r = blockIdx.x * CG_WG + threadIdx.x;
+  if (r >= N) return;
+  const uint32_t r0 = r & ~15u, r1 = min(r0 + 16u, N), j0 = aprp[r], n = aprp[r + 1] - j0;
+  for (uint32_t k = 0; k < n; k++) {
+    uint32_t at = aprp[r0];
+    for (uint32_t i = r0; i < r1; i++) {
+      const uint32_t m = aprp[i + 1] - aprp[i];
+      at += min(m, k) + (i < r && m > k ? 1u : 0u);
+    }
+    pos[j0 + k] = at;
+    pcol[at] = col[j0 + k];
+  }
+}
+
+__global__ __launch_bounds__(CG_WG) void k_ap_relist(uint32_t n, const uint32_t *__restrict__ pos,
+                                                     uint32_t *__restrict__ list)
+{
+  const uint32_t i = blockIdx.x * CG_WG + threadIdx.x;
+  if (i < n) list[i] = pos[list[i]];
+}
+
+/* a block row of A P as it is stored, and widened */
+template <typename T>
+struct cg_raw { cg_row<T> r; };
+template <>
+struct cg_raw<uint16_t> { uint2 r; };
+
+template <typename T>
+__device__ __forceinline__ void cg_ldraw(const T *p, cg_raw<T> &o) { o.r = cg_ld(p); }
+__device__ __forceinline__ void cg_ldraw(const uint16_t *p, cg_raw<uint16_t> &o)
+{
+  o.r = *reinterpret_cast<const uint2 *>(p);
+}
+template <typename T>
+__device__ __forceinline__ cg_row<double> cg_widen(const cg_raw<T> &o)
+{
+  return {{(double)o.r.v[0], (double)o.r.v[1], (double)o.r.v[2], (double)o.r.v[3]}};
+}
+__device__ __forceinline__ cg_row<double> cg_widen(const cg_raw<uint16_t> &o)
+{
+  return {{__uint_as_float(o.r.x << 16), __uint_as_float(o.r.x & 0xffff0000u), __uint_as_float(o.r.y << 16),
+           __uint_as_float(o.r.y & 0xffff0000u)}};
+}
+
+/* lane I's value in each quad of lanes */
+template <int I>
+__device__ __forceinline__ double cg_quad(double v)
+{
+  return __hiloint2double(__builtin_amdgcn_mov_dpp(__double2hiint(v), I * 0x55, 0xf, 0xf, true),
+                          __builtin_amdgcn_mov_dpp(__double2loint(v), I * 0x55, 0xf, 0xf, true));
+}
+
+#define AP_BATCH 8u   /* blocks of a row loaded together: all of them on a lattice */
+
+/* up to AP_BATCH blocks of the row's n from the k0-th on, from place base on;
+ * adds them to acc and moves base past the slice's */
+template <typename TS>
+__device__ __forceinline__ void ap_batch(const TS *__restrict__ ap, const uint32_t *__restrict__ apcol,
+                                         const double *__restrict__ zc, uint32_t &base, uint32_t k0, uint32_t n,
+                                         int c, double &acc)
+{
+  uint32_t at[AP_BATCH], kk[AP_BATCH];
+#pragma unroll
+  for (uint32_t k = 0; k < AP_BATCH; k++) {
+    const uint64_t on = __ballot(k0 + k < n);
+    const uint32_t below =
+        __builtin_amdgcn_mbcnt_hi((uint32_t)(on >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)on, 0u));
+    /* whole quads are on or off: lane c has c more below it than its row */
+    at[k] = k0 + k < n ? base + (below - (uint32_t)c) / 4u : base;
+    base += (uint32_t)__popcll(on) / 4u;
+  }
+  cg_raw<TS> a[AP_BATCH];
+  double z[AP_BATCH];   /* one component a lane */
+#pragma unroll
+  for (uint32_t k = 0; k < AP_BATCH; k++) kk[k] = apcol[at[k]];
+#pragma unroll
+  for (uint32_t k = 0; k < AP_BATCH; k++) cg_ldraw(ap + 16 * (size_t)at[k] + 4 * c, a[k]);
+#pragma unroll
+  for (uint32_t k = 0; k < AP_BATCH; k++) z[k] = zc[4 * (size_t)kk[k] + c];
+#pragma unroll
+  for (uint32_t k = 0; k < AP_BATCH; k++) {
+    const cg_row<double> w = cg_widen(a[k]);
+    double s = acc + w.v[0] * cg_quad<0>(z[k]);
+    s = s + w.v[1] * cg_quad<1>(z[k]);
+    s = s + w.v[2] * cg_quad<2>(z[k]);
+    s = s + w.v[3] * cg_quad<3>(z[k]);
+    acc = k0 + k < n ? s : acc;
+  }
 }
 
 /* t = b - (A P) z_c; per row the A P blocks in ascending aggregate, each
- * component summed a[c][0] z0 + ... + a[c][3] z3 in FP64; stored as TT
- * (float where the fine sweeps round it to FP32 on reading anyway) */
-template <typename T, typename TT>
+ * component summed a[c][0] z0 + ... + a[c][3] z3 in FP64, the row's first
+ * AP_BATCH blocks from ap1 (BF16 with a BF16 preconditioner, else ap itself),
+ * the rest from ap; stored as TT (float where the fine sweeps round it to
+ * FP32 on reading anyway).  Bound by memory: 288x96x96 in BF16 0.224 -> 0.170 ms
+ * (before: 8 padded slots a row, a quad loading each z four times over, 112
+ * VGPRs; the compact copy alone left it at 0.224). */
+template <typename TS, typename TA, typename TT>
 __global__ __launch_bounds__(CG_WG) void k_coarse_resid(uint32_t N, const uint32_t *__restrict__ aprp,
-                                                        const uint32_t *__restrict__ apcol, const T *__restrict__ ap,
+                                                        const uint32_t *__restrict__ apcol,
+                                                        const TA *__restrict__ ap, const TS *__restrict__ ap1,
                                                         const double *__restrict__ zc,
                                                         const double *__restrict__ b, TT *__restrict__ t)
 {
   const uint32_t r = kf_xcd_block() * (CG_WG / 4) + (threadIdx.x >> 2);
   const int c = threadIdx.x & 3;
   if (r >= N) return;
+  const uint32_t n = aprp[r + 1] - aprp[r];
+  uint32_t base = aprp[r & ~15u];
   double acc = 0.0;
-  for (uint32_t k = aprp[r]; k < aprp[r + 1]; k++) {
-    double a0, a1, a2, a3;
-    cg_row4<T>(ap, k, c, a0, a1, a2, a3);
-    const double *z = zc + 4 * (size_t)apcol[k];
-    acc = acc + a0 * z[0];
-    acc = acc + a1 * z[1];
-    acc = acc + a2 * z[2];
-    acc = acc + a3 * z[3];
-  }
-  const size_t o = 4 * (size_t)r + c;
-  t[o] = (TT)(b[o] - acc);
-}
-
-/* ---- A P per 16-row slice, for the remainder product ------------------------
- *
- * As the Jacobi sweeps' factors (jacobi.hip): slot k of a slice's 16 rows is
- * 16 consecutive blocks, so one load instruction of a wavefront reads one
- * contiguous run; AP_SLOTS = 8 slots a row (a lattice row has 5 or 8 A P
- * blocks), a slot past the row's end holds zeros and aggregate 0 and is
- * selected away, entries past the last slot are read from the CSR copy.
- * Used with a BF16 preconditioner only, the values rounded to nearest even
- * from the FP32 sums: padded to 8 slots, an FP32 or FP64 copy would read
- * more bytes than the CSR form (5.6 blocks a row), and measured slower. */
-#define AP_SLOTS 8
-
-__device__ __forceinline__ void cg_st(uint16_t *o, double v)
-{
-  uint32_t u = __float_as_uint((float)v);
-  u += 0x7FFFu + ((u >> 16) & 1u);
-  *o = (uint16_t)(u >> 16);
-}
-
-template <typename TS, typename TA>
-__global__ __launch_bounds__(CG_WG) void k_ap_pack(uint32_t N, const uint32_t *__restrict__ aprp,
-                                                   const uint32_t *__restrict__ apcol, const TA *__restrict__ ap,
-                                                   TS *__restrict__ sv, uint32_t *__restrict__ sc)
-{
-  const uint32_t r = kf_xcd_block() * (CG_WG / 4) + (threadIdx.x >> 2);
-  const int c = threadIdx.x & 3;
-  if (r >= N) return;
-  const uint32_t j0 = aprp[r], n = aprp[r + 1] - j0, q = r & 15u;
-  for (int k = 0; k < AP_SLOTS; k++) {
-    const size_t slot = (size_t)(r >> 4) * AP_SLOTS + k;
-    TS *o = sv + (slot * 16 + q) * 16 + 4 * c;
-    const TA *src = ap + 16 * (size_t)(j0 + k) + 4 * c;
-    for (int i = 0; i < 4; i++) cg_st(o + i, (uint32_t)k < n ? (double)src[i] : 0.0);
-    if (c == 0) sc[slot * 16 + q] = (uint32_t)k < n ? apcol[j0 + k] : 0u;
-  }
-}
-
-__device__ __forceinline__ void cg_ld4(const double *p, double a[4])
-{
-  const double2 lo = reinterpret_cast<const double2 *>(p)[0], hi = reinterpret_cast<const double2 *>(p)[1];
-  a[0] = lo.x; a[1] = lo.y; a[2] = hi.x; a[3] = hi.y;
-}
-__device__ __forceinline__ void cg_ld4(const uint16_t *p, double a[4])
-{
-  const uint2 v = *reinterpret_cast<const uint2 *>(p);
-  a[0] = __uint_as_float(v.x << 16);
-  a[1] = __uint_as_float(v.x & 0xffff0000u);
-  a[2] = __uint_as_float(v.y << 16);
-  a[3] = __uint_as_float(v.y & 0xffff0000u);
-}
-
-/* t = b - (A P) z_c over the sliced copy: per row the A P blocks in
- * ascending aggregate (its slots, then its CSR tail), each component summed
- * a[c][0] z0 + ... + a[c][3] z3 in FP64, the slots loaded in one batch;
- * stored as TT (float where the fine sweeps round it to FP32 on reading
- * anyway) */
-template <typename TS, typename TA, typename TT>
-__global__ __launch_bounds__(CG_WG) void k_coarse_resid_sl(uint32_t N, const uint32_t *__restrict__ aprp,
-                                                           const uint32_t *__restrict__ apcol,
-                                                           const TA *__restrict__ ap, const TS *__restrict__ sv,
-                                                           const uint32_t *__restrict__ sc,
-                                                           const double *__restrict__ zc,
-                                                           const double *__restrict__ b, TT *__restrict__ t)
-{
-  const uint32_t r = kf_xcd_block() * (CG_WG / 4) + (threadIdx.x >> 2);
-  const int c = threadIdx.x & 3;
-  if (r >= N) return;
-  const uint32_t j0 = aprp[r], n = aprp[r + 1] - j0, q = r & 15u;
-  const size_t base = (size_t)(r >> 4) * AP_SLOTS;
-  uint32_t kk[AP_SLOTS];
-#pragma unroll
-  for (int k = 0; k < AP_SLOTS; k++) kk[k] = sc[(base + k) * 16 + q];
-  double a[AP_SLOTS][4];
-#pragma unroll
-  for (int k = 0; k < AP_SLOTS; k++) cg_ld4(sv + ((base + k) * 16 + q) * 16 + 4 * c, a[k]);
-  double z[AP_SLOTS][4];
-#pragma unroll
-  for (int k = 0; k < AP_SLOTS; k++) cg_ld4(zc + 4 * (size_t)kk[k], z[k]);
-  double acc = 0.0;
-#pragma unroll
-  for (int k = 0; k < AP_SLOTS; k++) {
-    double s = acc + a[k][0] * z[k][0];
-    s = s + a[k][1] * z[k][1];
-    s = s + a[k][2] * z[k][2];
-    s = s + a[k][3] * z[k][3];
-    acc = (uint32_t)k < n ? s : acc;
-  }
-  for (uint32_t k = AP_SLOTS; k < n; k++) {
-    double a0, a1, a2, a3;
-    cg_row4<TA>(ap, j0 + k, c, a0, a1, a2, a3);
-    const double *zz = zc + 4 * (size_t)apcol[j0 + k];
-    acc = acc + a0 * zz[0];
-    acc = acc + a1 * zz[1];
-    acc = acc + a2 * zz[2];
-    acc = acc + a3 * zz[3];
-  }
+  ap_batch<TS>(ap1, apcol, zc, base, 0u, n, c, acc);
+  for (uint32_t k0 = AP_BATCH; __any(k0 < n); k0 += AP_BATCH) ap_batch<TA>(ap, apcol, zc, base, k0, n, c, acc);
   const size_t o = 4 * (size_t)r + c;
   t[o] = (TT)(b[o] - acc);
 }
@@ -281,11 +318,23 @@ static kf_coarse *coarse_build(kf_ctx *c)
   k->mptr = cupload(h.mptr, (size_t)k->nc + 1);
   k->mlist = cupload(h.mlist, N);
   k->aprp = cupload(h.aprp, N + 1);
-  k->apcol = cupload(h.apcol, h.nap);
+  uint32_t *col = cupload(h.apcol, h.nap);
+  /* one block more than there is, for lanes without one */
+  KF_CHECK(hipMalloc((void **)&k->appos, (h.nap + 1) * sizeof(uint32_t)));
+  KF_CHECK(hipMalloc((void **)&k->apcol, (h.nap + 1) * sizeof(uint32_t)));
+  KF_CHECK(hipMemset(k->apcol + h.nap, 0, sizeof(uint32_t)));
   k->apgptr = cupload(h.apgptr, h.nap + 1);
   k->apglist = cupload(h.apglist, nnzb);
   k->gptr = cupload(h.gptr, k->cnnzb + 1);
   k->glist = cupload(h.glist, h.nap);
+  hipLaunchKernelGGL(k_ap_places, dim3(kf_blocks_for(N, CG_WG)), dim3(CG_WG), 0, c->stream, (uint32_t)N, k->aprp, col,
+                     k->appos, k->apcol);
+  KF_LAUNCH_CHECK();
+  hipLaunchKernelGGL(k_ap_relist, dim3(kf_blocks_for(h.nap, CG_WG)), dim3(CG_WG), 0, c->stream, (uint32_t)h.nap,
+                     k->appos, k->glist);
+  KF_LAUNCH_CHECK();
+  KF_CHECK(hipStreamSynchronize(c->stream));
+  KF_CHECK(hipFree(col));
   KF_CHECK(hipMalloc((void **)&k->rc, 4 * (size_t)k->nc * sizeof(double)));
   KF_CHECK(hipMalloc((void **)&k->zc, 4 * (size_t)k->nc * sizeof(double)));
   KF_CHECK(hipMalloc((void **)&k->t, 4 * N * sizeof(double)));
@@ -293,24 +342,12 @@ static kf_coarse *coarse_build(kf_ctx *c)
   return k;
 }
 
-/* the sliced BF16 copy of A P, with a BF16 preconditioner */
-static void ap_pack(kf_ctx *c, kf_coarse *k)
-{
-  if (c->opt.prec != KF_PREC_BF16) return;
-  const uint32_t N = c->d.N, nslice = (N + 15) / 16;
-  if (!k->apsl) KF_CHECK(hipMalloc(&k->apsl, (size_t)nslice * AP_SLOTS * 256 * sizeof(uint16_t)));
-  if (!k->apsl_col) KF_CHECK(hipMalloc((void **)&k->apsl_col, (size_t)nslice * AP_SLOTS * 16 * sizeof(uint32_t)));
-  hipLaunchKernelGGL((k_ap_pack<uint16_t, float>), dim3(kf_blocks_for(N, CG_WG / 4)), dim3(CG_WG), 0, c->stream, N,
-                     k->aprp, k->apcol, (const float *)k->ap32, (uint16_t *)k->apsl, k->apsl_col);
-  KF_LAUNCH_CHECK();
-}
-
 /* P^T (A P) from A P into a coarse value array */
 template <typename T>
 static void galerkin_from_ap(kf_ctx *c, const kf_coarse *k, const T *ap, T *out)
 {
   hipLaunchKernelGGL(k_gather_sum<T>, dim3(kf_blocks_for(k->cnnzb, CG_WG / 4)), dim3(CG_WG), 0, c->stream,
-                     (uint32_t)k->cnnzb, k->gptr, k->glist, ap, out);
+                     (uint32_t)k->cnnzb, k->gptr, k->glist, ap, out, (const uint32_t *)NULL, (uint16_t *)NULL);
   KF_LAUNCH_CHECK();
 }
 
@@ -321,7 +358,7 @@ void kf_coarse_factor(kf_ctx *c)
   if (!c->coarse) c->coarse = coarse_build(c);
   kf_coarse *k = (kf_coarse *)c->coarse;
   kf_ctx *cc = k->cc;
-  const bool f64 = c->opt.prec == KF_PREC_FP64;
+  const bool f64 = c->opt.prec == KF_PREC_FP64, bf = c->opt.prec == KF_PREC_BF16;
   cc->opt.prec = c->opt.prec;   /* the coarse factors follow the fine level's precision */
   cc->opt.jacobi_sweeps = cc->opt.coarse_sweeps = c->opt.coarse_sweeps;
   if (cc->opt.coarse != c->opt.coarse - 1) {   /* the number of levels changed */
@@ -339,9 +376,9 @@ void kf_coarse_factor(kf_ctx *c)
   const int s = kf_prof_begin(c, KP_COARSE_FACTOR);
   const uint32_t nb = kf_blocks_for(k->nap, CG_WG / 4);
   if (f64) {
-    if (!k->ap64) KF_CHECK(hipMalloc((void **)&k->ap64, 16 * k->nap * sizeof(double)));
+    if (!k->ap64) KF_CHECK(hipMalloc((void **)&k->ap64, 16 * (k->nap + 1) * sizeof(double)));
     hipLaunchKernelGGL(k_gather_sum<double>, dim3(nb), dim3(CG_WG), 0, c->stream, (uint32_t)k->nap, k->apgptr,
-                       k->apglist, (const double *)c->a64, k->ap64);
+                       k->apglist, (const double *)c->a64, k->ap64, k->appos, (uint16_t *)NULL);
     KF_LAUNCH_CHECK();
     galerkin_from_ap<double>(c, k, k->ap64, cc->a64);
   } else {
@@ -349,14 +386,14 @@ void kf_coarse_factor(kf_ctx *c)
       fprintf(stderr, "kf: two-level preconditioner: no single-precision Jacobian (ComputeA must run first)\n");
       abort();
     }
-    if (!k->ap32) KF_CHECK(hipMalloc((void **)&k->ap32, 16 * k->nap * sizeof(float)));
+    if (!k->ap32) KF_CHECK(hipMalloc((void **)&k->ap32, 16 * (k->nap + 1) * sizeof(float)));
+    if (bf && !k->apbf) KF_CHECK(hipMalloc((void **)&k->apbf, 16 * (k->nap + 1) * sizeof(uint16_t)));
     if (!cc->a32) KF_CHECK(hipMalloc((void **)&cc->a32, 16 * k->cnnzb * sizeof(float)));
     hipLaunchKernelGGL(k_gather_sum<float>, dim3(nb), dim3(CG_WG), 0, c->stream, (uint32_t)k->nap, k->apgptr,
-                       k->apglist, (const float *)c->a32, k->ap32);
+                       k->apglist, (const float *)c->a32, k->ap32, k->appos, bf ? k->apbf : (uint16_t *)NULL);
     KF_LAUNCH_CHECK();
     galerkin_from_ap<float>(c, k, k->ap32, cc->a32);
   }
-  ap_pack(c, k);
   if (cc->opt.coarse) kf_coarse_factor(cc);   /* the next level, from the Galerkin values */
   kf_launch_ilu(cc);
   kf_prof_end(c, s);
@@ -371,7 +408,7 @@ void kf_coarse_apply(kf_ctx *c, const double *b, double *x)
     abort();
   }
   const bool f64 = c->opt.prec == KF_PREC_FP64, bf = c->opt.prec == KF_PREC_BF16;
-  if ((f64 ? !k->ap64 : !k->ap32) || (bf && !k->apsl)) {
+  if ((f64 ? !k->ap64 : !k->ap32) || (bf && !k->apbf)) {
     fprintf(stderr, "kf: two-level preconditioner: the preconditioner's precision changed since "
                     "ComputeNumericalILU\n");
     abort();
@@ -391,26 +428,15 @@ void kf_coarse_apply(kf_ctx *c, const double *b, double *x)
   const bool sweeps = c->opt.jacobi_sweeps > 0;
   const bool t32 = sweeps && !f64;
   if (t32 && !k->t32) KF_CHECK(hipMalloc((void **)&k->t32, n4 * sizeof(float)));
-  if (f64) {
-    hipLaunchKernelGGL((k_coarse_resid<double, double>), dim3(nb), dim3(CG_WG), 0, c->stream, d.N, k->aprp, k->apcol,
-                       (const double *)k->ap64, k->zc, b, k->t);
-  } else if (!bf) {
-    if (t32)
-      hipLaunchKernelGGL((k_coarse_resid<float, float>), dim3(nb), dim3(CG_WG), 0, c->stream, d.N, k->aprp, k->apcol,
-                         (const float *)k->ap32, k->zc, b, k->t32);
-    else
-      hipLaunchKernelGGL((k_coarse_resid<float, double>), dim3(nb), dim3(CG_WG), 0, c->stream, d.N, k->aprp, k->apcol,
-                         (const float *)k->ap32, k->zc, b, k->t);
-  } else {
-    if (t32)
-      hipLaunchKernelGGL((k_coarse_resid_sl<uint16_t, float, float>), dim3(nb), dim3(CG_WG), 0, c->stream, d.N,
-                         k->aprp, k->apcol, (const float *)k->ap32, (const uint16_t *)k->apsl, k->apsl_col, k->zc, b,
-                         k->t32);
-    else
-      hipLaunchKernelGGL((k_coarse_resid_sl<uint16_t, float, double>), dim3(nb), dim3(CG_WG), 0, c->stream, d.N,
-                         k->aprp, k->apcol, (const float *)k->ap32, (const uint16_t *)k->apsl, k->apsl_col, k->zc, b,
-                         k->t);
-  }
+#define CG_RESID(TS, TA, TT, ap, ap1, t)                                                                            \
+  hipLaunchKernelGGL((k_coarse_resid<TS, TA, TT>), dim3(nb), dim3(CG_WG), 0, c->stream, d.N, k->aprp, k->apcol,      \
+                     (const TA *)(ap), (const TS *)(ap1), k->zc, b, t)
+  if (f64) CG_RESID(double, double, double, k->ap64, k->ap64, k->t);
+  else if (bf && t32) CG_RESID(uint16_t, float, float, k->ap32, k->apbf, k->t32);
+  else if (bf) CG_RESID(uint16_t, float, double, k->ap32, k->apbf, k->t);
+  else if (t32) CG_RESID(float, float, float, k->ap32, k->ap32, k->t32);
+  else CG_RESID(float, float, double, k->ap32, k->ap32, k->t);
+#undef CG_RESID
   KF_LAUNCH_CHECK();
   kf_prof_end(c, s);
   if (sweeps) {
@@ -429,8 +455,8 @@ void kf_coarse_destroy(kf_ctx *c)
   if (!k) return;
   kf_coarse_destroy(k->cc);
   kf_ctx_destroy_matrix(k->cc);
-  void *ptrs[] = {k->agg, k->mptr, k->mlist, k->aprp, k->apcol, k->apgptr, k->apglist, k->gptr, k->glist,
-                  k->ap64, k->ap32, k->apsl, k->apsl_col, k->rc, k->zc, k->t, k->t32};
+  void *ptrs[] = {k->agg, k->mptr, k->mlist, k->aprp, k->appos, k->apcol, k->apgptr, k->apglist, k->gptr, k->glist,
+                  k->ap64, k->ap32, k->apbf, k->rc, k->zc, k->t, k->t32};
   for (size_t i = 0; i < sizeof(ptrs) / sizeof(ptrs[0]); i++)
     if (ptrs[i]) KF_CHECK(hipFree(ptrs[i]));
   delete k;
