@@ -397,56 +397,28 @@ __device__ __forceinline__ double spectral_boundary(const kf_dv &d, uint32_t v, 
   return acc;
 }
 
-/* SPECTRAL: also the edge's time-step term into eterm (the driver's first
- * residual of a pseudo-time step, whose state the time step then uses).
- * The end points' coordinates come from the interleaved copy (one 32-byte
- * gather each instead of three; 0.507 -> 0.479 ms on the 2.65M-vertex
- * lattice).  Interleaving the gradient too (12 values per vertex) made the
- * gradient kernel's stores slower than the gathers it saved here.
- * Bound by memory and by the L1's lookups (83 % of its cycles).  The fluxes go
- * to their places in sliced-ELL order, where k_residual finds one end's share
- * of its incidences as dense lines: its loads fall from 1.6 to 1.1 GB at
- * 288x96x96 (0.310 -> 0.199 ms), the scattered stores here cost 0.05 ms of that
- * (0.505 -> 0.551 ms; stored lane by lane 0.569). */
-template <bool SPECTRAL>
-__global__ __launch_bounds__(256) void k_edge_flux(kf_dv d, const double *__restrict__ q,
-                                                   const double *__restrict__ gx, const double *__restrict__ gy,
-                                                   const double *__restrict__ gz, double *__restrict__ eres,
-                                                   double *__restrict__ eterm)
+/* the state at the edge's midpoint, extrapolated from an end
+ * (src/flux.c:237-290) */
+__device__ __forceinline__ d4 extrapolate(const d4 &q, const d4 &gx, const d4 &gy, const d4 &gz, double rx, double ry,
+                                          double rz)
 {
-  const uint32_t i = kf_xcd_block() * 256u + threadIdx.x;
-  if (i >= d.E) return;
-  const uint2 nn = reinterpret_cast<const uint2 *>(d.en)[i];
-  const uint32_t node0 = nn.x, node1 = nn.y;
-  const kf_egeo eg = kf_edge_geo(d.egeo, i);
-  const double xn = eg.xn, yn = eg.yn, zn = eg.zn, ln = eg.ln;
-  const d4 c0 = ld4(d.xyzw, node0), c1 = ld4(d.xyzw, node1);
-  const double x0 = c0.p, y0 = c0.u, z0 = c0.v;
-  const double x1 = c1.p, y1 = c1.u, z1 = c1.v;
-  const double xmean = 0.5 * (x0 + x1);
-  const double ymean = 0.5 * (y0 + y1);
-  const double zmean = 0.5 * (z0 + z1);
+  d4 s;
+  s.p = q.p + gx.p * rx; s.p += gy.p * ry; s.p += gz.p * rz;
+  s.u = q.u + gx.u * rx; s.u += gy.u * ry; s.u += gz.u * rz;
+  s.v = q.v + gx.v * rx; s.v += gy.v * ry; s.v += gz.v * rz;
+  s.w = q.w + gx.w * rx; s.w += gy.w * ry; s.w += gz.w * rz;
+  return s;
+}
+
+/* an edge's flux from the states on its two sides (L: n0's) */
+__device__ __forceinline__ d4 roe_flux(const d4 &L, const d4 &R, double xn, double yn, double zn, double ln)
+{
+  const double pL = L.p, uL = L.u, vL = L.v, wL = L.w, pR = R.p, uR = R.u, vR = R.v, wR = R.w;
   double X1, Y1, Z1, X2, Y2, Z2;
   tangent_basis(xn, yn, zn, X1, Y1, Z1, X2, Y2, Z2);
-
-  const d4 q0 = ld4(q, node0), q1 = ld4(q, node1);
-  const d4 g0x = ld4(gx, node0), g0y = ld4(gy, node0), g0z = ld4(gz, node0);
-  const d4 g1x = ld4(gx, node1), g1y = ld4(gy, node1), g1z = ld4(gz, node1);
-
-  double rx = xmean - x0, ry = ymean - y0, rz = zmean - z0;
-  double pL = q0.p + g0x.p * rx; pL += g0y.p * ry; pL += g0z.p * rz;
-  double uL = q0.u + g0x.u * rx; uL += g0y.u * ry; uL += g0z.u * rz;
-  double vL = q0.v + g0x.v * rx; vL += g0y.v * ry; vL += g0z.v * rz;
-  double wL = q0.w + g0x.w * rx; wL += g0y.w * ry; wL += g0z.w * rz;
   double ubarL = xn * uL; ubarL += yn * vL; ubarL += zn * wL;
-
-  rx = xmean - x1; ry = ymean - y1; rz = zmean - z1;
-  double pR = q1.p + g1x.p * rx; pR += g1y.p * ry; pR += g1z.p * rz;
-  double uR = q1.u + g1x.u * rx; uR += g1y.u * ry; uR += g1z.u * rz;
-  double vR = q1.v + g1x.v * rx; vR += g1y.v * ry; vR += g1z.v * rz;
-  double wR = q1.w + g1x.w * rx; wR += g1y.w * ry; wR += g1z.w * rz;
   double ubarR = xn * uR; ubarR += yn * vR; ubarR += zn * wR;
-
+  d4 res;
   const double u = 0.5 * (uL + uR), v = 0.5 * (vL + vR), w = 0.5 * (wL + wR);
   double ubar = xn * u; ubar += yn * v; ubar += zn * w;
   double phi1 = xn * B_; phi1 += u * ubar;
@@ -490,14 +462,47 @@ __global__ __launch_bounds__(256) void k_edge_flux(kf_dv d, const double *__rest
   const double fluxm2 = ln * (uR * ubarR + xn * pR);
   const double fluxm3 = ln * (vR * ubarR + yn * pR);
   const double fluxm4 = ln * (wR * ubarR + zn * pR);
-  const double res1 = 0.5 * (fluxp1 + fluxm1 - ln * t1);
-  const double res2 = 0.5 * (fluxp2 + fluxm2 - ln * t2);
-  const double res3 = 0.5 * (fluxp3 + fluxm3 - ln * t3);
-  const double res4 = 0.5 * (fluxp4 + fluxm4 - ln * t4);
+  res.p = 0.5 * (fluxp1 + fluxm1 - ln * t1);
+  res.u = 0.5 * (fluxp2 + fluxm2 - ln * t2);
+  res.v = 0.5 * (fluxp3 + fluxm3 - ln * t3);
+  res.w = 0.5 * (fluxp4 + fluxm4 - ln * t4);
+  return res;
+}
+
+/* SPECTRAL: also the edge's time-step term into eterm (the driver's first
+ * residual of a pseudo-time step, whose state the time step then uses).
+ * The end points' coordinates come from the interleaved copy (one 32-byte
+ * gather each instead of three; 0.507 -> 0.479 ms on the 2.65M-vertex
+ * lattice).  Interleaving the gradient too (12 values per vertex) made the
+ * gradient kernel's stores slower than the gathers it saved here.
+ * Bound by memory and by the L1's lookups (83 % of its cycles).  The fluxes go
+ * to their places in sliced-ELL order, where k_residual finds one end's share
+ * of its incidences as dense lines: its loads fall from 1.6 to 1.1 GB at
+ * 288x96x96 (0.310 -> 0.199 ms), the scattered stores here cost 0.05 ms of that
+ * (0.505 -> 0.551 ms; stored lane by lane 0.569). */
+template <bool SPECTRAL>
+__global__ __launch_bounds__(256) void k_edge_flux(kf_dv d, const double *__restrict__ q,
+                                                   const double *__restrict__ gx, const double *__restrict__ gy,
+                                                   const double *__restrict__ gz, double *__restrict__ eres,
+                                                   double *__restrict__ eterm)
+{
+  const uint32_t i = kf_xcd_block() * 256u + threadIdx.x;
+  if (i >= d.E) return;
+  const uint2 nn = reinterpret_cast<const uint2 *>(d.en)[i];
+  const uint32_t node0 = nn.x, node1 = nn.y;
+  const kf_egeo eg = kf_edge_geo(d.egeo, i);
+  const d4 c0 = ld4(d.xyzw, node0), c1 = ld4(d.xyzw, node1);
+  const double xmean = 0.5 * (c0.p + c1.p), ymean = 0.5 * (c0.u + c1.u), zmean = 0.5 * (c0.v + c1.v);
+  const d4 q0 = ld4(q, node0), q1 = ld4(q, node1);
+  const d4 L = extrapolate(q0, ld4(gx, node0), ld4(gy, node0), ld4(gz, node0), xmean - c0.p, ymean - c0.u,
+                           zmean - c0.v);
+  const d4 R = extrapolate(q1, ld4(gx, node1), ld4(gy, node1), ld4(gz, node1), xmean - c1.p, ymean - c1.u,
+                           zmean - c1.v);
+  const d4 res = roe_flux(L, R, eg.xn, eg.yn, eg.zn, eg.ln);
   const uint32_t at = d.edge_pos[i];
-  if (__ballot(1) == ~0ull) st4_pair(eres, at, res1, res2, res3, res4);
-  else st4(eres, at, res1, res2, res3, res4);
-  if (SPECTRAL) eterm[at] = spectral_term(q0, q1, xn, yn, zn, ln);
+  if (__ballot(1) == ~0ull) st4_pair(eres, at, res.p, res.u, res.v, res.w);
+  else st4(eres, at, res.p, res.u, res.v, res.w);
+  if (SPECTRAL) eterm[at] = spectral_term(q0, q1, eg.xn, eg.yn, eg.zn, eg.ln);
 }
 
 /* ---- slip-wall face pressure terms: src/flux.c:477-537 ------------------- */
@@ -575,13 +580,44 @@ __device__ __forceinline__ void freestream_term(const kf_dv &d, uint32_t i, cons
 /* ---- per-vertex residual: edges (edge order), walls (colour order), free
  * stream, exactly the reference's order of updates to r[v] --------------- */
 
-/* SPECTRAL: also the vertex's time-step sum (edge terms in edge order, then
+/* Both kernels below:
+ * SPECTRAL: also the vertex's time-step sum (edge terms in edge order, then
  * the boundary-node terms: k_timestep's order) into sr, before the division
- * by the CFL */
-/* FD: q is iJacVec's perturbed state w, and r receives its combination
+ * by the CFL.
+ * FD: q is iJacVec's perturbed state w, and r receives its combination
  * ((R(w) - fd.r) + cdt (w - q0)) |x| / h (src/kernel.c:33-44) instead of
  * R(w): the operations of k_fd_combine on the same operands, so the same
  * bits, without R(w)'s round trip through memory */
+
+/* the free stream's terms, and what of the vertex's sums goes where */
+template <bool SPECTRAL, bool FD>
+__device__ __forceinline__ void finish_residual(const kf_dv &d, const double *__restrict__ q, uint32_t v, double r0,
+                                                double r1, double r2, double r3, double acc, double *__restrict__ r,
+                                                double *__restrict__ sr, const kf_fdb &fd)
+{
+  if (SPECTRAL) sr[v] = spectral_boundary(d, v, ld4(q, v), acc);
+  const uint32_t f0 = d.fnptr[v], f1 = d.fnptr[v + 1];
+  if (f0 < f1) {
+    const d4 qi = ld4(q, v);
+    for (uint32_t s = f0; s < f1; s++) {
+      double o[4];
+      freestream_term(d, d.fnent[s], qi, o);
+      r0 += o[0]; r1 += o[1]; r2 += o[2]; r3 += o[3];
+    }
+  }
+  if (FD) {
+    const double a = *fd.xnorm / fd.h;
+    const double cd = fd.cdt[v];
+    const d4 rb = ld4(fd.r, v), wv = ld4(q, v), q0 = ld4(fd.q0, v);
+    r0 = (r0 - rb.p + cd * (wv.p - q0.p)) * a;
+    r1 = (r1 - rb.u + cd * (wv.u - q0.u)) * a;
+    r2 = (r2 - rb.v + cd * (wv.v - q0.v)) * a;
+    r3 = (r3 - rb.w + cd * (wv.w - q0.w)) * a;
+  }
+  st4(r, v, r0, r1, r2, r3);
+}
+
+/* from the edges' fluxes in eres, one thread per vertex */
 template <bool SPECTRAL, bool FD>
 __global__ __launch_bounds__(256) void k_residual(kf_dv d, const double *__restrict__ q,
                                                   const double *__restrict__ eres, double *__restrict__ r,
@@ -616,32 +652,104 @@ __global__ __launch_bounds__(256) void k_residual(kf_dv d, const double *__restr
         if (SPECTRAL) acc = acc + et[i];
       }
   }
-  if (SPECTRAL) sr[v] = spectral_boundary(d, v, ld4(q, v), acc);
   for (uint32_t s = d.sfptr[v]; s < d.sfptr[v + 1]; s++) {
     const uint32_t ent = d.sfent[s];
     double xn, yn, zn, pc;
     wall_term(d, q, ent >> 2, ent & 3u, xn, yn, zn, pc);
     r1 += xn * pc; r2 += yn * pc; r3 += zn * pc;
   }
-  const uint32_t f0 = d.fnptr[v], f1 = d.fnptr[v + 1];
-  if (f0 < f1) {
-    const d4 qi = ld4(q, v);
-    for (uint32_t s = f0; s < f1; s++) {
-      double o[4];
-      freestream_term(d, d.fnent[s], qi, o);
-      r0 += o[0]; r1 += o[1]; r2 += o[2]; r3 += o[3];
+  finish_residual<SPECTRAL, FD>(d, q, v, r0, r1, r2, r3, acc, r, sr, fd);
+}
+
+/* a plus the values of a group of P lanes (4 or 16) in the order of the lanes */
+template <int P, int J = 0>
+__device__ __forceinline__ double group_add(double a, double v)
+{
+  if constexpr (J < P) {
+    constexpr int ctrl = P == 4 ? J * 0x55 : 0x150 + J;   /* quad_perm, row_newbcast */
+    a = a + __hiloint2double(__builtin_amdgcn_mov_dpp(__double2hiint(v), ctrl, 0xf, 0xf, true),
+                             __builtin_amdgcn_mov_dpp(__double2loint(v), ctrl, 0xf, 0xf, true));
+    return group_add<P, J + 1>(a, v);
+  }
+  return a;
+}
+
+/* The residual of a small mesh in one kernel: P lanes per vertex, a
+ * lane per incidence, whose flux it forms itself (an edge's two ends the same
+ * one: the same operands in the same order), and per wall face; the group adds
+ * them in order.  A lane without one adds +0, which leaves the bits of sums
+ * that start at +0.  Twice the arithmetic of the edge kernel, but neither its
+ * launch nor the fluxes' way through memory nor a thread's chain of faces. */
+template <int P, bool SPECTRAL, bool FD>
+__global__ __launch_bounds__(256) void k_flux_residual(kf_dv d, const double *__restrict__ q,
+                                                       const double *__restrict__ gx, const double *__restrict__ gy,
+                                                       const double *__restrict__ gz, double *__restrict__ r,
+                                                       double *__restrict__ sr, kf_fdb fd)
+{
+  const uint32_t t = kf_xcd_block() * 256u + threadIdx.x, v = t / P, l = t % P;
+  if (v >= d.N) return;   /* whole groups leave together */
+  const uint32_t deg = d.deg[v], sf0 = d.sfptr[v], sf1 = d.sfptr[v + 1];
+  const size_t base = (size_t)d.sell_ptr[v >> 6] * 64u + (v & 63u);
+  const d4 qv = ld4(q, v), cv = ld4(d.xyzw, v);
+  const d4 gvx = ld4(gx, v), gvy = ld4(gy, v), gvz = ld4(gz, v);
+  double r0 = 0.0, r1 = 0.0, r2 = 0.0, r3 = 0.0, acc = 0.0;
+  for (uint32_t k0 = 0; k0 < deg; k0 += P) {
+    const bool on = k0 + l < deg;
+    const size_t idx = base + 64 * (size_t)(on ? k0 + l : deg - 1u);
+    const uint32_t s = d.sell_nbs[idx], nb = s & 0x7fffffffu;
+    const bool side1 = s >> 31;
+    const kf_egeo eg = kf_edge_geo(d.sell_geo, idx);
+    const d4 cn = ld4(d.xyzw, nb), qn = ld4(q, nb);
+    const d4 gnx = ld4(gx, nb), gny = ld4(gy, nb), gnz = ld4(gz, nb);
+    const double xm = 0.5 * (cv.p + cn.p), ym = 0.5 * (cv.u + cn.u), zm = 0.5 * (cv.v + cn.v);
+    const d4 sv = extrapolate(qv, gvx, gvy, gvz, xm - cv.p, ym - cv.u, zm - cv.v);
+    const d4 sn = extrapolate(qn, gnx, gny, gnz, xm - cn.p, ym - cn.u, zm - cn.v);
+    const d4 L = {side1 ? sn.p : sv.p, side1 ? sn.u : sv.u, side1 ? sn.v : sv.v, side1 ? sn.w : sv.w};
+    const d4 R = {side1 ? sv.p : sn.p, side1 ? sv.u : sn.u, side1 ? sv.v : sn.v, side1 ? sv.w : sn.w};
+    d4 e = roe_flux(L, R, eg.xn, eg.yn, eg.zn, eg.ln);
+    if (side1) { e.p = -e.p; e.u = -e.u; e.v = -e.v; e.w = -e.w; }   /* n1 subtracts: r - e == r + (-e) */
+    r0 = group_add<P>(r0, on ? e.p : 0.0);
+    r1 = group_add<P>(r1, on ? e.u : 0.0);
+    r2 = group_add<P>(r2, on ? e.v : 0.0);
+    r3 = group_add<P>(r3, on ? e.w : 0.0);
+    if (SPECTRAL) {   /* the same from either end */
+      const double et = spectral_term(qv, qn, eg.xn, eg.yn, eg.zn, eg.ln);
+      acc = group_add<P>(acc, on ? et : 0.0);
     }
   }
-  if (FD) {
-    const double a = *fd.xnorm / fd.h;
-    const double cd = fd.cdt[v];
-    const d4 rb = ld4(fd.r, v), wv = ld4(q, v), q0 = ld4(fd.q0, v);
-    r0 = (r0 - rb.p + cd * (wv.p - q0.p)) * a;
-    r1 = (r1 - rb.u + cd * (wv.u - q0.u)) * a;
-    r2 = (r2 - rb.v + cd * (wv.v - q0.v)) * a;
-    r3 = (r3 - rb.w + cd * (wv.w - q0.w)) * a;
+  for (uint32_t s0 = sf0; s0 < sf1; s0 += P) {
+    const bool on = s0 + l < sf1;
+    const uint32_t ent = d.sfent[on ? s0 + l : sf1 - 1u];
+    double xn, yn, zn, pc;
+    wall_term(d, q, ent >> 2, ent & 3u, xn, yn, zn, pc);
+    r1 = group_add<P>(r1, on ? xn * pc : 0.0);
+    r2 = group_add<P>(r2, on ? yn * pc : 0.0);
+    r3 = group_add<P>(r3, on ? zn * pc : 0.0);
   }
-  st4(r, v, r0, r1, r2, r3);
+  if (l) return;
+  finish_residual<SPECTRAL, FD>(d, q, v, r0, r1, r2, r3, acc, r, sr, fd);
+}
+
+/* Meshes up to FLUX_ONE_ROWS vertices take one kernel, up to FLUX_WIDE_ROWS
+ * 16 lanes to a vertex (the 3072 wavefronts the chip holds of it), else 4.
+ * One residual (gradient, launches and all), two kernels against one:
+ * 1.6K vertices 21.8 / 17.4 us, 12K 24.0 / 19.3, 22K 28.6 / 25.0, 36K
+ * 35.2 / 33.3, 66K 44.8 / 44.7, 111K 60.3 / 68.4; 4 lanes for 16: 1.6K 20.4,
+ * 6K 22.0 for 20.0, 12K 20.0, 22K 25.0 for 26.7. */
+#define FLUX_ONE_ROWS 32768u
+#define FLUX_WIDE_ROWS 12288u
+
+template <int P>
+static void flux_residual(kf_ctx *c, const double *q, const double *gx, const double *gy, const double *gz, double *r,
+                          double *sr, const kf_fdb *fd)
+{
+  const kf_dv &d = c->d;
+  const dim3 g(kf_blocks_for(P * (size_t)d.N, 256)), b(256);
+  const kf_fdb none = {};
+  double *const no = NULL;
+  if (sr) hipLaunchKernelGGL((k_flux_residual<P, true, false>), g, b, 0, c->stream, d, q, gx, gy, gz, r, sr, none);
+  else if (fd) hipLaunchKernelGGL((k_flux_residual<P, false, true>), g, b, 0, c->stream, d, q, gx, gy, gz, r, no, *fd);
+  else hipLaunchKernelGGL((k_flux_residual<P, false, false>), g, b, 0, c->stream, d, q, gx, gy, gz, r, no, none);
 }
 
 void kf_launch_flux(kf_ctx *c, const double *q, double *gx, double *gy, double *gz, double *r, double *sr,
@@ -656,6 +764,25 @@ void kf_launch_flux(kf_ctx *c, const double *q, double *gx, double *gy, double *
   else hipLaunchKernelGGL(k_grad<false>, gv, b, 0, c->stream, d, q, gx, gy, gz, c->opt.first_order);
   KF_LAUNCH_CHECK();
   kf_prof_end(c, s);
+  if (sr && fd) {
+    fprintf(stderr, "kf: the residual with time-step sums takes no combination\n");
+    abort();
+  }
+  const kf_fdb none = {};
+  /* one kernel reads other vertices' state and gradient as it writes r: not
+   * over them */
+  const size_t n4 = 4 * (size_t)d.N;
+  bool over = false;
+  for (const double *a : {q, (const double *)gx, (const double *)gy, (const double *)gz})
+    over = over || (a < r + n4 && r < a + n4);
+  if (d.N <= FLUX_ONE_ROWS && !over) {
+    s = kf_prof_begin(c, KP_RES);
+    if (d.N <= FLUX_WIDE_ROWS) flux_residual<16>(c, q, gx, gy, gz, r, sr, fd);
+    else flux_residual<4>(c, q, gx, gy, gz, r, sr, fd);
+    KF_LAUNCH_CHECK();
+    kf_prof_end(c, s);
+    return;
+  }
   s = kf_prof_begin(c, KP_EDGE);
   if (sr && !c->eterm) KF_CHECK(hipMalloc((void **)&c->eterm, (c->neres + 1) * sizeof(double)));
   if (sr) hipLaunchKernelGGL(k_edge_flux<true>, ge, b, 0, c->stream, d, q, gx, gy, gz, d.eres, c->eterm);
@@ -663,20 +790,14 @@ void kf_launch_flux(kf_ctx *c, const double *q, double *gx, double *gy, double *
   KF_LAUNCH_CHECK();
   kf_prof_end(c, s);
   s = kf_prof_begin(c, KP_RES);
-  const kf_fdb none = {};
-  if (sr && fd) {
-    fprintf(stderr, "kf: the residual with time-step sums takes no combination\n");
-    abort();
-  }
   if (sr)
-    hipLaunchKernelGGL((k_residual<true, false>), dim3(kf_blocks_for(d.N, 256)), dim3(256), 0, c->stream, d, q,
-                       d.eres, r, c->eterm, sr, none);
+    hipLaunchKernelGGL((k_residual<true, false>), gv, b, 0, c->stream, d, q, d.eres, r, c->eterm, sr, none);
   else if (fd)
-    hipLaunchKernelGGL((k_residual<false, true>), dim3(kf_blocks_for(d.N, 256)), dim3(256), 0, c->stream, d, q,
-                       d.eres, r, (const double *)NULL, (double *)NULL, *fd);
+    hipLaunchKernelGGL((k_residual<false, true>), gv, b, 0, c->stream, d, q, d.eres, r, (const double *)NULL,
+                       (double *)NULL, *fd);
   else
-    hipLaunchKernelGGL((k_residual<false, false>), dim3(kf_blocks_for(d.N, 256)), dim3(256), 0, c->stream, d, q,
-                       d.eres, r, (const double *)NULL, (double *)NULL, none);
+    hipLaunchKernelGGL((k_residual<false, false>), gv, b, 0, c->stream, d, q, d.eres, r, (const double *)NULL,
+                       (double *)NULL, none);
   KF_LAUNCH_CHECK();
   kf_prof_end(c, s);
 }
