@@ -172,6 +172,8 @@ unsigned long long kfs_mgs_aborts(GEOMETRY *g);
 /* resident (one-launch) orthogonalisations so far on this context */
 unsigned long long kfs_mgs_launches(GEOMETRY *g);
 void kfs_fd_perturb(GEOMETRY *g, const double *x, double h, int slot, double *w);
+/* kfs_nrm2 of x (of the state's length) into the slot, then kfs_fd_perturb */
+void kfs_norm_perturb(GEOMETRY *g, const double *x, double h, int slot, double *w);
 void kfs_fd_combine(GEOMETRY *g, const double *r, const double *w, double h, int slot, double *y);
 /* ComputeFlux(w) then kfs_fd_combine in one pass (y must not alias w or r) */
 void kfs_flux_fd(GEOMETRY *g, const double *w, GRADIENT *grad, double *y, const double *r, double h, int slot);

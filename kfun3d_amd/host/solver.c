@@ -35,10 +35,9 @@
 static void ijacvec(GEOMETRY *g, const double *x, const double *r, const double norm, GRADIENT *grad, double *w,
                     double *y, int have)
 {
-  const size_t sz = g->c->sz;
-  if (have < 1) kfs_nrm2(g, sz, x, KFS_SLOT_XNORM);
   const double h = FD_EPS * norm;
-  if (have < 2) kfs_fd_perturb(g, x, h, KFS_SLOT_XNORM, w);
+  if (have < 1) kfs_norm_perturb(g, x, h, KFS_SLOT_XNORM, w);
+  else if (have < 2) kfs_fd_perturb(g, x, h, KFS_SLOT_XNORM, w);
   if (y == r || y == w) {   /* aliased output: the two passes, as before */
     ComputeFlux(g, w, grad, y);
     kfs_fd_combine(g, r, w, h, KFS_SLOT_XNORM, y);
@@ -55,10 +54,9 @@ static void ijacvec(GEOMETRY *g, const double *x, const double *r, const double 
 static void ijacvec_solve(GEOMETRY *g, const double *x, const double *r, const double norm, GRADIENT *grad,
                           double *w, double *y, int have, double *out)
 {
-  const size_t sz = g->c->sz;
-  if (have < 1) kfs_nrm2(g, sz, x, KFS_SLOT_XNORM);
   const double h = FD_EPS * norm;
-  if (have < 2) kfs_fd_perturb(g, x, h, KFS_SLOT_XNORM, w);
+  if (have < 1) kfs_norm_perturb(g, x, h, KFS_SLOT_XNORM, w);
+  else if (have < 2) kfs_fd_perturb(g, x, h, KFS_SLOT_XNORM, w);
   if (kfs_fd_residual(g)) {
     kfs_flux_fd(g, w, grad, y, r, h, KFS_SLOT_XNORM);
     ComputeSparseTriangularSolve(g, y, out);
