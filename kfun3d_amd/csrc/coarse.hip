@@ -37,7 +37,7 @@
  */
 #include <cstring>
 
-#include "kf_dev.h"
+#include "coarse_dev.h"
 
 #define CG_WG 256   /* 64 block rows per workgroup */
 
@@ -66,30 +66,6 @@ static T *cupload(const T *h, size_t n)
   KF_CHECK(hipMalloc((void **)&p, (n ? n : 1) * sizeof(T)));
   if (n) KF_CHECK(hipMemcpy(p, h, n * sizeof(T), hipMemcpyHostToDevice));
   return p;
-}
-
-/* four values of a block row */
-template <typename T>
-struct cg_row { T v[4]; };
-
-__device__ __forceinline__ cg_row<float> cg_ld(const float *p)
-{
-  const float4 t = *reinterpret_cast<const float4 *>(p);
-  return {{t.x, t.y, t.z, t.w}};
-}
-__device__ __forceinline__ cg_row<double> cg_ld(const double *p)
-{
-  const double2 lo = reinterpret_cast<const double2 *>(p)[0], hi = reinterpret_cast<const double2 *>(p)[1];
-  return {{lo.x, lo.y, hi.x, hi.y}};
-}
-__device__ __forceinline__ void cg_st(float *p, const cg_row<float> &r)
-{
-  *reinterpret_cast<float4 *>(p) = make_float4(r.v[0], r.v[1], r.v[2], r.v[3]);
-}
-__device__ __forceinline__ void cg_st(double *p, const cg_row<double> &r)
-{
-  reinterpret_cast<double2 *>(p)[0] = make_double2(r.v[0], r.v[1]);
-  reinterpret_cast<double2 *>(p)[1] = make_double2(r.v[2], r.v[3]);
 }
 
 /* rounded to nearest even */
@@ -143,9 +119,7 @@ __global__ __launch_bounds__(CG_WG) void k_restrict(uint32_t nc, const uint32_t 
   const uint32_t I = kf_xcd_block() * (CG_WG / 4) + (threadIdx.x >> 2);
   const int c = threadIdx.x & 3;
   if (I >= nc) return;
-  double s = 0.0;
-  for (uint32_t m = mptr[I]; m < mptr[I + 1]; m++) s += v[4 * (size_t)mlist[m] + c];
-  rc[4 * (size_t)I + c] = s;
+  rc[4 * (size_t)I + c] = member_sum(I, c, mptr, mlist, v);
 }
 
 /* ---- A P by places ------------------------------------------------------------
@@ -182,75 +156,6 @@ __global__ __launch_bounds__(CG_WG) void k_ap_relist(uint32_t n, const uint32_t 
   if (i < n) list[i] = pos[list[i]];
 }
 
-/* a block row of A P as it is stored, and widened */
-template <typename T>
-struct cg_raw { cg_row<T> r; };
-template <>
-struct cg_raw<uint16_t> { uint2 r; };
-
-template <typename T>
-__device__ __forceinline__ void cg_ldraw(const T *p, cg_raw<T> &o) { o.r = cg_ld(p); }
-__device__ __forceinline__ void cg_ldraw(const uint16_t *p, cg_raw<uint16_t> &o)
-{
-  o.r = *reinterpret_cast<const uint2 *>(p);
-}
-template <typename T>
-__device__ __forceinline__ cg_row<double> cg_widen(const cg_raw<T> &o)
-{
-  return {{(double)o.r.v[0], (double)o.r.v[1], (double)o.r.v[2], (double)o.r.v[3]}};
-}
-__device__ __forceinline__ cg_row<double> cg_widen(const cg_raw<uint16_t> &o)
-{
-  return {{__uint_as_float(o.r.x << 16), __uint_as_float(o.r.x & 0xffff0000u), __uint_as_float(o.r.y << 16),
-           __uint_as_float(o.r.y & 0xffff0000u)}};
-}
-
-/* lane I's value in each quad of lanes */
-template <int I>
-__device__ __forceinline__ double cg_quad(double v)
-{
-  return __hiloint2double(__builtin_amdgcn_mov_dpp(__double2hiint(v), I * 0x55, 0xf, 0xf, true),
-                          __builtin_amdgcn_mov_dpp(__double2loint(v), I * 0x55, 0xf, 0xf, true));
-}
-
-#define AP_BATCH 8u   /* blocks of a row loaded together: all of them on a lattice */
-
-/* up to AP_BATCH blocks of the row's n from the k0-th on, from place base on;
- * adds them to acc and moves base past the slice's */
-template <typename TS>
-__device__ __forceinline__ void ap_batch(const TS *__restrict__ ap, const uint32_t *__restrict__ apcol,
-                                         const double *__restrict__ zc, uint32_t &base, uint32_t k0, uint32_t n,
-                                         int c, double &acc)
-{
-  uint32_t at[AP_BATCH], kk[AP_BATCH];
-#pragma unroll
-  for (uint32_t k = 0; k < AP_BATCH; k++) {
-    const uint64_t on = __ballot(k0 + k < n);
-    const uint32_t below =
-        __builtin_amdgcn_mbcnt_hi((uint32_t)(on >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)on, 0u));
-    /* whole quads are on or off: lane c has c more below it than its row */
-    at[k] = k0 + k < n ? base + (below - (uint32_t)c) / 4u : base;
-    base += (uint32_t)__popcll(on) / 4u;
-  }
-  cg_raw<TS> a[AP_BATCH];
-  double z[AP_BATCH];   /* one component a lane */
-#pragma unroll
-  for (uint32_t k = 0; k < AP_BATCH; k++) kk[k] = apcol[at[k]];
-#pragma unroll
-  for (uint32_t k = 0; k < AP_BATCH; k++) cg_ldraw(ap + 16 * (size_t)at[k] + 4 * c, a[k]);
-#pragma unroll
-  for (uint32_t k = 0; k < AP_BATCH; k++) z[k] = zc[4 * (size_t)kk[k] + c];
-#pragma unroll
-  for (uint32_t k = 0; k < AP_BATCH; k++) {
-    const cg_row<double> w = cg_widen(a[k]);
-    double s = acc + w.v[0] * cg_quad<0>(z[k]);
-    s = s + w.v[1] * cg_quad<1>(z[k]);
-    s = s + w.v[2] * cg_quad<2>(z[k]);
-    s = s + w.v[3] * cg_quad<3>(z[k]);
-    acc = k0 + k < n ? s : acc;
-  }
-}
-
 /* t = b - (A P) z_c; per row the A P blocks in ascending aggregate, each
  * component summed a[c][0] z0 + ... + a[c][3] z3 in FP64, the row's first
  * AP_BATCH blocks from ap1 (BF16 with a BF16 preconditioner, else ap itself),
@@ -268,11 +173,7 @@ __global__ __launch_bounds__(CG_WG) void k_coarse_resid(uint32_t N, const uint32
   const uint32_t r = kf_xcd_block() * (CG_WG / 4) + (threadIdx.x >> 2);
   const int c = threadIdx.x & 3;
   if (r >= N) return;
-  const uint32_t n = aprp[r + 1] - aprp[r];
-  uint32_t base = aprp[r & ~15u];
-  double acc = 0.0;
-  ap_batch<TS>(ap1, apcol, zc, base, 0u, n, c, acc);
-  for (uint32_t k0 = AP_BATCH; __any(k0 < n); k0 += AP_BATCH) ap_batch<TA>(ap, apcol, zc, base, k0, n, c, acc);
+  const double acc = ap_product<TS, TA>(r, c, aprp, apcol, ap, ap1, zc);
   const size_t o = 4 * (size_t)r + c;
   t[o] = (TT)(b[o] - acc);
 }
@@ -399,6 +300,39 @@ void kf_coarse_factor(kf_ctx *c)
   kf_prof_end(c, s);
 }
 
+/* The levels below c in one launch, from the members' sums of b to k->zc,
+ * where they are small enough for it (false: they are not, nothing launched) */
+static bool small_levels(kf_ctx *c, const kf_coarse *k, const double *b)
+{
+  kf_small_levels s;
+  int n = 0;
+  for (;;) {
+    kf_ctx *cc = k->cc;
+    if (n == KF_SMALL_LEVELS) return false;
+    kf_small_level &l = s.l[n++];
+    memset(&l, 0, sizeof(l));
+    if (cc->opt.prec != c->opt.prec || !kf_jac_small_level(cc, &l)) return false;
+    l.mptr = k->mptr;
+    l.mlist = k->mlist;
+    l.b = k->rc;
+    l.x = k->zc;
+    if (!cc->opt.coarse) break;
+    kf_coarse *kk = (kf_coarse *)cc->coarse;
+    const bool f64 = c->opt.prec == KF_PREC_FP64, bf = c->opt.prec == KF_PREC_BF16;
+    if (!kk || (f64 ? !kk->ap64 : !kk->ap32) || (bf && !kk->apbf)) return false;
+    if (!f64 && !kk->t32) KF_CHECK(hipMalloc((void **)&kk->t32, 4 * (size_t)cc->d.N * sizeof(float)));
+    l.aprp = kk->aprp;
+    l.apcol = kk->apcol;
+    l.agg = kk->agg;
+    l.ap = f64 ? (const void *)kk->ap64 : (const void *)kk->ap32;
+    l.ap1 = bf ? (const void *)kk->apbf : l.ap;
+    l.t = f64 ? (void *)kk->t : (void *)kk->t32;
+    k = kk;
+  }
+  kf_jac_small_levels(c, s, n, b);
+  return true;
+}
+
 /* x = M b with the two-level preconditioner (b, x device, 4N, not aliased) */
 void kf_coarse_apply(kf_ctx *c, const double *b, double *x)
 {
@@ -417,12 +351,14 @@ void kf_coarse_apply(kf_ctx *c, const double *b, double *x)
   kf_check_aligned(x, "x");
   const kf_dv &d = c->d;
   const int s = kf_prof_begin(c, KP_COARSE);
-  hipLaunchKernelGGL(k_restrict, dim3(kf_blocks_for(k->nc, CG_WG / 4)), dim3(CG_WG), 0, c->stream, k->nc, k->mptr,
-                     k->mlist, b, k->rc);
-  KF_LAUNCH_CHECK();
-  if (k->cc->opt.coarse) kf_coarse_apply(k->cc, k->rc, k->zc);   /* the coarse system by the same scheme */
-  else if (k->cc->opt.jacobi_sweeps > 0) kf_launch_jacobi(k->cc, k->rc, k->zc);
-  else kf_launch_sptrsv(k->cc, k->rc, k->zc, NULL);
+  if (!small_levels(c, k, b)) {
+    hipLaunchKernelGGL(k_restrict, dim3(kf_blocks_for(k->nc, CG_WG / 4)), dim3(CG_WG), 0, c->stream, k->nc, k->mptr,
+                       k->mlist, b, k->rc);
+    KF_LAUNCH_CHECK();
+    if (k->cc->opt.coarse) kf_coarse_apply(k->cc, k->rc, k->zc);   /* the coarse system by the same scheme */
+    else if (k->cc->opt.jacobi_sweeps > 0) kf_launch_jacobi(k->cc, k->rc, k->zc);
+    else kf_launch_sptrsv(k->cc, k->rc, k->zc, NULL);
+  }
   const uint32_t nb = kf_blocks_for(d.N, CG_WG / 4);
   const size_t n4 = 4 * (size_t)d.N;
   const bool sweeps = c->opt.jacobi_sweeps > 0;

@@ -30,7 +30,7 @@
  */
 #include <mutex>
 
-#include "kf_dev.h"
+#include "coarse_dev.h"
 
 #define JAC_WG 256   /* 64 rows per workgroup */
 
@@ -343,51 +343,155 @@ __global__ __launch_bounds__(JAC_WG) void k_jac_upper_sl(uint32_t N, const uint3
 
 /* A whole solve of jacobi_solve_sl in one workgroup, for systems of at most
  * JAC_SMALL_ROWS rows (the small levels of the multilevel preconditioner,
- * where each sweep's launch costs more than its work): the same sweeps,
- * rows, buffers and operations, a barrier between two sweeps instead of a
+ * where each sweep's launch costs more than its work): the same operations
+ * on the same operands, a quad's row of both factors in registers for all
+ * sweeps, the vectors in LDS, a barrier between two sweeps instead of a
  * launch. */
 #define JAC_SMALL_WG 512   /* 2 waves per SIMD: registers for a whole row, no spills */
 #define JAC_SMALL_ROWS (JAC_SMALL_WG / 4)
+
+/* jsum_sl with the slots in registers and the vector in LDS */
+template <int K, typename TM, typename TV>
+__device__ __forceinline__ TV jsum_held(const uint32_t kk[K], const TV m[K][4], int c, uint32_t n,
+                                        const uint32_t *__restrict__ col, const TM *__restrict__ a, uint32_t jcsr,
+                                        const TV (*x)[4])
+{
+  TV s = TV(0);
+#pragma unroll
+  for (int k = 0; k < K; k++) {
+    const TV t = jdot(m[k], x[kk[k]]);
+    s = (uint32_t)k < n ? t + s : s;
+  }
+  for (uint32_t k = K; k < n; k++) {
+    TV m0[4];
+    jrow<TM, TV>(a, jcsr + k, c, m0);
+    const TV t = jdot(m0, x[col[jcsr + k]]);
+    s = t + s;
+  }
+  return s;
+}
+
+template <typename TV>
+__device__ __forceinline__ TV jdinv_held(const TV dg[4], TV u)
+{
+  const TV uv[4] = {jquad<0>(u), jquad<1>(u), jquad<2>(u), jquad<3>(u)};
+  return jdot(dg, uv);
+}
+
+template <int K, typename TM, typename TV, typename TB>
+__device__ __forceinline__ void jac_small(uint32_t N, const uint32_t *__restrict__ rowptr,
+                                          const uint32_t *__restrict__ col, const uint32_t *__restrict__ diag,
+                                          const TM *__restrict__ a, const jsl_view &v, const TB *__restrict__ b,
+                                          double *__restrict__ x, TV (*xs)[JAC_SMALL_ROWS][4], int k,
+                                          const uint32_t *__restrict__ pagg, const double *__restrict__ pzc)
+{
+  const int c = threadIdx.x & 3;
+  const uint32_t row = threadIdx.x >> 2;   /* one row per quad: N <= JAC_SMALL_ROWS */
+  const bool on = row < N;
+  const uint32_t r = on ? row : 0u, sl = r >> 4, q = r & 15u;
+  const uint32_t j0 = rowptr[r], jd = diag[r], nl = jd - j0, nu = rowptr[r + 1] - jd - 1;
+  const size_t nk = (size_t)v.nslice * K;
+  const TM *sv = static_cast<const TM *>(v.val);
+  uint32_t kl[K], ku[K];
+  TV ml[K][4], mu[K][4], dg[4];
+#pragma unroll
+  for (int i = 0; i < K; i++) {
+    const size_t at = ((size_t)sl * K + i) * 16 + q;
+    kl[i] = v.col[at];
+    ku[i] = v.col[nk * 16 + at];
+    jld4<TM, TV>(sv + at * 16 + 4 * c, ml[i]);
+    jld4<TM, TV>(sv + nk * 256 + at * 16 + 4 * c, mu[i]);
+  }
+  jld4<TM, TV>(sv + 2 * nk * 256 + ((size_t)sl * 16 + q) * 16 + 4 * c, dg);
+  const TV br = (TV)b[4 * (size_t)r + c];
+  int cur = 0;
+  if (on) xs[0][row][c] = br;   /* the first sweep reads b itself */
+  __syncthreads();
+  TV y = TV(0);
+  for (int sw = 1; sw <= k; sw++) {
+    y = (-jsum_held<K, TM, TV>(kl, ml, c, nl, col, a, j0, xs[cur])) + br;
+    cur ^= 1;
+    if (on) xs[cur][row][c] = sw == k ? jdinv_held(dg, y) : y;   /* the backward sweeps start from D^-1 y */
+    __syncthreads();
+  }
+  for (int sw = 1; sw <= k; sw++) {
+    const TV u = (-jsum_held<K, TM, TV>(ku, mu, c, nu, col, a, jd + 1, xs[cur])) + y;
+    const TV xr = jdinv_held(dg, u);
+    if (sw == k) {
+      double xo = (double)xr;
+      if (on) {
+        if (pagg) xo = xo + pzc[4 * (size_t)pagg[r] + c];
+        x[4 * (size_t)r + c] = xo;
+      }
+    } else {
+      cur ^= 1;
+      if (on) xs[cur][row][c] = xr;
+      __syncthreads();
+    }
+  }
+}
+
 template <int K, typename TM, typename TV, typename TB>
 __global__ __launch_bounds__(JAC_SMALL_WG) void k_jac_small(uint32_t N, const uint32_t *__restrict__ rowptr,
                                                             const uint32_t *__restrict__ col,
                                                             const uint32_t *__restrict__ diag,
                                                             const TM *__restrict__ a, jsl_view v,
-                                                            const TB *__restrict__ b, double *__restrict__ x,
-                                                            TV *__restrict__ y, TV *__restrict__ p0,
-                                                            TV *__restrict__ p1, int k,
+                                                            const TB *__restrict__ b, double *__restrict__ x, int k,
                                                             const uint32_t *__restrict__ pagg,
                                                             const double *__restrict__ pzc)
 {
+  __shared__ __align__(16) TV xs[2][JAC_SMALL_ROWS][4];
+  jac_small<K, TM, TV, TB>(N, rowptr, col, diag, a, v, b, x, xs, k, pagg, pzc);
+}
+
+/* a level's solve of k_jac_small_levels: of its members' sums (the last
+ * level), else of the remainder t, then x += P z_c */
+template <int K, typename TM, typename TV>
+__device__ __forceinline__ void small_level_solve(const kf_small_level &l, const double *zc,
+                                                  TV (*xs)[JAC_SMALL_ROWS][4])
+{
+  const jsl_view v = {l.nslice, l.val, l.scol};
+  const TM *a = static_cast<const TM *>(l.a);
+  if (zc)
+    jac_small<K, TM, TV, TV>(l.N, l.rowptr, l.col, l.diag, a, v, static_cast<const TV *>(l.t), l.x, xs, l.sweeps,
+                             l.agg, zc);
+  else
+    jac_small<K, TM, TV, double>(l.N, l.rowptr, l.col, l.diag, a, v, l.b, l.x, xs, l.sweeps, (const uint32_t *)NULL,
+                                 (const double *)NULL);
+}
+
+/* All levels of at most JAC_SMALL_ROWS rows in one workgroup: down by the
+ * members' sums, up by remainder and sweeps, the launches' operations in
+ * their order with a barrier in each one's place.  Bound by its chain of
+ * loads from memory that the larger levels have swept out of the caches:
+ * five levels (81 rows to 1) 37 us, as 13 launches 64. */
+template <typename TM, typename TV, typename TA>
+__global__ __launch_bounds__(JAC_SMALL_WG) void k_jac_small_levels(kf_small_levels s, int n,
+                                                                   const double *__restrict__ b)
+{
+  __shared__ __align__(16) TV xs[2][JAC_SMALL_ROWS][4];
   const int c = threadIdx.x & 3;
-  const uint32_t r = threadIdx.x >> 2;   /* one row per quad: N <= JAC_SMALL_ROWS */
-  const bool on = r < N;
-  TV *const xread = k >= 2 ? (((k - 1) & 1) ? p0 : p1) : NULL;
-  TV *cur = xread == p0 ? p1 : p0;
-  const TV *prev = NULL;
-  for (int sw = 1; sw <= k; sw++) {
-    TV *out = sw == k ? y : ((sw & 1) ? p0 : p1);
-    if (on) {
-      if (sw == 1 && sw == k) jac_lower_row<K, TM, TV, TB, TB, true>(r, c, rowptr, col, diag, a, v, b, b, out, cur);
-      else if (sw == 1) jac_lower_row<K, TM, TV, TB, TB, false>(r, c, rowptr, col, diag, a, v, b, b, out, (TV *)NULL);
-      else if (sw == k) jac_lower_row<K, TM, TV, TB, TV, true>(r, c, rowptr, col, diag, a, v, b, prev, out, cur);
-      else jac_lower_row<K, TM, TV, TB, TV, false>(r, c, rowptr, col, diag, a, v, b, prev, out, (TV *)NULL);
-    }
-    prev = out;
+  const uint32_t r = threadIdx.x >> 2;
+  for (int i = 0; i < n; i++) {
+    const kf_small_level &l = s.l[i];
+    if (r < l.N) l.b[4 * (size_t)r + c] = member_sum(r, c, l.mptr, l.mlist, i ? s.l[i - 1].b : b);
     __syncthreads();
   }
-  TV *other = cur == p0 ? p1 : p0;
-  for (int sw = 1; sw <= k; sw++) {
-    if (sw == k) {
-      if (on) jac_upper_row<K, TM, TV, double>(r, c, rowptr, col, diag, a, v, y, cur, x, pagg, pzc);
-    } else {
-      if (on) jac_upper_row<K, TM, TV, TV>(r, c, rowptr, col, diag, a, v, y, cur, other, (const uint32_t *)NULL,
-                                           (const double *)NULL);
-      TV *t = cur;
-      cur = other;
-      other = t;
+  for (int i = n - 1; i >= 0; i--) {
+    const kf_small_level &l = s.l[i];
+    const double *zc = i + 1 < n ? s.l[i + 1].x : NULL;
+    if (zc) {
+      if (r < l.N) {
+        const size_t o = 4 * (size_t)r + c;
+        static_cast<TV *>(l.t)[o] =
+            (TV)(l.b[o] - ap_product<TM, TA>(r, c, l.aprp, l.apcol, static_cast<const TA *>(l.ap),
+                                             static_cast<const TM *>(l.ap1), zc));
+      }
       __syncthreads();
     }
+    if (l.K == 7) small_level_solve<7, TM, TV>(l, zc, xs);
+    else small_level_solve<8, TM, TV>(l, zc, xs);
+    __syncthreads();
   }
 }
 
@@ -525,6 +629,13 @@ static void upper_sl(kf_ctx *c, const TM *a, const jsl_view &v, const TV *y, con
   KF_LAUNCH_CHECK();
 }
 
+/* KF_JAC_SMALL=0: no solves in one workgroup */
+static bool jac_small_on()
+{
+  static const bool on = !(getenv("KF_JAC_SMALL") && atoi(getenv("KF_JAC_SMALL")) == 0);
+  return on;
+}
+
 /* jacobi_solve over the sliced factors, the right-hand side in TB (double,
  * or float where the sweeps compute in FP32 anyway: the same bits), and
  * with pagg non-NULL the prolongation x += P z_c fused into the last sweep */
@@ -532,12 +643,11 @@ template <int K, typename TM, typename TV, typename TB>
 static void jacobi_solve_sl(kf_ctx *c, const TM *a, const TB *b, double *x, TV *y, TV *p0, TV *p1, int k,
                             const jsl_view &v, const uint32_t *pagg, const double *pzc)
 {
-  static const bool small_on = !(getenv("KF_JAC_SMALL") && atoi(getenv("KF_JAC_SMALL")) == 0);
-  if (small_on && c->d.N <= JAC_SMALL_ROWS) {   /* the whole solve in one workgroup (KF_JAC_SMALL=0: never) */
+  if (jac_small_on() && c->d.N <= JAC_SMALL_ROWS) {   /* the whole solve in one workgroup */
     const kf_dv &d = c->d;
     const int s = kf_prof_begin(c, KP_JAC_L);
     hipLaunchKernelGGL((k_jac_small<K, TM, TV, TB>), dim3(1), dim3(JAC_SMALL_WG), 0, c->stream, d.N, d.rowptr, d.col,
-                       d.diag, a, v, b, x, y, p0, p1, k, pagg, pzc);
+                       d.diag, a, v, b, x, k, pagg, pzc);
     KF_LAUNCH_CHECK();
     kf_prof_end(c, s);
     return;
@@ -675,6 +785,39 @@ static void jacobi_launch(kf_ctx *c, const TB *b, double *x, const uint32_t *pag
     else jacobi_solve_sl<8, uint16_t, float, TB>(c, c->abf, b, x, y, p0, p1, k, v, pagg, pzc);
   }
   c->ystate[1] = ~(uint64_t)0;
+}
+
+/* c's part of a level of k_jac_small_levels */
+bool kf_jac_small_level(kf_ctx *c, kf_small_level *o)
+{
+  const int k = c->opt.jacobi_sweeps;
+  if (!jac_small_on() || c->d.N > JAC_SMALL_ROWS || k < 1 || k > KF_JACOBI_MAX) return false;
+  const bool f64 = c->opt.prec == KF_PREC_FP64;
+  o->a = f64 ? (const void *)c->a64 : c->opt.prec == KF_PREC_FP32 ? (const void *)c->a32 : (const void *)c->abf;
+  if (!o->a) return false;
+  const jsl_view v = jsl_pack(c);
+  o->N = c->d.N;
+  o->nslice = v.nslice;
+  o->K = c->jsl_k;
+  o->sweeps = k;
+  o->rowptr = c->d.rowptr;
+  o->col = c->d.col;
+  o->diag = c->d.diag;
+  o->scol = v.col;
+  o->val = v.val;
+  return true;
+}
+
+/* n levels, the first one's members those of b; c: the level above them */
+void kf_jac_small_levels(kf_ctx *c, const kf_small_levels &s, int n, const double *b)
+{
+  const dim3 one(1), wg(JAC_SMALL_WG);
+  if (c->opt.prec == KF_PREC_FP64)
+    hipLaunchKernelGGL((k_jac_small_levels<double, double, double>), one, wg, 0, c->stream, s, n, b);
+  else if (c->opt.prec == KF_PREC_FP32)
+    hipLaunchKernelGGL((k_jac_small_levels<float, float, float>), one, wg, 0, c->stream, s, n, b);
+  else hipLaunchKernelGGL((k_jac_small_levels<uint16_t, float, float>), one, wg, 0, c->stream, s, n, b);
+  KF_LAUNCH_CHECK();
 }
 
 /* x ~ U^-1 L^-1 b with c->opt.jacobi_sweeps sweeps each way, in the
