@@ -145,7 +145,7 @@ struct kf_small_level {
   uint32_t N, nslice;
   int K, sweeps;
   const uint32_t *rowptr, *col, *diag, *scol;
-  const void *a, *val;
+  const void *a, *val, *near;
   const uint32_t *mptr, *mlist;     /* members, of the level above */
   double *b, *x;
   /* towards the level below it (none: aprp is NULL) */

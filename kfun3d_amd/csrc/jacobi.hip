@@ -187,7 +187,11 @@ __global__ __launch_bounds__(JAC_WG) void k_jac_upper(uint32_t N, const uint32_t
  *   L:  [slice][k][row of slice][16]    the k-th block left of the diagonal
  *   U:  [slice][k][row of slice][16]    the k-th block right of it
  *   D:  [slice][row of slice][16]       the inverted diagonal block
- * and the slots' columns (jsl_col): L then U, [slice][k][row of slice].  A
+ * and the slots' columns (jsl_col): L then U, [slice][k][row of slice], or,
+ * with K = 7 and no column further than 32767 rows from its own, one 16-byte
+ * record a row and side (jsl_near): its distances and its length, in place of
+ * seven columns and two row pointers (312 -> 292 bytes a row and sweep in
+ * BF16, one load for nine).  A
  * slot past a row's end holds zeros and the row's own column; the sweeps
  * select it away (the counts come from rowptr and diag), so the sums are
  * the CSR kernels' to the bit.  Entries past slot K (rows longer than K,
@@ -225,13 +229,10 @@ __device__ __forceinline__ void jld4<float, float>(const float *p, float m[4])
 /* s over a row's part: slots [0, min(n, K)) from the slice, the rest of the
  * n entries from the CSR array from position jcsr */
 template <int K, typename TM, typename TV, typename TX>
-__device__ __forceinline__ TV jsum_sl(const TM *__restrict__ sv, const uint32_t *__restrict__ sc, uint32_t base,
-                                      uint32_t q, int c, uint32_t n, const uint32_t *__restrict__ col,
-                                      const TM *__restrict__ a, uint32_t jcsr, const TX *__restrict__ x)
+__device__ __forceinline__ TV jsum_sl(const TM *__restrict__ sv, const uint32_t kk[K], uint32_t base, uint32_t q,
+                                      int c, uint32_t n, const uint32_t *__restrict__ col, const TM *__restrict__ a,
+                                      uint32_t jcsr, const TX *__restrict__ x)
 {
-  uint32_t kk[K];
-#pragma unroll
-  for (int k = 0; k < K; k++) kk[k] = sc[(size_t)(base + k) * 16 + q];
   TV m[K][4], xv[K][4];
 #pragma unroll
   for (int k = 0; k < K; k++) jld4<TM, TV>(sv + ((size_t)(base + k) * 16 + q) * 16 + 4 * c, m[k]);
@@ -269,8 +270,33 @@ __device__ __forceinline__ TV jdinv_sl(const TM *__restrict__ dv, size_t o, TV u
 struct jsl_view {
   uint32_t nslice;
   const void *val;        /* L, U, D */
-  const uint32_t *col;    /* L, U */
+  const uint32_t *col;    /* L, U; or */
+  const uint4 *near;      /* L, U: a record a row */
 };
+
+/* row r's columns in its slots, its length n and where its entries start in
+ * the CSR arrays (side 0: L, 1: U) */
+template <int K>
+__device__ __forceinline__ void jsl_row(const jsl_view &v, int side, uint32_t r, const uint32_t *__restrict__ rowptr,
+                                        const uint32_t *__restrict__ diag, uint32_t kk[K], uint32_t &n,
+                                        uint32_t &jcsr)
+{
+  if (K == 7 && v.near) {
+    const uint4 m = v.near[(size_t)side * v.nslice * 16 + r];
+    const uint32_t w[4] = {m.x, m.y, m.z, m.w};
+#pragma unroll
+    for (int k = 0; k < K; k++) kk[k] = r + (uint32_t)(int32_t)(int16_t)(w[k / 2] >> (k & 1 ? 16 : 0));
+    n = m.w >> 16;
+    jcsr = 0;   /* no entry is past the slots */
+    return;
+  }
+  const uint32_t jd = diag[r];
+  if (side) { jcsr = jd + 1; n = rowptr[r + 1] - jcsr; }
+  else { jcsr = rowptr[r]; n = jd - jcsr; }
+  const uint32_t *sc = v.col + (size_t)side * v.nslice * K * 16;
+#pragma unroll
+  for (int k = 0; k < K; k++) kk[k] = sc[((size_t)(r >> 4) * K + k) * 16 + (r & 15u)];
+}
 
 /* row r of one forward sweep (lane c of its quad) */
 template <int K, typename TM, typename TV, typename TB, typename TX, bool DIAG>
@@ -279,9 +305,11 @@ __device__ __forceinline__ void jac_lower_row(uint32_t r, int c, const uint32_t 
                                               const TM *__restrict__ a, const jsl_view &v, const TB *__restrict__ b,
                                               const TX *__restrict__ xin, TV *__restrict__ y, TV *__restrict__ x0)
 {
-  const uint32_t sl = r >> 4, q = r & 15u, j0 = rowptr[r], jd = diag[r];
+  const uint32_t sl = r >> 4, q = r & 15u;
+  uint32_t kk[K], n, jcsr;
+  jsl_row<K>(v, 0, r, rowptr, diag, kk, n, jcsr);
   const TM *sv = static_cast<const TM *>(v.val);
-  const TV s = jsum_sl<K, TM, TV, TX>(sv, v.col, sl * K, q, c, jd - j0, col, a, j0, xin);
+  const TV s = jsum_sl<K, TM, TV, TX>(sv, kk, sl * K, q, c, n, col, a, jcsr, xin);
   const TV u = (-s) + (TV)b[4 * (size_t)r + c];
   y[4 * (size_t)r + c] = u;
   if (DIAG) {
@@ -312,11 +340,12 @@ __device__ __forceinline__ void jac_upper_row(uint32_t r, int c, const uint32_t 
                                               const TV *__restrict__ xin, TO *__restrict__ x,
                                               const uint32_t *__restrict__ pagg, const double *__restrict__ pzc)
 {
-  const uint32_t sl = r >> 4, q = r & 15u, jd = diag[r];
+  const uint32_t sl = r >> 4, q = r & 15u;
+  uint32_t kk[K], n, jcsr;
+  jsl_row<K>(v, 1, r, rowptr, diag, kk, n, jcsr);
   const TM *sv = static_cast<const TM *>(v.val);
   const size_t nk = (size_t)v.nslice * K;
-  const TV s = jsum_sl<K, TM, TV, TV>(sv + nk * 256, v.col + nk * 16, sl * K, q, c, rowptr[r + 1] - jd - 1, col, a,
-                                      jd + 1, xin);
+  const TV s = jsum_sl<K, TM, TV, TV>(sv + nk * 256, kk, sl * K, q, c, n, col, a, jcsr, xin);
   const TV u = (-s) + y[4 * (size_t)r + c];
   const TM *dv = sv + 2 * nk * 256;
   TO xo = (TO)jdinv_sl<TM, TV>(dv, ((size_t)sl * 16 + q) * 16 + 4 * c, u);
@@ -389,16 +418,15 @@ __device__ __forceinline__ void jac_small(uint32_t N, const uint32_t *__restrict
   const uint32_t row = threadIdx.x >> 2;   /* one row per quad: N <= JAC_SMALL_ROWS */
   const bool on = row < N;
   const uint32_t r = on ? row : 0u, sl = r >> 4, q = r & 15u;
-  const uint32_t j0 = rowptr[r], jd = diag[r], nl = jd - j0, nu = rowptr[r + 1] - jd - 1;
   const size_t nk = (size_t)v.nslice * K;
   const TM *sv = static_cast<const TM *>(v.val);
-  uint32_t kl[K], ku[K];
+  uint32_t kl[K], ku[K], nl, nu, jl, ju;
+  jsl_row<K>(v, 0, r, rowptr, diag, kl, nl, jl);
+  jsl_row<K>(v, 1, r, rowptr, diag, ku, nu, ju);
   TV ml[K][4], mu[K][4], dg[4];
 #pragma unroll
   for (int i = 0; i < K; i++) {
     const size_t at = ((size_t)sl * K + i) * 16 + q;
-    kl[i] = v.col[at];
-    ku[i] = v.col[nk * 16 + at];
     jld4<TM, TV>(sv + at * 16 + 4 * c, ml[i]);
     jld4<TM, TV>(sv + nk * 256 + at * 16 + 4 * c, mu[i]);
   }
@@ -409,13 +437,13 @@ __device__ __forceinline__ void jac_small(uint32_t N, const uint32_t *__restrict
   __syncthreads();
   TV y = TV(0);
   for (int sw = 1; sw <= k; sw++) {
-    y = (-jsum_held<K, TM, TV>(kl, ml, c, nl, col, a, j0, xs[cur])) + br;
+    y = (-jsum_held<K, TM, TV>(kl, ml, c, nl, col, a, jl, xs[cur])) + br;
     cur ^= 1;
     if (on) xs[cur][row][c] = sw == k ? jdinv_held(dg, y) : y;   /* the backward sweeps start from D^-1 y */
     __syncthreads();
   }
   for (int sw = 1; sw <= k; sw++) {
-    const TV u = (-jsum_held<K, TM, TV>(ku, mu, c, nu, col, a, jd + 1, xs[cur])) + y;
+    const TV u = (-jsum_held<K, TM, TV>(ku, mu, c, nu, col, a, ju, xs[cur])) + y;
     const TV xr = jdinv_held(dg, u);
     if (sw == k) {
       double xo = (double)xr;
@@ -450,7 +478,7 @@ template <int K, typename TM, typename TV>
 __device__ __forceinline__ void small_level_solve(const kf_small_level &l, const double *zc,
                                                   TV (*xs)[JAC_SMALL_ROWS][4])
 {
-  const jsl_view v = {l.nslice, l.val, l.scol};
+  const jsl_view v = {l.nslice, l.val, l.scol, static_cast<const uint4 *>(l.near)};
   const TM *a = static_cast<const TM *>(l.a);
   if (zc)
     jac_small<K, TM, TV, TV>(l.N, l.rowptr, l.col, l.diag, a, v, static_cast<const TV *>(l.t), l.x, xs, l.sweeps,
@@ -501,7 +529,8 @@ template <int K, typename TM>
 __global__ __launch_bounds__(JAC_WG) void k_jac_pack(uint32_t N, uint32_t nslice, const uint32_t *__restrict__ rowptr,
                                                      const uint32_t *__restrict__ col,
                                                      const uint32_t *__restrict__ diag, const TM *__restrict__ a,
-                                                     TM *__restrict__ val, uint32_t *__restrict__ scol)
+                                                     TM *__restrict__ val, uint32_t *__restrict__ scol,
+                                                     uint4 *__restrict__ near)
 {
   const uint32_t r = kf_xcd_block() * (JAC_WG / 4) + (threadIdx.x >> 2);
   const int c = threadIdx.x & 3;
@@ -524,7 +553,12 @@ __global__ __launch_bounds__(JAC_WG) void k_jac_pack(uint32_t N, uint32_t nslice
       } else {
         o[0] = o[1] = o[2] = o[3] = TM(0);
       }
-      if (c == 0) pc[slot * 16 + q] = (uint32_t)k < n ? col[first + k] : r;
+      if (c == 0 && !near) pc[slot * 16 + q] = (uint32_t)k < n ? col[first + k] : r;
+    }
+    if (c == 0 && near) {
+      uint32_t w[4] = {0u, 0u, 0u, n << 16};
+      for (uint32_t k = 0; k < n && k < 7u; k++) w[k / 2] |= ((col[first + k] - r) & 0xffffu) << (k & 1u ? 16 : 0);
+      near[(size_t)part * nslice * 16 + r] = make_uint4(w[0], w[1], w[2], w[3]);
     }
   }
   TM *o = val + 2 * nk * 256 + ((size_t)sl * 16 + q) * 16 + 4 * c;
@@ -684,10 +718,10 @@ static void jsl_pack_as(kf_ctx *c, const TM *a, uint32_t nslice)
   const dim3 grid(kf_blocks_for(d.N, JAC_WG / 4)), block(JAC_WG);
   if (c->jsl_k == 7)
     hipLaunchKernelGGL((k_jac_pack<7, TM>), grid, block, 0, c->stream, d.N, nslice, d.rowptr, d.col, d.diag, a,
-                       (TM *)c->jsl_val, c->jsl_col);
+                       (TM *)c->jsl_val, c->jsl_col, (uint4 *)c->jsl_near);
   else
     hipLaunchKernelGGL((k_jac_pack<8, TM>), grid, block, 0, c->stream, d.N, nslice, d.rowptr, d.col, d.diag, a,
-                       (TM *)c->jsl_val, c->jsl_col);
+                       (TM *)c->jsl_val, c->jsl_col, (uint4 *)NULL);
   KF_LAUNCH_CHECK();
 }
 
@@ -713,7 +747,9 @@ void *kf_jac_slices(kf_ctx *c, uint32_t *K, uint32_t *nslice)
     KF_CHECK(hipFree(c->jsl_val));
     c->jsl_val = NULL;
   }
-  if (!c->jsl_col) KF_CHECK(hipMalloc((void **)&c->jsl_col, 2 * nk * 16 * sizeof(uint32_t)));
+  if (c->jsl_k == 7 && c->cols_near) {
+    if (!c->jsl_near) KF_CHECK(hipMalloc(&c->jsl_near, 2 * (size_t)ns * 16 * sizeof(uint4)));
+  } else if (!c->jsl_col) KF_CHECK(hipMalloc((void **)&c->jsl_col, 2 * nk * 16 * sizeof(uint32_t)));
   if (!c->jsl_val) {
     KF_CHECK(hipMalloc(&c->jsl_val, (2 * nk + ns) * 256 * es));
     c->jsl_esize = es;
@@ -734,6 +770,7 @@ static jsl_view jsl_pack(kf_ctx *c)
   v.val = kf_jac_slices(c, &K, &nslice);
   v.nslice = nslice;
   v.col = c->jsl_col;
+  v.near = (const uint4 *)c->jsl_near;
   if (!c->jsl_fresh) {
     jsl_pack_now(c, nslice);
     c->jsl_fresh = 1;
@@ -804,6 +841,7 @@ bool kf_jac_small_level(kf_ctx *c, kf_small_level *o)
   o->col = c->d.col;
   o->diag = c->d.diag;
   o->scol = v.col;
+  o->near = v.near;
   o->val = v.val;
   return true;
 }

@@ -179,7 +179,9 @@ struct kf_ctx {
   double *jac64;            /* Jacobi sweeps' ping-pong buffers (2 x 4N, FP64 ...) */
   float *jac32;             /* ... or FP32) */
   void *jsl_val;            /* the factors packed per 16-row slice for the Jacobi sweeps (jacobi.hip) */
-  uint32_t *jsl_col;        /* ... their columns */
+  uint32_t *jsl_col;        /* ... their columns, or ... */
+  void *jsl_near;           /* ... a record of distances a row and side (with cols_near and 7 slots) */
+  int cols_near;            /* no column is further than 32767 rows from its row's */
   size_t jsl_esize;         /* bytes per packed value */
   uint32_t jsl_k;           /* slots per row and side */
   int jsl_fresh;            /* 1: packed from the current factors */
