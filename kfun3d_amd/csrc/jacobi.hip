@@ -233,15 +233,19 @@ __device__ __forceinline__ TV jsum_sl(const TM *__restrict__ sv, const uint32_t 
                                       int c, uint32_t n, const uint32_t *__restrict__ col, const TM *__restrict__ a,
                                       uint32_t jcsr, const TX *__restrict__ x)
 {
-  TV m[K][4], xv[K][4];
+  TV m[K][4], xv[K];
 #pragma unroll
   for (int k = 0; k < K; k++) jld4<TM, TV>(sv + ((size_t)(base + k) * 16 + q) * 16 + 4 * c, m[k]);
+  /* a component a lane, which the quad exchanges: loaded whole by each lane,
+   * the vectors took the L1's time and 14 registers more (288x96x96 in BF16,
+   * all levels: 1033 -> 973 us) */
 #pragma unroll
-  for (int k = 0; k < K; k++) jvec<TV, TX>(x, kk[k], xv[k]);
+  for (int k = 0; k < K; k++) xv[k] = (TV)x[4 * (size_t)kk[k] + c];
   TV s = TV(0);
 #pragma unroll
   for (int k = 0; k < K; k++) {
-    const TV t = jdot(m[k], xv[k]);
+    const TV xq[4] = {jquad<0>(xv[k]), jquad<1>(xv[k]), jquad<2>(xv[k]), jquad<3>(xv[k])};
+    const TV t = jdot(m[k], xq);
     s = (uint32_t)k < n ? t + s : s;
   }
   for (uint32_t k = K; k < n; k++) {
