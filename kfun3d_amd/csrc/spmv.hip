@@ -13,64 +13,79 @@
  * of  a_j[c][0] x0 + a_j[c][1] x1 + a_j[c][2] x2 + a_j[c][3] x3,  each
  * product added to the running sum in that order, in FP64 (FP32-stored
  * values are widened first).  The four lanes of a quad read one 128-byte
- * block (FP64) row by row, so a wave's loads are whole blocks; the column's
- * four x values are the same address for the quad.  Workgroups are remapped
- * XCD by XCD (kf_xcd_block) so that each XCD works on a contiguous slab of
- * rows and its x gathers stay in its L2.  Two blocks are in flight per lane
- * step.  Bytes per launch: nnzb (16 s + 4) + 64 N with s the stored value
- * size (HBM-bound).
+ * block (FP64) row by row, so a wave's loads are whole blocks; of the column's
+ * four x values each loads one, and the quad exchanges them.  Workgroups are
+ * remapped XCD by XCD (kf_xcd_block) so that each XCD works on a contiguous
+ * slab of rows and its x gathers stay in its L2.  Bytes per launch:
+ * nnzb (16 s + 4) + 64 N with s the stored value size (HBM-bound: 4 to 8 blocks
+ * in flight a lane and 4 to 8 wavefronts a SIMD measure the same).
  */
 #include "kf_dev.h"
 
 #define SPMV_WG 256   /* 64 rows per workgroup */
 
+/* a block row as it is stored */
 template <typename T>
-__device__ __forceinline__ void load_row4(const T *a, size_t j, int c, double &a0, double &a1, double &a2, double &a3);
-
+struct spmv_row;
 template <>
-__device__ __forceinline__ void load_row4<double>(const double *a, size_t j, int c, double &a0, double &a1, double &a2,
-                                                  double &a3)
+struct spmv_row<double> {
+  double2 u, v;
+  __device__ __forceinline__ void load(const double *p)
+  {
+    u = reinterpret_cast<const double2 *>(p)[0];
+    v = reinterpret_cast<const double2 *>(p)[1];
+  }
+  __device__ __forceinline__ void get(double a[4]) const { a[0] = u.x; a[1] = u.y; a[2] = v.x; a[3] = v.y; }
+};
+template <>
+struct spmv_row<float> {
+  float4 u;
+  __device__ __forceinline__ void load(const float *p) { u = *reinterpret_cast<const float4 *>(p); }
+  __device__ __forceinline__ void get(double a[4]) const
+  {
+    a[0] = (double)u.x; a[1] = (double)u.y; a[2] = (double)u.z; a[3] = (double)u.w;
+  }
+};
+
+/* lane I's value in each quad of lanes */
+template <int I>
+__device__ __forceinline__ double spmv_quad(double v)
 {
-  const double2 *p = reinterpret_cast<const double2 *>(a + 16 * j + 4 * c);
-  const double2 u = p[0], v = p[1];
-  a0 = u.x; a1 = u.y; a2 = v.x; a3 = v.y;
+  return __hiloint2double(__builtin_amdgcn_mov_dpp(__double2hiint(v), I * 0x55, 0xf, 0xf, true),
+                          __builtin_amdgcn_mov_dpp(__double2loint(v), I * 0x55, 0xf, 0xf, true));
 }
 
-template <>
-__device__ __forceinline__ void load_row4<float>(const float *a, size_t j, int c, double &a0, double &a1, double &a2,
-                                                 double &a3)
-{
-  const float4 u = *reinterpret_cast<const float4 *>(a + 16 * j + 4 * c);
-  a0 = (double)u.x; a1 = (double)u.y; a2 = (double)u.z; a3 = (double)u.w;
-}
-
 template <typename T>
-__global__ __launch_bounds__(SPMV_WG) void k_bsr_spmv(uint32_t N, const uint32_t *__restrict__ rowptr,
+__global__ __launch_bounds__(SPMV_WG, 6) void k_bsr_spmv(uint32_t N, const uint32_t *__restrict__ rowptr,
                                                       const uint32_t *__restrict__ col, const T *__restrict__ a,
                                                       const double *__restrict__ x, double *__restrict__ y)
 {
+  constexpr uint32_t B = sizeof(T) == 4 ? 8 : 4;   /* blocks in flight, 32 registers of them */
   const uint32_t r = kf_xcd_block() * (SPMV_WG / 4) + (threadIdx.x >> 2);
   const int c = threadIdx.x & 3;
-  if (r >= N) return;
-  const uint32_t j0 = rowptr[r], j1 = rowptr[r + 1];
+  if (r >= N) return;   /* whole quads leave together */
+  const uint32_t j1 = rowptr[r + 1];
   double acc = 0.0;
-  uint32_t j = j0;
-  for (; j + 1 < j1; j += 2) {
-    const uint32_t k0 = col[j], k1 = col[j + 1];
-    double p0, p1, p2, p3, q0, q1, q2, q3;
-    load_row4<T>(a, j, c, p0, p1, p2, p3);
-    load_row4<T>(a, j + 1, c, q0, q1, q2, q3);
-    const double4 u = *reinterpret_cast<const double4 *>(x + 4 * (size_t)k0);
-    const double4 v = *reinterpret_cast<const double4 *>(x + 4 * (size_t)k1);
-    acc = acc + p0 * u.x; acc = acc + p1 * u.y; acc = acc + p2 * u.z; acc = acc + p3 * u.w;
-    acc = acc + q0 * v.x; acc = acc + q1 * v.y; acc = acc + q2 * v.z; acc = acc + q3 * v.w;
-  }
-  if (j < j1) {
-    const uint32_t k0 = col[j];
-    double p0, p1, p2, p3;
-    load_row4<T>(a, j, c, p0, p1, p2, p3);
-    const double4 u = *reinterpret_cast<const double4 *>(x + 4 * (size_t)k0);
-    acc = acc + p0 * u.x; acc = acc + p1 * u.y; acc = acc + p2 * u.z; acc = acc + p3 * u.w;
+  for (uint32_t j = rowptr[r]; j < j1; j += B) {
+    uint32_t kk[B];
+    spmv_row<T> m[B];
+    double xc[B];   /* a component a lane */
+#pragma unroll
+    for (uint32_t i = 0; i < B; i++) kk[i] = col[min(j + i, j1 - 1u)];
+#pragma unroll
+    for (uint32_t i = 0; i < B; i++) m[i].load(a + 16 * (size_t)min(j + i, j1 - 1u) + 4 * c);
+#pragma unroll
+    for (uint32_t i = 0; i < B; i++) xc[i] = x[4 * (size_t)kk[i] + c];
+#pragma unroll
+    for (uint32_t i = 0; i < B; i++) {
+      double w[4];
+      m[i].get(w);
+      double s = acc + w[0] * spmv_quad<0>(xc[i]);
+      s = s + w[1] * spmv_quad<1>(xc[i]);
+      s = s + w[2] * spmv_quad<2>(xc[i]);
+      s = s + w[3] * spmv_quad<3>(xc[i]);
+      acc = j + i < j1 ? s : acc;
+    }
   }
   y[4 * (size_t)r + c] = acc;
 }
