@@ -14,7 +14,7 @@
  * product added to the running sum in that order, in FP64 (FP32-stored
  * values are widened first).  The four lanes of a quad read one 128-byte
  * block (FP64) row by row, so a wave's loads are whole blocks; of the column's
- * four x values each loads one, and the quad exchanges them.  Workgroups are
+ * four x values each loads one, and the quad exchanges them (FP32 blocks).  Workgroups are
  * remapped XCD by XCD (kf_xcd_block) so that each XCD works on a contiguous
  * slab of rows and its x gathers stay in its L2.  Bytes per launch:
  * nnzb (16 s + 4) + 64 N with s the stored value size (HBM-bound: 4 to 8 blocks
@@ -60,13 +60,42 @@ __global__ __launch_bounds__(SPMV_WG, 6) void k_bsr_spmv(uint32_t N, const uint3
                                                       const uint32_t *__restrict__ col, const T *__restrict__ a,
                                                       const double *__restrict__ x, double *__restrict__ y)
 {
-  constexpr uint32_t B = sizeof(T) == 4 ? 8 : 4;   /* blocks in flight, 32 registers of them */
   const uint32_t r = kf_xcd_block() * (SPMV_WG / 4) + (threadIdx.x >> 2);
   const int c = threadIdx.x & 3;
   if (r >= N) return;   /* whole quads leave together */
   const uint32_t j1 = rowptr[r + 1];
   double acc = 0.0;
-  for (uint32_t j = rowptr[r]; j < j1; j += B) {
+  uint32_t j = rowptr[r];
+  if constexpr (sizeof(T) == 8) {
+    /* two blocks at a time, the column's whole vector in each lane: a block of
+     * FP64 is a line by itself and the product at the memory's rate (288x96x96
+     * 1.04 ms; 1.08 with the exchange below, four blocks at a time) */
+    for (; j + 1 < j1; j += 2) {
+      const uint32_t k0 = col[j], k1 = col[j + 1];
+      spmv_row<T> m0, m1;
+      m0.load(a + 16 * (size_t)j + 4 * c);
+      m1.load(a + 16 * (size_t)(j + 1) + 4 * c);
+      const double4 u = *reinterpret_cast<const double4 *>(x + 4 * (size_t)k0);
+      const double4 v = *reinterpret_cast<const double4 *>(x + 4 * (size_t)k1);
+      double p[4], q[4];
+      m0.get(p);
+      m1.get(q);
+      acc = acc + p[0] * u.x; acc = acc + p[1] * u.y; acc = acc + p[2] * u.z; acc = acc + p[3] * u.w;
+      acc = acc + q[0] * v.x; acc = acc + q[1] * v.y; acc = acc + q[2] * v.z; acc = acc + q[3] * v.w;
+    }
+    if (j < j1) {
+      spmv_row<T> m0;
+      m0.load(a + 16 * (size_t)j + 4 * c);
+      const double4 u = *reinterpret_cast<const double4 *>(x + 4 * (size_t)col[j]);
+      double p[4];
+      m0.get(p);
+      acc = acc + p[0] * u.x; acc = acc + p[1] * u.y; acc = acc + p[2] * u.z; acc = acc + p[3] * u.w;
+    }
+    y[4 * (size_t)r + c] = acc;
+    return;
+  }
+  constexpr uint32_t B = 8;   /* blocks in flight */
+  for (; j < j1; j += B) {
     uint32_t kk[B];
     spmv_row<T> m[B];
     double xc[B];   /* a component a lane */
