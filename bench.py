@@ -68,7 +68,8 @@ HBM_PEAK_GBS = 8000.0
 FP64_PEAK_GFLOPS = 78600.0
 # the kernel sources a traffic profile is valid for (hashed into the profile)
 KERNEL_SOURCES = ["kfun3d_amd/csrc/" + f for f in ("flux.hip", "fill.hip", "ilu.hip", "sptrsv.hip", "blas.hip",
-                                                   "spmv.hip", "jacobi.hip", "handoff.h", "sync.h", "kf_dev.h")]
+                                                   "spmv.hip", "jacobi.hip", "coarse_dev.h", "handoff.h", "sync.h",
+                                                   "kf_dev.h")]
 
 
 def alg_bytes(kind, N, E, S, Nf, nnzb, s):
@@ -90,12 +91,12 @@ def alg_bytes(kind, N, E, S, Nf, nnzb, s):
         "trsv_lower": E * (16 * s + 4) + 64 * N,  # lower blocks + cols; b in, x out
         "trsv_upper": (E + N) * (16 * s + 4) + 64 * N,
         "spmv": (N + 2 * E) * (16 * s + 4) + 64 * N,   # every block + col; x in, y out
-        # one Jacobi sweep (per launch), the compulsory bytes: the half's blocks + cols, row bounds and
-        # diagonal index, b (FP64) or y in, the new vector out, vectors in the sweep's precision (8 bytes
+        # one Jacobi sweep (per launch), the compulsory bytes: the half's blocks, a 16-byte record
+        # of columns and length a row, b (FP64) or y in, the new vector out, vectors in the sweep's precision (8 bytes
         # FP64, 4 otherwise); the old vector's gathers, the fused D^-1 y of the last forward sweep and
         # the FP64 store of the last backward one are not counted (a lower bound)
-        "jacobi_lower": E * (16 * s + 4) + 8 * N + 4 * N * (8 + (8 if s == 8 else 4)),
-        "jacobi_upper": (E + N) * (16 * s + 4) + 8 * N + 4 * N * 2 * (8 if s == 8 else 4),
+        "jacobi_lower": E * 16 * s + 16 * N + 4 * N * (8 + (8 if s == 8 else 4)),
+        "jacobi_upper": (E + N) * 16 * s + 16 * N + 4 * N * 2 * (8 if s == 8 else 4),
     }[kind]
 
 
