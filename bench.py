@@ -20,7 +20,7 @@ it.
 roofline: the kernel class that takes the most time in one profiled solve of
 the value path (HIP events on the context stream around every class,
 kf_profile; that solve also gives kernel_ms and kernel_share); achieved =
-its algorithmic bytes per launch (ALG_BYTES) / its average launch time over
+its algorithmic bytes per launch (alg_bytes) / its average launch time over
 the timed solves, which record events around that class only
 (kf_profile_only); traffic = the HBM
 bytes per launch from the committed FETCH_SIZE / WRITE_SIZE counter passes
@@ -72,9 +72,17 @@ KERNEL_SOURCES = ["kfun3d_amd/csrc/" + f for f in ("flux.hip", "fill.hip", "ilu.
                                                    "kf_dev.h")]
 
 
-def alg_bytes(kind, N, E, S, Nf, nnzb, s):
+# a mesh of at most FLUX_ONE_ROWS vertices has its edge fluxes formed by the
+# residual's own kernel, with 16 lanes to a vertex up to FLUX_WIDE_ROWS and 4
+# above (the lines of flux.hip)
+FLUX_ONE_ROWS = 32768
+FLUX_WIDE_ROWS = 12288
+
+
+def alg_bytes(kind, N, E, S, Nf, nnzb, s, copies=0):
     """Compulsory HBM bytes of one launch (each array moved once); s = bytes
-    per stored matrix value."""
+    per stored matrix value; copies = bytes per value of the factors' other
+    copies that the factorisation stores (ilu_copies)."""
     return {
         # idx 8E, normal+area 32E, LSQ terms 48E; xyz 24N, q 32N, r 32N, grad written + read 2*96N
         "residual": 88 * E + 280 * N,
@@ -85,9 +93,12 @@ def alg_bytes(kind, N, E, S, Nf, nnzb, s):
         "residual_gather": 40 * E + 32 * N,       # ent 8E, flux in 32E; r 32N
         # with iJacVec's combination (k_residual<false, true>): + base residual, state, base state 96N, cdt 8N
         "residual_fd": 40 * E + 136 * N,
+        # both in one kernel (k_flux_residual<P, false, true>): nbr | side 8E, normal 64E; xyz 24N, q 32N,
+        # grad 96N, r 32N; base residual, state, base state 96N, cdt 8N
+        "flux_residual_fd": 72 * E + 288 * N,
         "timestep": 40 * E + 40 * N,
         "fill": 40 * E + 40 * N + 16 * s * nnzb,
-        "ilu": 2 * 16 * s * nnzb + 4 * nnzb,
+        "ilu": (2 * s + copies) * 16 * nnzb + 4 * nnzb,
         "trsv_lower": E * (16 * s + 4) + 64 * N,  # lower blocks + cols; b in, x out
         "trsv_upper": (E + N) * (16 * s + 4) + 64 * N,
         "spmv": (N + 2 * E) * (16 * s + 4) + 64 * N,   # every block + col; x in, y out
@@ -103,8 +114,30 @@ def alg_bytes(kind, N, E, S, Nf, nnzb, s):
 PROFILE_TO_KIND = {"grad": "grad_mom", "edge_flux": "edge_flux", "residual": "residual_fd", "timestep": "timestep",
                    "fill": "fill", "ilu": "ilu", "trsv_lower": "trsv_lower", "trsv_upper": "trsv_upper",
                    "spmv": "spmv", "jacobi_lower": "jacobi_lower", "jacobi_upper": "jacobi_upper"}
+F32_KINDS = ("fill", "ilu")   # in FP32 with either single-precision mode
 MATRIX_KINDS = ("fill", "ilu", "trsv_lower", "trsv_upper", "spmv", "jacobi_lower", "jacobi_upper")
 TYPE = {"fp64": ("double", "double"), "fp32": ("float", "float"), "bf16": ("unsigned short", "float")}
+
+
+def profile_kind(dom, N):
+    """alg_bytes' kind of a kf_profile class on N vertices"""
+    if dom == "residual" and N <= FLUX_ONE_ROWS:
+        return "flux_residual_fd"
+    return PROFILE_TO_KIND[dom]
+
+
+def value_bytes(kind, prec):
+    """bytes per matrix value that a kernel of this kind moves"""
+    if kind not in MATRIX_KINDS or prec == "fp64":
+        return 8
+    return 4 if prec == "fp32" or kind in F32_KINDS else 2
+
+
+def ilu_copies(prec, sweeps):
+    """bytes per value that the factorisation stores beside the factors: the
+    BF16 copy, and the Jacobi sweeps' sliced copy in the stored type"""
+    stored = {"fp64": 8, "fp32": 4, "bf16": 2}[prec]
+    return (stored if prec == "bf16" else 0) + (stored if sweeps else 0)
 
 
 def jacobi_names(dom, prec, sweeps, held, multilevel=False):
@@ -123,16 +156,18 @@ def jacobi_names(dom, prec, sweeps, held, multilevel=False):
             for i in range(sweeps)]
 
 
-def kernel_name(dom, prec, held, fold):
-    """the rocprofv3 name of the kernel behind a kf_profile class (for the
-    forward sweep, the instantiation GMRES's inner steps launch)"""
+def kernel_name(dom, prec, held, fold, N):
+    """the rocprofv3 name of the kernel behind a kf_profile class on N
+    vertices (for the forward sweep, the instantiation GMRES's inner steps
+    launch)"""
     tm, tv = TYPE[prec]
     if dom == "trsv_upper":
         return "k_trsv_upper<%d, %s, %s>" % (held, tm, tv)
     if dom == "trsv_lower":
         return "k_trsv_lower<%d, %s, %s, %s>" % (held, tm, tv, "true" if fold else "false")
     if dom == "ilu":
-        return "k_ilu_rows<%s, %s>" % (("double", "true") if prec == "fp64" else ("float", "false"))
+        # the values, the exact sweep, and the type the copies are stored in
+        return "k_ilu_rows<%s, %s>" % ("double, true" if prec == "fp64" else "float, false", tm)
     if dom == "fill":
         return "k_fill<%s>" % ("double" if prec == "fp64" else "float")
     if dom == "spmv":
@@ -141,6 +176,8 @@ def kernel_name(dom, prec, held, fold):
         return "k_jac_lower_sl<%d, %s, %s, double, double, true>" % (held, tm, tv)
     if dom == "jacobi_upper":
         return "k_jac_upper_sl<%d, %s, %s, double>" % (held, tm, tv)
+    if dom == "residual" and N <= FLUX_ONE_ROWS:
+        return "k_flux_residual<%d, false, true>" % (16 if N <= FLUX_WIDE_ROWS else 4)
     return {"grad": "k_grad<true>", "edge_flux": "k_edge_flux<false>", "residual": "k_residual<false, true>",
             "timestep": "k_timestep"}[dom]
 
@@ -306,13 +343,12 @@ def roofline(prof, path, sizes, config, held, fold):
     nnzb = N + 2 * E
     dom = max((k for k in prof if k in PROFILE_TO_KIND), key=lambda k: prof[k][0])
     ms, n = prof[dom]
-    kind = PROFILE_TO_KIND[dom]
+    kind = profile_kind(dom, N)
     per = sweeps if kind in ("jacobi_lower", "jacobi_upper") else 1
-    s = {"fp64": 8, "fp32": 4, "bf16": 2}[prec] if kind in MATRIX_KINDS else 8
-    ab = alg_bytes(kind, N, E, S, Nf, nnzb, s)
+    ab = alg_bytes(kind, N, E, S, Nf, nnzb, value_bytes(kind, prec), ilu_copies(prec, sweeps))
     achieved = ab / (ms / (n * per) / 1e3) / 1e9
     name = jacobi_names(dom, prec, sweeps, held, parse_path(path)[2] > 0) if per > 1 else \
-        kernel_name(dom, prec, held, fold)
+        kernel_name(dom, prec, held, fold, N)
     traffic, src = measured_traffic(config, name)
     return {"kernel": name, "bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": achieved / HBM_PEAK_GBS, "traffic": traffic, "alg_bytes_per_launch": ab,
@@ -645,7 +681,7 @@ def traffic_profile(K, config, root, precs):
         multi = parse_path(prec)[2] > 0
         f = _pmc_means(os.path.join(root, "fetch_%s" % prec), "FETCH_SIZE", finest=multi)
         w = _pmc_means(os.path.join(root, "write_%s" % prec), "WRITE_SIZE", finest=multi)
-        s = {"fp64": 8, "fp32": 4, "bf16": 2}[parse_path(prec)[0]]
+        pp, sw = parse_path(prec)[:2]
         for k in sorted(set(f) & set(w)):
             base = k.split("<")[0]
             if base not in kinds:
@@ -659,13 +695,9 @@ def traffic_profile(K, config, root, precs):
                 continue   # the fine and the coarse factorisations share the persistent grid: not separable
             if multi and kind in ("jacobi_lower", "jacobi_upper"):
                 held = int(k.split("<")[1].split(",")[0])
-                pp, sw = parse_path(prec)[:2]
                 if k not in jacobi_names(kind, pp, sw, held, True):
                     continue   # a coarse level's sweeps (other instantiations of the same kernels)
-            ss = s if kind in MATRIX_KINDS else 8
-            if base in ("k_fill", "k_ilu_rows") and s != 8:
-                ss = 4   # the fill and the factorisation run in FP32 for both single-precision modes
-            ab = alg_bytes(kind, N, E, S, Nf, nnzb, ss)
+            ab = alg_bytes(kind, N, E, S, Nf, nnzb, value_bytes(kind, pp), ilu_copies(pp, sw))
             b = f[k][0] * 1024.0 * fscale + w[k][0] * 1024.0 * wscale
             if k in out["kernels"]:
                 continue
