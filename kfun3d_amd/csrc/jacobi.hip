@@ -527,14 +527,44 @@ __global__ __launch_bounds__(JAC_SMALL_WG) void k_jac_small_levels(kf_small_leve
   }
 }
 
-/* the sliced copy from the CSR factors (a quad per row, lane c copying
- * block row c) */
+/* the sliced copy's pattern, once per allocation: the columns, and the zeros
+ * of the empty slots (a quad per row, lane c writing block row c) */
+template <int K, typename TM>
+__global__ __launch_bounds__(JAC_WG) void k_jac_pattern(uint32_t N, uint32_t nslice,
+                                                        const uint32_t *__restrict__ rowptr,
+                                                        const uint32_t *__restrict__ col,
+                                                        const uint32_t *__restrict__ diag, TM *__restrict__ val,
+                                                        uint32_t *__restrict__ scol, uint4 *__restrict__ near)
+{
+  const uint32_t r = kf_xcd_block() * (JAC_WG / 4) + (threadIdx.x >> 2);
+  const int c = threadIdx.x & 3;
+  if (r >= N) return;
+  const uint32_t sl = r >> 4, q = r & 15u, j0 = rowptr[r], jd = diag[r], j1 = rowptr[r + 1];
+  const size_t nk = (size_t)nslice * K;
+  for (int part = 0; part < 2; part++) {
+    const uint32_t first = part ? jd + 1 : j0, n = part ? j1 - jd - 1 : jd - j0;
+    for (int k = 0; k < K; k++) {
+      const size_t slot = part * nk + (size_t)sl * K + k;
+      if ((uint32_t)k >= n) {
+        TM *o = val + (slot * 16 + q) * 16 + 4 * c;
+        o[0] = o[1] = o[2] = o[3] = TM(0);
+      }
+      if (c == 0 && !near) scol[slot * 16 + q] = (uint32_t)k < n ? col[first + k] : r;
+    }
+    if (c == 0 && near) {
+      uint32_t w[4] = {0u, 0u, 0u, n << 16};
+      for (uint32_t k = 0; k < n && k < 7u; k++) w[k / 2] |= ((col[first + k] - r) & 0xffffu) << (k & 1u ? 16 : 0);
+      near[(size_t)part * nslice * 16 + r] = make_uint4(w[0], w[1], w[2], w[3]);
+    }
+  }
+}
+
+/* the sliced copy's values from the CSR factors (a quad per row, lane c
+ * copying block row c) */
 template <int K, typename TM>
 __global__ __launch_bounds__(JAC_WG) void k_jac_pack(uint32_t N, uint32_t nslice, const uint32_t *__restrict__ rowptr,
-                                                     const uint32_t *__restrict__ col,
                                                      const uint32_t *__restrict__ diag, const TM *__restrict__ a,
-                                                     TM *__restrict__ val, uint32_t *__restrict__ scol,
-                                                     uint4 *__restrict__ near)
+                                                     TM *__restrict__ val)
 {
   const uint32_t r = kf_xcd_block() * (JAC_WG / 4) + (threadIdx.x >> 2);
   const int c = threadIdx.x & 3;
@@ -544,25 +574,14 @@ __global__ __launch_bounds__(JAC_WG) void k_jac_pack(uint32_t N, uint32_t nslice
   for (int part = 0; part < 2; part++) {
     const uint32_t first = part ? jd + 1 : j0, n = part ? j1 - jd - 1 : jd - j0;
     TM *pv = val + (size_t)part * nk * 256;
-    uint32_t *pc = scol + (size_t)part * nk * 16;
     for (int k = 0; k < K; k++) {
-      const size_t slot = (size_t)sl * K + k;
-      TM *o = pv + (slot * 16 + q) * 16 + 4 * c;
-      if ((uint32_t)k < n) {
-        const TM *src = a + 16 * (size_t)(first + k) + 4 * c;
-        o[0] = src[0];
-        o[1] = src[1];
-        o[2] = src[2];
-        o[3] = src[3];
-      } else {
-        o[0] = o[1] = o[2] = o[3] = TM(0);
-      }
-      if (c == 0 && !near) pc[slot * 16 + q] = (uint32_t)k < n ? col[first + k] : r;
-    }
-    if (c == 0 && near) {
-      uint32_t w[4] = {0u, 0u, 0u, n << 16};
-      for (uint32_t k = 0; k < n && k < 7u; k++) w[k / 2] |= ((col[first + k] - r) & 0xffffu) << (k & 1u ? 16 : 0);
-      near[(size_t)part * nslice * 16 + r] = make_uint4(w[0], w[1], w[2], w[3]);
+      if ((uint32_t)k >= n) break;
+      TM *o = pv + (((size_t)sl * K + k) * 16 + q) * 16 + 4 * c;
+      const TM *src = a + 16 * (size_t)(first + k) + 4 * c;
+      o[0] = src[0];
+      o[1] = src[1];
+      o[2] = src[2];
+      o[3] = src[3];
     }
   }
   TM *o = val + 2 * nk * 256 + ((size_t)sl * 16 + q) * 16 + 4 * c;
@@ -716,30 +735,36 @@ static void jacobi_solve_sl(kf_ctx *c, const TM *a, const TB *b, double *x, TV *
 }
 
 template <typename TM>
+static void jsl_pattern_as(kf_ctx *c, uint32_t nslice)
+{
+  const kf_dv &d = c->d;
+  const dim3 grid(kf_blocks_for(d.N, JAC_WG / 4)), block(JAC_WG);
+  if (c->jsl_k == 7)
+    hipLaunchKernelGGL((k_jac_pattern<7, TM>), grid, block, 0, c->stream, d.N, nslice, d.rowptr, d.col, d.diag,
+                       (TM *)c->jsl_val, c->jsl_col, (uint4 *)c->jsl_near);
+  else
+    hipLaunchKernelGGL((k_jac_pattern<8, TM>), grid, block, 0, c->stream, d.N, nslice, d.rowptr, d.col, d.diag,
+                       (TM *)c->jsl_val, c->jsl_col, (uint4 *)NULL);
+  KF_LAUNCH_CHECK();
+}
+
+template <typename TM>
 static void jsl_pack_as(kf_ctx *c, const TM *a, uint32_t nslice)
 {
   const kf_dv &d = c->d;
   const dim3 grid(kf_blocks_for(d.N, JAC_WG / 4)), block(JAC_WG);
   if (c->jsl_k == 7)
-    hipLaunchKernelGGL((k_jac_pack<7, TM>), grid, block, 0, c->stream, d.N, nslice, d.rowptr, d.col, d.diag, a,
-                       (TM *)c->jsl_val, c->jsl_col, (uint4 *)c->jsl_near);
+    hipLaunchKernelGGL((k_jac_pack<7, TM>), grid, block, 0, c->stream, d.N, nslice, d.rowptr, d.diag, a,
+                       (TM *)c->jsl_val);
   else
-    hipLaunchKernelGGL((k_jac_pack<8, TM>), grid, block, 0, c->stream, d.N, nslice, d.rowptr, d.col, d.diag, a,
-                       (TM *)c->jsl_val, c->jsl_col, (uint4 *)NULL);
+    hipLaunchKernelGGL((k_jac_pack<8, TM>), grid, block, 0, c->stream, d.N, nslice, d.rowptr, d.diag, a,
+                       (TM *)c->jsl_val);
   KF_LAUNCH_CHECK();
 }
 
-static void jsl_pack_now(kf_ctx *c, uint32_t nslice)
-{
-  if (c->jsl_esize == 8) jsl_pack_as<double>(c, c->a64, nslice);
-  else if (c->jsl_esize == 4) jsl_pack_as<float>(c, c->a32, nslice);
-  else jsl_pack_as<uint16_t>(c, c->abf, nslice);
-}
-
-/* the sliced copy's memory in the context's precision.  A new one is packed
- * from whatever the factor array holds: that writes the columns and the
- * zeros of the empty slots, which the factorisation leaves alone when it
- * writes the copy itself (ilu.hip). */
+/* the sliced copy's memory in the context's precision; a new one has its
+ * columns and the zeros of its empty slots, which neither the factorisation
+ * (ilu.hip) nor k_jac_pack writes */
 void *kf_jac_slices(kf_ctx *c, uint32_t *K, uint32_t *nslice)
 {
   const uint32_t ns = (c->d.N + 15) / 16;
@@ -758,7 +783,9 @@ void *kf_jac_slices(kf_ctx *c, uint32_t *K, uint32_t *nslice)
     KF_CHECK(hipMalloc(&c->jsl_val, (2 * nk + ns) * 256 * es));
     c->jsl_esize = es;
     c->jsl_fresh = 0;
-    jsl_pack_now(c, ns);
+    if (es == 8) jsl_pattern_as<double>(c, ns);
+    else if (es == 4) jsl_pattern_as<float>(c, ns);
+    else jsl_pattern_as<uint16_t>(c, ns);
   }
   *K = c->jsl_k;
   *nslice = ns;
@@ -776,7 +803,9 @@ static jsl_view jsl_pack(kf_ctx *c)
   v.col = c->jsl_col;
   v.near = (const uint4 *)c->jsl_near;
   if (!c->jsl_fresh) {
-    jsl_pack_now(c, nslice);
+    if (c->jsl_esize == 8) jsl_pack_as<double>(c, c->a64, nslice);
+    else if (c->jsl_esize == 4) jsl_pack_as<float>(c, c->a32, nslice);
+    else jsl_pack_as<uint16_t>(c, c->abf, nslice);
     c->jsl_fresh = 1;
   }
   return v;
