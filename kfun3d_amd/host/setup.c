@@ -537,18 +537,22 @@ void kf_build_sell(const GEOMETRY *g, const kf_prep *p, kf_sell *out)
   out->wx = wx; out->wy = wy; out->wz = wz;
 }
 
-/* own[e]: the side whose end has edge e.  deg: how many each vertex then has.
- * Returns the entries of the sliced lists. */
-static size_t edge_slots(size_t N, size_t E, const uint32_t *n0, const uint32_t *n1, const unsigned char *own,
-                         uint32_t *deg)
+/* len[s]: the longest list of slice s's vertices when edge e is in the list of
+ * its end own[e] (NULL: of its n0).  Returns the entries of the sliced lists. */
+static size_t edge_slots(const kf_prep *p, const unsigned char *own, uint32_t *len)
 {
-  memset(deg, 0, N * sizeof(uint32_t));
-  for (size_t e = 0; e < E; e++) deg[own[e] ? n1[e] : n0[e]]++;
+  const size_t N = p->N, nslice = (N + 63) / 64;
   size_t rows = 0;
-  for (size_t s = 0; s < N; s += 64) {
+#pragma omp parallel for schedule(static) reduction(+ : rows)
+  for (size_t s = 0; s < nslice; s++) {
     uint32_t l = 0;
-    for (size_t v = s; v < N && v < s + 64; v++)
-      if (deg[v] > l) l = deg[v];
+    for (size_t v = s * 64; v < N && v < s * 64 + 64; v++) {
+      uint32_t d = 0;
+      for (uint32_t k = p->vptr[v]; k < p->vptr[v + 1]; k++)
+        d += (own ? own[p->vent[k] >> 1] : 0u) == (p->vent[k] & 1u);
+      if (d > l) l = d;
+    }
+    len[s] = l;
     rows += l;
   }
   return rows * 64;
@@ -557,44 +561,55 @@ static size_t edge_slots(size_t N, size_t E, const uint32_t *n0, const uint32_t 
 /* The edges' places, by one of the two ends: its n0, or the end that has fewer
  * edges so far where that fills the slices better (on a lattice numbered along
  * its axes every vertex is the n0 of as many edges as the next; on other
- * numberings one is the n0 of none of its edges, the next of all). */
+ * numberings one is the n0 of none of its edges, the next of all).  The
+ * second rule takes the edges one after another, and only where the first
+ * leaves an eighth of the places empty; all else is by slices, in parallel. */
 size_t kf_place_edges(const GEOMETRY *g, const kf_prep *p, uint32_t *pos)
 {
-  const size_t N = p->N, E = g->e->sz;
-  const uint32_t *n0 = g->e->eptr->n0, *n1 = g->e->eptr->n1;
-  const size_t nslice = (N + 63) / 64;
-  unsigned char *own = (unsigned char *)kf_xcalloc(E + 1, 1);
-  uint32_t *deg = (uint32_t *)kf_xcalloc(N + 1, sizeof(uint32_t));
-  size_t n = edge_slots(N, E, n0, n1, own, deg);
+  const size_t N = p->N, E = g->e->sz, nslice = (N + 63) / 64;
+  uint32_t *len = (uint32_t *)kf_xcalloc(nslice + 1, sizeof(uint32_t));
+  unsigned char *own = NULL;
+  size_t n = edge_slots(p, NULL, len);
   if (8 * n > 9 * E) {
-    memset(deg, 0, N * sizeof(uint32_t));
+    const uint32_t *n0 = g->e->eptr->n0, *n1 = g->e->eptr->n1;
+    uint32_t *deg = (uint32_t *)kf_xcalloc(N + 1, sizeof(uint32_t));
+    uint32_t *even = (uint32_t *)kf_xcalloc(nslice + 1, sizeof(uint32_t));
+    own = (unsigned char *)kf_xcalloc(E + 1, 1);
     for (size_t e = 0; e < E; e++) {
       own[e] = deg[n1[e]] < deg[n0[e]];
       deg[own[e] ? n1[e] : n0[e]]++;
     }
-    const size_t even = edge_slots(N, E, n0, n1, own, deg);
-    if (even >= n) {
-      memset(own, 0, E);
-      edge_slots(N, E, n0, n1, own, deg);
-    } else n = even;
-  }
-  size_t row = 0;
-  for (size_t s = 0; s < nslice; s++) {
-    uint32_t l = 0;
-    for (size_t v = s * 64; v < N && v < s * 64 + 64; v++) {
-      size_t at = row * 64 + (v & 63);
-      for (uint32_t k = p->vptr[v]; k < p->vptr[v + 1]; k++) {
-        const uint32_t e = p->vent[k] >> 1;
-        if (own[e] != (p->vent[k] & 1u)) continue;
-        pos[e] = (uint32_t)at;
-        at += 64;
-      }
-      if (deg[v] > l) l = deg[v];
+    free(deg);
+    const size_t ne = edge_slots(p, own, even);
+    uint32_t *drop = even;
+    if (ne >= n) {
+      free(own);
+      own = NULL;
+    } else {
+      n = ne;
+      drop = len;
+      len = even;
     }
-    row += l;
+    free(drop);
   }
+  size_t *row = (size_t *)kf_xmalloc((nslice + 1) * sizeof(size_t)), rows = 0;
+  for (size_t s = 0; s < nslice; s++) {
+    row[s] = rows;
+    rows += len[s];
+  }
+#pragma omp parallel for schedule(static)
+  for (size_t v = 0; v < N; v++) {
+    size_t at = row[v >> 6] * 64 + (v & 63);
+    for (uint32_t k = p->vptr[v]; k < p->vptr[v + 1]; k++) {
+      const uint32_t e = p->vent[k] >> 1;
+      if ((own ? own[e] : 0u) != (p->vent[k] & 1u)) continue;
+      pos[e] = (uint32_t)at;
+      at += 64;
+    }
+  }
+  free(row);
+  free(len);
   free(own);
-  free(deg);
   return n;
 }
 
