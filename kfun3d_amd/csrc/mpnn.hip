@@ -696,9 +696,9 @@ __device__ __forceinline__ void mp_update_bwd(const float dh[16], uint32_t n, bo
   gv = mp_tile_mm<32, 32>(T, T + 64 * MP_TS, gv);
 }
 
-#define MP_BWD_LDS (MP_TW * 4096)   /* bytes: the wavefronts' sums, or their 3 tiles of 2304 */
-#define MP_BWD_TILES (96 * MP_TS)   /* values: a wavefront's tiles */
-static_assert(MP_TW * MP_BWD_TILES * 2 <= 2 * MP_BWD_LDS, "the tiles fit");
+#define MP_BWD_TILES (96 * MP_TS)   /* values: a wavefront's 3 tiles of 32 rows */
+#define MP_BWD_LDS (MP_TW * MP_BWD_TILES * 2)   /* bytes: the wavefronts' tiles, and after them their sums */
+static_assert(MP_BWD_LDS >= MP_TW * 4096, "mp_wsum's 1024 floats a wavefront fit");
 
 /* Backward of the correction given gv = dL/d delta (N x 4, FP32) and z:
  *   dOP1_v = [g_v z_v^T | (g_v / deg v) zs_v^T]       zs_v = sum_u z_u
@@ -715,7 +715,7 @@ __global__ __launch_bounds__(MP_RB, 2) void k_mp_head_bwd(kf_dv d, uint32_t chun
                                                        float *__restrict__ dhn, float *__restrict__ dm,
                                                        float *__restrict__ part)
 {
-  __shared__ __align__(16) unsigned char lds[2 * MP_BWD_LDS];
+  __shared__ __align__(16) unsigned char lds[MP_BWD_LDS];
   short *T = reinterpret_cast<short *>(lds) + (threadIdx.x >> 6) * MP_BWD_TILES;
   float *sh = reinterpret_cast<float *>(lds);
   const uint32_t li = threadIdx.x & 31u, hf = (threadIdx.x >> 5) & 1u;
@@ -835,7 +835,7 @@ __global__ __launch_bounds__(MP_RB, 2) void k_mp_round_bwd(uint32_t N, uint32_t 
                                                         float *__restrict__ dhn, float *__restrict__ dm,
                                                         float *__restrict__ part)
 {
-  __shared__ __align__(16) unsigned char lds[2 * MP_BWD_LDS];
+  __shared__ __align__(16) unsigned char lds[MP_BWD_LDS];
   short *T = reinterpret_cast<short *>(lds) + (threadIdx.x >> 6) * MP_BWD_TILES;
   float *sh = reinterpret_cast<float *>(lds);
   const uint32_t li = threadIdx.x & 31u, h4 = (threadIdx.x & 32u) >> 3;
