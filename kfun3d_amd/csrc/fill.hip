@@ -194,7 +194,7 @@ __device__ __forceinline__ void freestream_block(T xn, T yn, T zn, T U, T V, T p
  * edges ascend with their ends. */
 template <typename T>
 struct fill_rows {
-  static constexpr int PC = sizeof(T), STRIDE = 9;   /* 16-byte pieces of a block, of a row */
+  static constexpr int STRIDE = 9;   /* 16-byte pieces of a row */
   float4 w[64 * STRIDE];
 };
 
