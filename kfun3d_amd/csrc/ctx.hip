@@ -23,11 +23,6 @@ static T *dupload(const T *h, size_t n)
   return p;
 }
 
-static void dfree(void *p)
-{
-  if (p) KF_CHECK(hipFree(p));
-}
-
 /* launch-shape knobs of the level-scheduled kernels (tuning only) */
 static void ctx_knobs(kf_ctx *c)
 {
@@ -216,10 +211,6 @@ extern "C" void kf_ctx_create(GEOMETRY *g, const kf_prep *p, const kf_options *o
   kf_sell_records(c, ne);
   kf_phase("places of the fluxes, records");
   kf_grad_setup(c);
-  /* the lists' neighbours and edges were for these two: the records hold both */
-  dfree(d.sell_nbr);
-  dfree(d.sell_ent);
-  d.sell_nbr = d.sell_ent = NULL;
   kf_phase("LSQ moments (device)");
 
   /* boundary */
@@ -284,6 +275,11 @@ extern "C" void kf_ctx_create(GEOMETRY *g, const kf_prep *p, const kf_options *o
 
 static void kf_unbind_ctx(kf_ctx *c);
 
+static void dfree(void *p)
+{
+  if (p) KF_CHECK(hipFree(p));
+}
+
 /* A context holding only a block matrix -- the coarse level of the
  * two-level preconditioner: pattern, plans, tickets, values and factors.
  * It shares the parent's stream (so its launches are ordered with the
@@ -329,7 +325,7 @@ extern "C" void kf_ctx_destroy(GEOMETRY *g)
     KF_CHECK(hipStreamDestroy(c->fstream));
   }
   kf_dv &d = c->d;
-  void *ptrs[] = {d.en, d.egeo, d.edge_pos, d.sell_geo, d.sell_pos, d.x, d.y, d.z, d.xyzw, d.sell_ptr, d.deg,
+  void *ptrs[] = {d.en, d.egeo, d.edge_pos, d.sell_geo, d.sell_pos, d.x, d.y, d.z, d.xyzw, d.sell_ptr, d.deg, d.sell_nbr, d.sell_ent,
                   d.sell_blk, d.sell_wx, d.sell_wy, d.sell_wz, d.lsq, d.sell_nbs, d.sf0, d.sf1, d.sf2, d.color, d.sfptr, d.sfent, d.snx, d.sny,
                   d.snz, d.snptr, d.snent, d.fnx, d.fny, d.fnz, d.fnptr, d.fnent, d.rowptr, d.col, d.diag, d.eres,
                   d.red, d.scal, d.err, c->lrows, c->rdone,

@@ -327,7 +327,7 @@ __global__ __launch_bounds__(256) void k_grad(kf_dv d, const double *__restrict_
       }
     } else {
       for (; k < deg; k++, idx += 64) {
-        const uint32_t nb = kf_sell_nbr(d, idx);
+        const uint32_t nb = d.sell_nbr[idx];
         grad_add(a0, a1, a2, qs, ld4(q, nb), d.sell_wx[idx], d.sell_wy[idx], d.sell_wz[idx]);
       }
     }
@@ -814,7 +814,7 @@ __global__ __launch_bounds__(256) void k_timestep(kf_dv d, const double *__restr
   size_t idx = (size_t)d.sell_ptr[v >> 6] * 64u + (v & 63u);
   const d4 qv = ld4(q, v);
   for (uint32_t k = 0; k < deg; k++, idx += 64) {
-    const d4 qn = ld4(q, kf_sell_nbr(d, idx));
+    const d4 qn = ld4(q, d.sell_nbs[idx] & 0x7fffffffu);
     const kf_egeo eg = kf_edge_geo(d.sell_geo, idx);
     acc = acc + spectral_term(qv, qn, eg.xn, eg.yn, eg.zn, eg.ln);   /* the same from either end */
   }

@@ -9,12 +9,10 @@
  *             slice s = v / 64, lane l = v % 64, owns entries
  *             (sell_ptr[s] + k) * 64 + l for k < deg[v], ascending edge id
  *             (the order the reference's one-thread edge loops accumulate in):
- *               sell_nbs  neighbour | side << 31        (u32, side 1: v is n1)
- *               sell_pos  place of the edge's flux << 1 | side (u32)
+ *               sell_nbr  neighbour vertex              (u32)
+ *               sell_ent  edge << 1 | side              (u32, side 1: v is n1)
  *               sell_blk  BSR block of (v, neighbour)   (u32)
- *               sell_geo  the edge's normal and area    (4 x f64)
- *               sell_w*   LSQ term of the edge seen from v, 3 x f64 SoA (not
- *                         kept where the vertices' moments reproduce it)
+ *               sell_w*   LSQ term of the edge seen from v, 3 x f64 SoA
  *   BSR       rowptr[N+1], col[nnzb], diag[N]; blocks of 16 values row-major,
  *             FP64 (a64) or FP32 (a32); BF16 factor copy (abf)
  *   levels    rows in level order of the lower (L) / upper (U) triangle,
@@ -74,8 +72,7 @@ struct kf_dv {
   double *x, *y, *z;
   double *xyzw;                 /* (x, y, z, 0) per vertex: one 32-byte gather for the edge kernel */
   uint32_t *sell_ptr, *deg;
-  uint32_t *sell_nbr, *sell_ent;   /* of the setup kernels only (NULL after them) */
-  uint32_t *sell_blk;
+  uint32_t *sell_nbr, *sell_ent, *sell_blk;
   double *sell_wx, *sell_wy, *sell_wz;   /* the LSQ terms per incidence (NULL once lsq is verified) */
   double *lsq;                  /* 7 x N: per-vertex LSQ moments w00 w01 w02 w11 w12 w22 w33 (one array each) */
   uint32_t *sell_nbs;           /* neighbour | side << 31 per incidence */
@@ -93,9 +90,6 @@ struct kf_dv {
   double *red, *scal;
   uint32_t *err;
 };
-
-/* the neighbour of the incidence at place idx of the sliced lists */
-__device__ __forceinline__ uint32_t kf_sell_nbr(const kf_dv &d, size_t idx) { return d.sell_nbs[idx] & 0x7fffffffu; }
 
 /* per-kernel HIP-event timing on the context stream (kf_profile) */
 enum kf_prof_id { KP_GRAD, KP_EDGE, KP_RES, KP_TSTEP, KP_FILL, KP_ILU, KP_TRSV_L, KP_TRSV_U, KP_SPMV, KP_JAC_L, KP_JAC_U,

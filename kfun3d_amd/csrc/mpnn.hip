@@ -392,12 +392,12 @@ __global__ __launch_bounds__(MP_RB) void k_mp_edge_vectors(kf_dv d, float4 *__re
   if (v >= d.N) return;
   size_t idx = (size_t)d.sell_ptr[v >> 6] * 64u + (v & 63u);
   for (uint32_t k = 0; k < d.deg[v]; k++, idx += 64) {
-    const uint32_t at = d.sell_pos[idx], u = kf_sell_nbr(d, idx);
+    const uint32_t ent = d.sell_ent[idx], u = d.sell_nbr[idx];
     const kf_egeo eg = kf_edge_geo(d.sell_geo, idx);
-    const double ar = (at & 1u) ? -eg.ln : eg.ln;
+    const double ar = (ent & 1u) ? -eg.ln : eg.ln;
     const size_t ui = (size_t)d.sell_ptr[u >> 6] * 64u + (u & 63u);
     uint32_t kr = 0;
-    while (kr + 1 < d.deg[u] && d.sell_pos[ui + 64 * (size_t)kr] != (at ^ 1u)) kr++;   /* u holds the other side */
+    while (kr + 1 < d.deg[u] && d.sell_ent[ui + 64 * (size_t)kr] != (ent ^ 1u)) kr++;   /* u holds the other side */
     ev[idx] = make_float4((float)(eg.xn * ar), (float)(eg.yn * ar), (float)(eg.zn * ar), __uint_as_float(kr));
   }
   ideg[v] = 1.0f / (float)max(d.deg[v], 1u);
@@ -455,7 +455,7 @@ __global__ __launch_bounds__(MP_RB) void k_mp_message(kf_dv d, const float4 *__r
 #pragma unroll
     for (int i = 0; i < 4; i++) {
       const size_t idx = base + 64 * (size_t)min(k0 + i, deg - 1);
-      u[i] = kf_sell_nbr(d, idx);
+      u[i] = d.sell_nbr[idx];
       e[i] = ev[idx];
     }
 #pragma unroll
@@ -518,7 +518,7 @@ __global__ __launch_bounds__(MP_RB) void k_mp_message_bwd(kf_dv d, uint32_t chun
 #pragma unroll
       for (int i = 0; i < 4; i++) {
         const size_t idx = base + 64 * (size_t)min(k0 + i, deg - 1);
-        u[i] = kf_sell_nbr(d, idx);
+        u[i] = d.sell_nbr[idx];
         e[i] = ev[idx];
       }
       const uint32_t own = pos[((size_t)v * words + (k0 >> 3)) * 8 + s] >> (4 * (k0 & 4u));
@@ -614,7 +614,7 @@ __global__ __launch_bounds__(MP_RB) void k_mp_apply(kf_dv d, const float4 *__res
   };
   uint32_t k = 0;
   for (; k + 1 < deg; k += 2, idx += 128) {
-    const uint32_t ua = kf_sell_nbr(d, idx), ub = kf_sell_nbr(d, idx + 64);
+    const uint32_t ua = d.sell_nbr[idx], ub = d.sell_nbr[idx + 64];
     const float4 ea = ev[idx], eb = ev[idx + 64];
     const float4 za = ld4(z, ua), zb = ld4(z, ub);
     const float4 *pa = (const float4 *)(OPQ + (size_t)ua * MP_H), *pb = (const float4 *)(OPQ + (size_t)ub * MP_H);
@@ -623,7 +623,7 @@ __global__ __launch_bounds__(MP_RB) void k_mp_apply(kf_dv d, const float4 *__res
     sum(eb, zb, qb);
   }
   if (k < deg) {
-    const uint32_t ua = kf_sell_nbr(d, idx);
+    const uint32_t ua = d.sell_nbr[idx];
     const float4 ea = ev[idx], za = ld4(z, ua);
     const float4 *pa = (const float4 *)(OPQ + (size_t)ua * MP_H);
     const float4 qa[4] = {pa[0], pa[1], pa[2], pa[3]};
@@ -741,7 +741,7 @@ __global__ __launch_bounds__(MP_RB, 2) void k_mp_head_bwd(kf_dv d, uint32_t chun
 #pragma unroll
       for (int i = 0; i < 4; i++) {
         const size_t idx = base + 64 * (size_t)min(k0 + i, deg - 1);
-        u[i] = kf_sell_nbr(d, idx);
+        u[i] = d.sell_nbr[idx];
         e[i] = ev[idx];
       }
 #pragma unroll
