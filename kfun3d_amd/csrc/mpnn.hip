@@ -697,8 +697,11 @@ __device__ __forceinline__ void mp_update_bwd(const float dh[16], uint32_t n, bo
 }
 
 #define MP_BWD_TILES (96 * MP_TS)   /* values: a wavefront's 3 tiles of 32 rows */
-#define MP_BWD_LDS (MP_TW * MP_BWD_TILES * 2)   /* bytes: the wavefronts' tiles, and after them their sums */
-static_assert(MP_BWD_LDS >= MP_TW * 4096, "mp_wsum's 1024 floats a wavefront fit");
+/* bytes: 6,912 a wavefront for its tiles, and after them 4,096 for its sums.
+ * With no more than the tiles need the compiler's code for k_mp_head_bwd is
+ * another, and slower (331,776 vertices: 147 against 135 us). */
+#define MP_BWD_LDS (MP_TW * 8192)
+static_assert(MP_BWD_LDS >= MP_TW * MP_BWD_TILES * 2 && MP_BWD_LDS >= MP_TW * 4096, "tiles and sums fit");
 
 /* Backward of the correction given gv = dL/d delta (N x 4, FP32) and z:
  *   dOP1_v = [g_v z_v^T | (g_v / deg v) zs_v^T]       zs_v = sum_u z_u
