@@ -196,7 +196,7 @@ extern "C" void kf_ctx_create(GEOMETRY *g, const kf_prep *p, const kf_options *o
   d.sell_ptr = dupload(sptr, nslice + 1);
   d.deg = dupload(deg, N);
   d.sell_nbr = dupload(nbr, ne);
-  d.sell_ent = dupload(ent, ne);
+  d.sell_pos = dupload(ent, ne);   /* kf_sell_records puts the place in the edge's stead */
   d.sell_blk = dupload(blk, ne);
   d.sell_wx = dupload(wx, ne);
   d.sell_wy = dupload(wy, ne);
@@ -325,7 +325,7 @@ extern "C" void kf_ctx_destroy(GEOMETRY *g)
     KF_CHECK(hipStreamDestroy(c->fstream));
   }
   kf_dv &d = c->d;
-  void *ptrs[] = {d.en, d.egeo, d.edge_pos, d.sell_geo, d.sell_pos, d.x, d.y, d.z, d.xyzw, d.sell_ptr, d.deg, d.sell_nbr, d.sell_ent,
+  void *ptrs[] = {d.en, d.egeo, d.edge_pos, d.sell_geo, d.sell_pos, d.x, d.y, d.z, d.xyzw, d.sell_ptr, d.deg, d.sell_nbr,
                   d.sell_blk, d.sell_wx, d.sell_wy, d.sell_wz, d.lsq, d.sell_nbs, d.sf0, d.sf1, d.sf2, d.color, d.sfptr, d.sfent, d.snx, d.sny,
                   d.snz, d.snptr, d.snent, d.fnx, d.fny, d.fnz, d.fnptr, d.fnent, d.rowptr, d.col, d.diag, d.eres,
                   d.red, d.scal, d.err, c->lrows, c->rdone,

@@ -113,7 +113,7 @@ __global__ __launch_bounds__(256) void k_lsq_moments(kf_dv d, double *__restrict
   /* w11, w12: src/weights.c:173-232 */
   for (uint32_t k = 0; k < deg; k++) {
     const size_t idx = base + 64 * (size_t)k;
-    const bool side1 = d.sell_ent[idx] & 1u;
+    const bool side1 = d.sell_pos[idx] & 1u;
     const d4 cn = ld4(d.xyzw, d.sell_nbr[idx]);
     double dx, dy, dz;
     edge_vector(cv, cn, side1, dx, dy, dz);
@@ -133,7 +133,7 @@ __global__ __launch_bounds__(256) void k_lsq_moments(kf_dv d, double *__restrict
   /* w22: src/weights.c:103-170 */
   for (uint32_t k = 0; k < deg; k++) {
     const size_t idx = base + 64 * (size_t)k;
-    const bool side1 = d.sell_ent[idx] & 1u;
+    const bool side1 = d.sell_pos[idx] & 1u;
     const d4 cn = ld4(d.xyzw, d.sell_nbr[idx]);
     double dx, dy, dz;
     edge_vector(cv, cn, side1, dx, dy, dz);
@@ -180,7 +180,7 @@ __global__ __launch_bounds__(256) void k_lsq_check(kf_dv d, const double *__rest
   bool ok = true;
   for (uint32_t k = 0; k < deg; k++) {
     const size_t idx = base + 64 * (size_t)k;
-    const bool side1 = d.sell_ent[idx] & 1u;
+    const bool side1 = d.sell_pos[idx] & 1u;
     const d4 cn = ld4(d.xyzw, d.sell_nbr[idx]);
     double dx, dy, dz, tx, ty, tz;
     edge_vector(cv, cn, side1, dx, dy, dz);
@@ -192,12 +192,11 @@ __global__ __launch_bounds__(256) void k_lsq_check(kf_dv d, const double *__rest
   if (!ok) atomicOr(bad, 1u);
 }
 
-/* neighbour | side << 31, the edge's (unit normal, area) and the place of its
- * flux << 1 | side of every incidence, in sliced-ELL order (zeros in its
- * padding): the vertex kernels read them as dense lines, where the per-edge
- * records are gathers of 32 bytes */
-__global__ __launch_bounds__(256) void k_sell_records(kf_dv d, uint32_t *__restrict__ nbs, double *__restrict__ geo,
-                                                      uint32_t *__restrict__ spos)
+/* neighbour | side << 31, the edge's (unit normal, area) and, over its number
+ * << 1 | side, the place of its flux << 1 | side, of every incidence in
+ * sliced-ELL order (zeros in its padding): the vertex kernels read them as
+ * dense lines, where the per-edge records are gathers of 32 bytes */
+__global__ __launch_bounds__(256) void k_sell_records(kf_dv d, uint32_t *__restrict__ nbs, double *__restrict__ geo)
 {
   const uint32_t v = blockIdx.x * 256u + threadIdx.x, slice = v >> 6;
   if (slice >= d.nslice) return;
@@ -207,13 +206,13 @@ __global__ __launch_bounds__(256) void k_sell_records(kf_dv d, uint32_t *__restr
     uint32_t s = 0, at = 0;
     kf_egeo eg = {0.0, 0.0, 0.0, 0.0};
     if (k < deg) {
-      const uint32_t ent = d.sell_ent[idx];
+      const uint32_t ent = d.sell_pos[idx];
       eg = kf_edge_geo(d.egeo, ent >> 1);
       s = d.sell_nbr[idx] | ent << 31;
       at = d.edge_pos[ent >> 1] << 1 | (ent & 1u);
     }
     nbs[idx] = s;
-    spos[idx] = at;
+    d.sell_pos[idx] = at;
     st4(geo, idx, eg.xn, eg.yn, eg.zn, eg.ln);
   }
 }
@@ -222,11 +221,9 @@ void kf_sell_records(kf_ctx *c, size_t ne)
 {
   kf_dv &d = c->d;
   KF_CHECK(hipMalloc((void **)&d.sell_nbs, (ne + 1) * sizeof(uint32_t)));
-  KF_CHECK(hipMalloc((void **)&d.sell_pos, (ne + 1) * sizeof(uint32_t)));
   KF_CHECK(hipMalloc((void **)&d.sell_geo, (4 * ne + 4) * sizeof(double)));
   if (!d.N) return;
-  hipLaunchKernelGGL(k_sell_records, dim3(kf_blocks_for(d.N, 256)), dim3(256), 0, c->stream, d, d.sell_nbs, d.sell_geo,
-                     d.sell_pos);
+  hipLaunchKernelGGL(k_sell_records, dim3(kf_blocks_for(d.N, 256)), dim3(256), 0, c->stream, d, d.sell_nbs, d.sell_geo);
   KF_LAUNCH_CHECK();
   KF_CHECK(hipStreamSynchronize(c->stream));
 }

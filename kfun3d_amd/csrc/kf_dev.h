@@ -10,9 +10,12 @@
  *             (sell_ptr[s] + k) * 64 + l for k < deg[v], ascending edge id
  *             (the order the reference's one-thread edge loops accumulate in):
  *               sell_nbr  neighbour vertex              (u32)
- *               sell_ent  edge << 1 | side              (u32, side 1: v is n1)
+ *               sell_nbs  neighbour | side << 31        (u32, side 1: v is n1)
+ *               sell_pos  place of the edge's flux << 1 | side (u32)
+ *               sell_geo  the edge's normal and area    (4 x f64)
  *               sell_blk  BSR block of (v, neighbour)   (u32)
- *               sell_w*   LSQ term of the edge seen from v, 3 x f64 SoA
+ *               sell_w*   LSQ term of the edge seen from v, 3 x f64 SoA (not
+ *                         kept where the vertices' moments reproduce it)
  *   BSR       rowptr[N+1], col[nnzb], diag[N]; blocks of 16 values row-major,
  *             FP64 (a64) or FP32 (a32); BF16 factor copy (abf)
  *   levels    rows in level order of the lower (L) / upper (U) triangle,
@@ -53,7 +56,6 @@
 #define KF_ERR_NONFINITE_PIVOT 1u
 #define KF_ERR_SPIN_LIMIT 2u
 
-/* everything a kernel reads, passed by value */
 /* an edge's (unit normal, area): record i of a list of them */
 struct kf_egeo { double xn, yn, zn, ln; };
 __device__ __forceinline__ kf_egeo kf_edge_geo(const double *__restrict__ geo, size_t i)
@@ -63,6 +65,7 @@ __device__ __forceinline__ kf_egeo kf_edge_geo(const double *__restrict__ geo, s
   return {lo.x, lo.y, hi.x, hi.y};
 }
 
+/* everything a kernel reads, passed by value */
 struct kf_dv {
   uint32_t N, E, S, NS, NF, nslice;
   uint32_t spin_sleep;          /* s_sleep(1) repeats between two polls */
@@ -72,7 +75,7 @@ struct kf_dv {
   double *x, *y, *z;
   double *xyzw;                 /* (x, y, z, 0) per vertex: one 32-byte gather for the edge kernel */
   uint32_t *sell_ptr, *deg;
-  uint32_t *sell_nbr, *sell_ent, *sell_blk;
+  uint32_t *sell_nbr, *sell_blk;
   double *sell_wx, *sell_wy, *sell_wz;   /* the LSQ terms per incidence (NULL once lsq is verified) */
   double *lsq;                  /* 7 x N: per-vertex LSQ moments w00 w01 w02 w11 w12 w22 w33 (one array each) */
   uint32_t *sell_nbs;           /* neighbour | side << 31 per incidence */

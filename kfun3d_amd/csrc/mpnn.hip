@@ -392,12 +392,12 @@ __global__ __launch_bounds__(MP_RB) void k_mp_edge_vectors(kf_dv d, float4 *__re
   if (v >= d.N) return;
   size_t idx = (size_t)d.sell_ptr[v >> 6] * 64u + (v & 63u);
   for (uint32_t k = 0; k < d.deg[v]; k++, idx += 64) {
-    const uint32_t ent = d.sell_ent[idx], u = d.sell_nbr[idx];
+    const uint32_t at = d.sell_pos[idx], u = d.sell_nbr[idx];
     const kf_egeo eg = kf_edge_geo(d.sell_geo, idx);
-    const double ar = (ent & 1u) ? -eg.ln : eg.ln;
+    const double ar = (at & 1u) ? -eg.ln : eg.ln;
     const size_t ui = (size_t)d.sell_ptr[u >> 6] * 64u + (u & 63u);
     uint32_t kr = 0;
-    while (kr + 1 < d.deg[u] && d.sell_ent[ui + 64 * (size_t)kr] != (ent ^ 1u)) kr++;   /* u holds the other side */
+    while (kr + 1 < d.deg[u] && d.sell_pos[ui + 64 * (size_t)kr] != (at ^ 1u)) kr++;   /* u holds the other side */
     ev[idx] = make_float4((float)(eg.xn * ar), (float)(eg.yn * ar), (float)(eg.zn * ar), __uint_as_float(kr));
   }
   ideg[v] = 1.0f / (float)max(d.deg[v], 1u);
