@@ -346,7 +346,8 @@ int  kf_last_error(const GEOMETRY *g);
  * launch count of one kernel class ("grad", "edge_flux", "residual",
  * "timestep", "fill", "ilu", "trsv_lower", "trsv_upper", "spmv",
  * "jacobi_lower", "jacobi_upper", "coarse_factor", "coarse"); -1 if
- * unknown.  kf_profile_only(g, name) clears and starts it for that one class
+ * unknown.  Meshes of at most 32,768 vertices form the edge fluxes in the
+ * kernel of "residual": no launch of theirs is of class "edge_flux".  kf_profile_only(g, name) clears and starts it for that one class
  * (fewer events in the timed work); -1 if unknown.  No counterpart in the
  * reference. */
 void kf_profile(GEOMETRY *g, int on);

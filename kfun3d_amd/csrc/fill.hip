@@ -254,7 +254,7 @@ __device__ __forceinline__ void store_blocks(fill_rows<float> &rows, float *__re
   }
 }
 
-/* Bound by memory: the records of the incidences once (36 bytes each, dense)
+/* Bound by memory: the records of the incidences once (40 bytes each, dense)
  * and the blocks once, at the rate of a copy.  173x61x47 (496K vertices), FP32
  * with the kept copy: 0.303 ms, 4.4 TB/s (0.379 ms and a copy of 0.126 ms with
  * lanes storing their own blocks and gathered edge records; 0.374 ms with

@@ -6,8 +6,10 @@
  * updates from one thread.  Here every sum is a gather: the vertex walks its
  * incidence list (ascending edge id) and adds the same terms in the same
  * order, so the FP64 result is bit-identical and the kernels are atomic free
- * and run-to-run deterministic.  The per-edge Roe flux is evaluated once per
- * edge (k_edge_flux) and read back by both end points.
+ * and run-to-run deterministic.  On meshes of more than FLUX_ONE_ROWS vertices
+ * the Roe flux is evaluated once per edge (k_edge_flux) and read back by both
+ * end points; on smaller ones each end evaluates it for itself, with the same
+ * operands in the same order, in the kernel that sums it (k_flux_residual).
  *
  * Compiled with -ffp-contract=off: no FMA contraction, IEEE division and
  * square root, so each expression rounds as in the reference.
@@ -475,8 +477,9 @@ __device__ __forceinline__ d4 roe_flux(const d4 &L, const d4 &R, double xn, doub
  * Bound by memory and by the L1's lookups (83 % of its cycles).  The fluxes go
  * to their places in sliced-ELL order, where k_residual finds one end's share
  * of its incidences as dense lines: its loads fall from 1.6 to 1.1 GB at
- * 288x96x96 (0.310 -> 0.199 ms), the scattered stores here cost 0.05 ms of that
- * (0.505 -> 0.551 ms; stored lane by lane 0.569). */
+ * 288x96x96 (0.302 -> 0.196 ms, by events over a loop of residuals), the
+ * scattered stores here cost 0.02 ms of that (0.468 -> 0.490 ms; stored lane by
+ * lane 0.02 more). */
 template <bool SPECTRAL>
 __global__ __launch_bounds__(256) void k_edge_flux(kf_dv d, const double *__restrict__ q,
                                                    const double *__restrict__ gx, const double *__restrict__ gy,
@@ -731,8 +734,10 @@ __global__ __launch_bounds__(256) void k_flux_residual(kf_dv d, const double *__
  * 16 lanes to a vertex (the 3072 wavefronts the chip holds of it), else 4.
  * One residual (gradient, launches and all), two kernels against one:
  * 1.6K vertices 21.8 / 17.4 us, 12K 24.0 / 19.3, 22K 28.6 / 25.0, 36K
- * 35.2 / 33.3, 66K 44.8 / 44.7, 111K 60.3 / 68.4; 4 lanes for 16: 1.6K 20.4,
- * 6K 22.0 for 20.0, 12K 20.0, 22K 25.0 for 26.7. */
+ * 35.2 / 33.3, 66K 44.8 / 44.7, 111K 60.3 / 68.4.  Measured again, 16 lanes
+ * against 4: 1.7K 14.5 / 17.7, 6.1K 16.4 / 17.4, 8.8K 17.7 / 17.4, 12.3K 17.1 /
+ * 17.8, and past the 3072 wavefronts 13.9K 20.0 / 17.3, 15.6K 20.8 / 17.5,
+ * 17.5K 21.2 / 21.0, 21.7K 22.8 / 21.6, 31.9K 27.6 / 22.5. */
 #define FLUX_ONE_ROWS 32768u
 #define FLUX_WIDE_ROWS 12288u
 

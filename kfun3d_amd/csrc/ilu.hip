@@ -258,7 +258,7 @@ struct ilu_layout {
 /* The tickets of a workgroup.  One atomic on the launch's counter draws a
  * batch of B consecutive tickets (they serialise at about 12 ns each: with 4
  * to an atomic they bounded the FP32 factors of 2.65M vertices at 8.1 ms, with
- * 8 those take 4.6), and the workgroup's wavefronts take them one by one from
+ * 8 those take 4.5), and the workgroup's wavefronts take them one by one from
  * LDS, in order and without waiting for one another.  B is the number of
  * wavefronts: more rows of one level to a wavefront take it longer, fewer
  * serialise.  The wavefront that takes the first of batch k
@@ -324,8 +324,9 @@ __device__ __forceinline__ uint32_t step_end(uint32_t moreg, const uint32_t *smo
  * table, so that all of a lane's loads go out together.  Against a version
  * that took each block's place from one of three tables on its own branch,
  * formed L(i,m) on 16 lanes through LDS and loaded each row when its
- * predecessor was done: FP64 (exact) 2.05 -> 1.65 ms on 331,776 vertices and
- * 12.7 -> 10.0 ms on 2.65M, FP32 1.36 -> 1.22 and 8.1 -> 4.6 ms. */
+ * predecessor was done: FP64 (exact) 2.05 -> 1.62 ms on 331,776 vertices and
+ * 12.7 -> 9.9 ms on 2.65M, FP32 1.36 -> 1.11 and 8.1 -> 4.5 ms (with the sweeps'
+ * copy stored as well 1.73, 10.8, 1.16 and 4.9). */
 /* where a row's factors go beside a: the BF16 copy (TS = uint16_t) and, with
  * Jacobi sweeps, the sweeps' sliced copy (val; layout at k_jac_lower_sl), in
  * TS.  Written from the row in LDS, they cost their own stores; as passes

@@ -12,13 +12,14 @@
  * component c:  y[4r + c] = sum over the row's blocks j in ascending column
  * of  a_j[c][0] x0 + a_j[c][1] x1 + a_j[c][2] x2 + a_j[c][3] x3,  each
  * product added to the running sum in that order, in FP64 (FP32-stored
- * values are widened first).  The four lanes of a quad read one 128-byte
- * block (FP64) row by row, so a wave's loads are whole blocks; of the column's
- * four x values each loads one, and the quad exchanges them (FP32 blocks).  Workgroups are
- * remapped XCD by XCD (kf_xcd_block) so that each XCD works on a contiguous
- * slab of rows and its x gathers stay in its L2.  Bytes per launch:
- * nnzb (16 s + 4) + 64 N with s the stored value size (HBM-bound: 4 to 8 blocks
- * in flight a lane and 4 to 8 wavefronts a SIMD measure the same).
+ * values are widened first).  The four lanes of a quad read a block row by
+ * row, so a wave's loads are whole blocks.  FP64: two blocks in flight, the
+ * column's whole vector in each lane.  FP32: eight blocks in flight, of the
+ * column's four x values each lane loads one and the quad exchanges them
+ * (there 4 to 8 blocks in flight and 4 to 8 wavefronts a SIMD measure the
+ * same).  Workgroups are remapped XCD by XCD (kf_xcd_block) so that each XCD
+ * works on a contiguous slab of rows and its x gathers stay in its L2.  Bytes
+ * per launch: nnzb (16 s + 4) + 64 N with s the stored value size (HBM-bound).
  */
 #include "kf_dev.h"
 
