@@ -918,7 +918,8 @@ __global__ __launch_bounds__(RB) void k_fd_perturb(size_t n, double h, const dou
 
 /* k_red_final's |x| from the partials (every block forms the same value;
  * block 0 stores it), then k_fd_perturb: one launch less in front of every
- * product, 4.5 us on the host and 5 on the device */
+ * product (iJacVec one after another: 1.7K vertices 24.5 -> 23.2 us, 12K
+ * 26.4 -> 25.2, 332K 143 -> 141) */
 #define PERTURB_BATCH 4
 __global__ __launch_bounds__(RB) void k_norm_perturb(size_t n, double h, const double *__restrict__ part,
                                                      double *__restrict__ xnorm, const double *__restrict__ x,
